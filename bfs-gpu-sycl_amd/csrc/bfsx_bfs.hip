@@ -2230,70 +2230,103 @@ __global__ __launch_bounds__(WG) void k_coop_levels(KArgs base, LevelCtl *ctl, C
   if (blockIdx.x == 0 && threadIdx.x == 0) write_level_end(ctl, cur, c.mirror);
 }
 
-// sum of out-degree over reached vertices < n_rows, reached count, max level
+// Vertex counts and out-degree sums per level: out[0] = deepest level + 1,
+// out[1 + l] = vertices at level l, out[1 + max_levels + l] = their degrees.
+//
+// One pass over the levels and the 16-bit degrees (6 bytes per vertex), four
+// vertices per lane as wide loads.  What bounds it is not those bytes but
+// adding to a few hot counters: a power-law graph has about seven levels, so
+// a wave's 64 vertices share two or three.  A wave therefore adds up its
+// equal levels in registers first (a ballot per distinct level, up to
+// HIST_ROUNDS of them, a grid's many levels per wave go to LDS lane by
+// lane), work-groups add in LDS, and there is one large work-group per CU:
+// global atomics on one line take 12 ns each, and 1024 groups spent more on
+// them than on the pass.
+constexpr uint32_t HIST_LDS_LEVELS = 1024;
+constexpr uint32_t HIST_WG = 1024;
+constexpr int HIST_ROUNDS = 4;
+
 template <typename PtrT>
-__global__ void k_summarize(const PtrT *col_ptr, const int32_t *levels, uint32_t n_rows,
-                            uint32_t n_cols, unsigned long long *out) {
-  unsigned long long edges = 0, reached = 0;
+__global__ __launch_bounds__(HIST_WG) void k_level_hist(const PtrT *col_ptr,
+                                                        const uint16_t *deg16,
+                                                        const int32_t *levels, uint32_t n_rows,
+                                                        uint32_t n_cols, uint32_t max_levels,
+                                                        unsigned long long *out) {
+  __shared__ unsigned long long s_cnt[HIST_LDS_LEVELS];
+  __shared__ unsigned long long s_edg[HIST_LDS_LEVELS];
+  __shared__ int s_max;
+  const bool lds = max_levels <= HIST_LDS_LEVELS;
+  unsigned long long *cnt = lds ? s_cnt : out + 1;
+  unsigned long long *edg = lds ? s_edg : out + 1 + max_levels;
+  if (lds)
+    for (uint32_t i = threadIdx.x; i < max_levels; i += HIST_WG) s_cnt[i] = s_edg[i] = 0;
+  if (threadIdx.x == 0) s_max = -1;
+  __syncthreads();
   int32_t mx = -1;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_cols;
-       i += gridDim.x * blockDim.x) {
-    const int32_t l = levels[i];
-    if (l >= 0) {
-      reached++;
+  // (whole waves: every lane takes part in the ballots)
+  const uint64_t n4 = ((uint64_t)n_cols + 3) / 4;
+  const uint64_t stride = (uint64_t)gridDim.x * HIST_WG;
+  const uint64_t first = blockIdx.x * (uint64_t)HIST_WG + (threadIdx.x & ~63u);
+  for (uint64_t base = first; base < n4; base += stride) {
+    const uint64_t v0 = (base + (threadIdx.x & 63)) * 4;
+    int32_t l4[4] = {-1, -1, -1, -1};
+    uint32_t d4[4] = {0, 0, 0, 0};
+    if (v0 + 4 <= n_cols) {
+      const int4 l = *reinterpret_cast<const int4 *>(levels + v0);
+      const ushort4 d = *reinterpret_cast<const ushort4 *>(deg16 + v0);
+      l4[0] = l.x, l4[1] = l.y, l4[2] = l.z, l4[3] = l.w;
+      d4[0] = d.x, d4[1] = d.y, d4[2] = d.z, d4[3] = d.w;
+    } else {
+      for (int k = 0; k < 4; k++)
+        if (v0 + k < n_cols) {
+          l4[k] = levels[v0 + k];
+          d4[k] = deg16[v0 + k];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int32_t l = l4[k];
       mx = l > mx ? l : mx;
-      if (i < n_rows) edges += (unsigned long long)(col_ptr[i + 1] - col_ptr[i]);
+      const bool in = l >= 0 && (uint32_t)l < max_levels;
+      const uint32_t d = in && v0 + k < n_rows ? d4[k] : 0u;
+      bool todo = in;
+      if (d == DEG16_ESCAPE) {  // (few) the whole degree
+        const uint32_t v = (uint32_t)(v0 + k);
+        atomicAdd(&cnt[l], 1ull);
+        atomicAdd(&edg[l], (unsigned long long)(col_ptr[v + 1] - col_ptr[v]));
+        todo = false;
+      }
+      unsigned long long m = __ballot(todo);
+      for (int r = 0; m && r < HIST_ROUNDS; r++) {
+        const int leader = __ffsll(m) - 1;
+        const int32_t L = __shfl(l, leader, 64);
+        const unsigned long long same = __ballot(todo && l == L);
+        const uint32_t sum = wave_sum(todo && l == L ? d : 0u);  // below 64 * 2^16
+        if ((int)__lane_id() == leader) {
+          atomicAdd(&cnt[L], (unsigned long long)__popcll(same));
+          if (sum) atomicAdd(&edg[L], (unsigned long long)sum);
+        }
+        if (l == L) todo = false;
+        m &= ~same;
+      }
+      if (todo) {
+        atomicAdd(&cnt[l], 1ull);
+        if (d) atomicAdd(&edg[l], (unsigned long long)d);
+      }
     }
   }
-  edges = wave_sum(edges);
-  reached = wave_sum(reached);
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
     const int32_t o = __shfl_xor(mx, d, 64);
     mx = o > mx ? o : mx;
   }
-  if ((threadIdx.x & 63) == 0) {
-    if (edges) atomicAdd(&out[0], edges);
-    if (reached) atomicAdd(&out[1], reached);
-    if (mx >= 0) atomicMax(&out[2], (unsigned long long)mx);
-  }
-}
-
-// per-level vertex counts and out-degree sums; LDS histogram per block when
-// the level count is small, global atomics otherwise
-constexpr uint32_t HIST_LDS_LEVELS = 1024;
-
-template <typename PtrT>
-__global__ __launch_bounds__(256) void k_level_hist(const PtrT *col_ptr, const int32_t *levels,
-                                                    uint32_t n_rows, uint32_t n_cols,
-                                                    uint32_t max_levels,
-                                                    unsigned long long *counts,
-                                                    unsigned long long *edges) {
-  __shared__ unsigned long long s_cnt[HIST_LDS_LEVELS];
-  __shared__ unsigned long long s_edg[HIST_LDS_LEVELS];
-  const bool lds = max_levels <= HIST_LDS_LEVELS;
-  if (lds)
-    for (uint32_t i = threadIdx.x; i < max_levels; i += blockDim.x) s_cnt[i] = s_edg[i] = 0;
+  if ((threadIdx.x & 63) == 0 && mx >= 0) atomicMax(&s_max, mx);
   __syncthreads();
-  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n_cols;
-       v += gridDim.x * blockDim.x) {
-    const int32_t l = levels[v];
-    if (l < 0 || (uint32_t)l >= max_levels) continue;
-    const unsigned long long d =
-        v < n_rows ? (unsigned long long)(col_ptr[v + 1] - col_ptr[v]) : 0ull;
-    if (lds) {
-      atomicAdd(&s_cnt[l], 1ull);
-      if (d) atomicAdd(&s_edg[l], d);
-    } else {
-      atomicAdd(&counts[l], 1ull);
-      if (d) atomicAdd(&edges[l], d);
-    }
-  }
-  __syncthreads();
+  if (threadIdx.x == 0 && s_max >= 0) atomicMax(&out[0], (unsigned long long)s_max + 1);
   if (lds)
-    for (uint32_t i = threadIdx.x; i < max_levels; i += blockDim.x) {
-      if (s_cnt[i]) atomicAdd(&counts[i], s_cnt[i]);
-      if (s_edg[i]) atomicAdd(&edges[i], s_edg[i]);
+    for (uint32_t i = threadIdx.x; i < max_levels; i += HIST_WG) {
+      if (s_cnt[i]) atomicAdd(&out[1 + i], s_cnt[i]);
+      if (s_edg[i]) atomicAdd(&out[1 + max_levels + i], s_edg[i]);
     }
 }
 
@@ -2869,35 +2902,19 @@ bool coop_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool le
   return ctx->ptr_bytes == 8 ? coop_levels_t<uint64_t>(ctx, a, c) : coop_levels_t<uint32_t>(ctx, a, c);
 }
 
-void reached_summary(bfsx_ctx *ctx, unsigned long long *d_out) {
-  const unsigned grid = cap_grid(((uint64_t)ctx->n_cols + 255) / 256,
-                                 (unsigned)ctx->cu_count * 8);
-  BFSX_HIP(hipMemsetAsync(d_out, 0, 3 * sizeof(unsigned long long), ctx->stream));
+void level_histogram(bfsx_ctx *ctx, uint32_t max_levels, unsigned long long *d_out) {
+  const unsigned grid = cap_grid(((uint64_t)ctx->n_cols + 4 * HIST_WG - 1) / (4 * HIST_WG),
+                                 (unsigned)ctx->cu_count);
+  BFSX_HIP(hipMemsetAsync(d_out, 0, sizeof(unsigned long long) * (2 * (size_t)max_levels + 1),
+                          ctx->stream));
   if (ctx->ptr_bytes == 8)
-    hipLaunchKernelGGL(k_summarize<uint64_t>, dim3(grid), dim3(256), 0, ctx->stream,
-                       ctx->col_ptr.as<uint64_t>(), ctx->levels.as<int32_t>(), ctx->n_rows,
-                       ctx->n_cols, d_out);
+    hipLaunchKernelGGL(k_level_hist<uint64_t>, dim3(grid), dim3(HIST_WG), 0, ctx->stream,
+                       ctx->col_ptr.as<uint64_t>(), ctx->deg16.as<uint16_t>(),
+                       ctx->levels.as<int32_t>(), ctx->n_rows, ctx->n_cols, max_levels, d_out);
   else
-    hipLaunchKernelGGL(k_summarize<uint32_t>, dim3(grid), dim3(256), 0, ctx->stream,
-                       ctx->col_ptr.as<uint32_t>(), ctx->levels.as<int32_t>(), ctx->n_rows,
-                       ctx->n_cols, d_out);
-  BFSX_HIP(hipGetLastError());
-}
-
-void level_histogram(bfsx_ctx *ctx, uint32_t max_levels, unsigned long long *d_counts,
-                     unsigned long long *d_edges) {
-  const unsigned grid = cap_grid(((uint64_t)ctx->n_cols + 255) / 256,
-                                 (unsigned)ctx->cu_count * 4);
-  BFSX_HIP(hipMemsetAsync(d_counts, 0, sizeof(unsigned long long) * max_levels, ctx->stream));
-  BFSX_HIP(hipMemsetAsync(d_edges, 0, sizeof(unsigned long long) * max_levels, ctx->stream));
-  if (ctx->ptr_bytes == 8)
-    hipLaunchKernelGGL(k_level_hist<uint64_t>, dim3(grid), dim3(256), 0, ctx->stream,
-                       ctx->col_ptr.as<uint64_t>(), ctx->levels.as<int32_t>(), ctx->n_rows,
-                       ctx->n_cols, max_levels, d_counts, d_edges);
-  else
-    hipLaunchKernelGGL(k_level_hist<uint32_t>, dim3(grid), dim3(256), 0, ctx->stream,
-                       ctx->col_ptr.as<uint32_t>(), ctx->levels.as<int32_t>(), ctx->n_rows,
-                       ctx->n_cols, max_levels, d_counts, d_edges);
+    hipLaunchKernelGGL(k_level_hist<uint32_t>, dim3(grid), dim3(HIST_WG), 0, ctx->stream,
+                       ctx->col_ptr.as<uint32_t>(), ctx->deg16.as<uint16_t>(),
+                       ctx->levels.as<int32_t>(), ctx->n_rows, ctx->n_cols, max_levels, d_out);
   BFSX_HIP(hipGetLastError());
 }
 

@@ -152,6 +152,9 @@ struct RunOut {
   double ms = 0;
   uint32_t n_levels = 0;
   uint32_t steps[BFSX_N_STEP_KINDS] = {0, 0, 0, 0};
+  // what the level ends counted: the sizes and the out-degree sums of all
+  // frontiers (a vertex is in exactly one)
+  unsigned long long reached = 0, edges = 0;
 };
 
 // Full copy of the control block into h_ctl (stream synchronised).
@@ -487,6 +490,8 @@ static RunOut search_graph_loop(bfsx_ctx *ctx, uint32_t root, int fixed, bool le
     out.steps[k] = ctx->h_ctl->kind_count[k];
     out.n_levels += out.steps[k];
   }
+  out.reached = ctx->h_ctl->visited_vertices;
+  out.edges = ctx->h_ctl->visited_edges;
   return out;
 }
 
@@ -548,6 +553,7 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
   ctx->trace.clear();
 
   RunOut out;
+  out.reached = 1;  // the root
   BFSX_HIP(hipEventRecord(ctx->ev0, s));
   uint64_t f_edges = 0, visited_v = 1, visited_e = 0, examined = 0;
   // The root level (one vertex) runs LLB, the choice k_init leaves in the
@@ -641,6 +647,7 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
     // scheduler inputs and outputs)
     if (timed) read_ctl(ctx);
     w.advance(new_fbm);
+    out.reached += w.F;
     if (timed) {
       r.level = level;
       r.choice = (uint32_t)choice;
@@ -672,9 +679,11 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
   float ms = 0;
   BFSX_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   out.ms = ms;
-  if (dev_loop) {  // the device loop's levels were counted per kind on the device
+  out.edges = w.VE;
+  if (dev_loop) {  // the device loop's levels were counted on the device
     read_ctl(ctx);
     for (int k = 0; k < BFSX_N_STEP_KINDS; k++) out.steps[k] = ctx->h_ctl->kind_count[k];
+    out.reached = ctx->h_ctl->visited_vertices;
   }
   return out;
 }
@@ -789,16 +798,15 @@ static void finish_run(bfsx_ctx *ctx, const RunOut &r, int32_t *levels_out,
                        uint32_t *parents_out, bfsx_run_stats *stats) {
   hipStream_t s = ctx->stream;
   if (stats) {
-    ensure(ctx->scratch, 64, s);
-    reached_summary(ctx, ctx->scratch.as<unsigned long long>());
-    unsigned long long h[3] = {0, 0, 0};
-    BFSX_HIP(hipMemcpyAsync(h, ctx->scratch.p, sizeof(h), hipMemcpyDeviceToHost, s));
-    BFSX_HIP(hipStreamSynchronize(s));
+    // The counts come from the level ends, which keep them exactly (they
+    // decide each level's step).  A pass over levels and col_ptr after the
+    // search recounted them: 295 us at scales 19 and 22 (as long as the
+    // search; its atomics on one line), 465 us at scale 26.
     std::memset(stats, 0, sizeof(*stats));
     stats->ms = r.ms;
-    stats->edges_count = h[0];
-    stats->reached = h[1];
-    stats->max_level = (uint32_t)h[2];
+    stats->edges_count = r.edges;
+    stats->reached = r.reached;
+    stats->max_level = r.n_levels - 1;  // the last frontier expanded
     stats->n_levels = r.n_levels;
     for (int i = 0; i < BFSX_N_STEP_KINDS; i++) stats->steps[i] = r.steps[i];
   }
@@ -1157,10 +1165,7 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
         BFSX_HIP(hipStreamSynchronize(s));
         for (uint32_t i = 0; i < probe_batch && !found; i++) {
           if (!ok[i]) continue;
-          search(ctx, cand[i], BFSX_LLB, 0, false);
-          bfsx_run_stats st;
-          finish_run(ctx, RunOut{}, nullptr, nullptr, &st);
-          if (st.reached * 2 > ctx->n_cols) found = true;
+          if (search(ctx, cand[i], BFSX_LLB, 0, false).reached * 2 > ctx->n_cols) found = true;
         }
       }
       release(dv);
@@ -1233,20 +1238,19 @@ int bfsx_level_histogram(bfsx_ctx *ctx, uint64_t *counts, uint64_t *edges, uint3
     if (!ctx->has_graph || !ctx->levels.p) fail(BFSX_ERR_STATE, "no search has run");
     if (max_levels == 0 || max_levels > (1u << 24)) fail(BFSX_ERR_ARG, "max_levels out of range");
     hipStream_t s = ctx->stream;
-    ensure(ctx->scratch, sizeof(unsigned long long) * (2 * (size_t)max_levels + 3), s);
+    ensure(ctx->scratch, sizeof(unsigned long long) * (2 * (size_t)max_levels + 1), s);
     unsigned long long *d = ctx->scratch.as<unsigned long long>();
-    reached_summary(ctx, d);
-    level_histogram(ctx, max_levels, d + 3, d + 3 + max_levels);
-    std::vector<unsigned long long> h(2 * (size_t)max_levels + 3);
+    level_histogram(ctx, max_levels, d);
+    std::vector<unsigned long long> h(2 * (size_t)max_levels + 1);
     BFSX_HIP(hipMemcpyAsync(h.data(), d, sizeof(unsigned long long) * h.size(),
                             hipMemcpyDeviceToHost, s));
     BFSX_HIP(hipStreamSynchronize(s));
-    const uint32_t nl = h[1] ? (uint32_t)h[2] + 1 : 0;
+    const uint32_t nl = (uint32_t)h[0];
     if (n_levels) *n_levels = nl;
     if (nl > max_levels) fail(BFSX_ERR_OVERFLOW, "more levels than max_levels");
     for (uint32_t i = 0; i < max_levels; i++) {
-      if (counts) counts[i] = h[3 + i];
-      if (edges) edges[i] = h[3 + max_levels + i];
+      if (counts) counts[i] = h[1 + i];
+      if (edges) edges[i] = h[1 + max_levels + i];
     }
   });
 }
@@ -1415,10 +1419,7 @@ int bfsx_autotune(bfsx_ctx *ctx, const uint32_t *roots, uint32_t n_roots, int st
     if (passes < 1 || passes > 4) fail(BFSX_ERR_ARG, "passes must be in [1,4]");
     std::vector<double> edges(n_roots);
     for (uint32_t i = 0; i < n_roots; i++) {
-      const RunOut r = search(ctx, roots[i], strategy, 0, false);
-      bfsx_run_stats st;
-      finish_run(ctx, r, nullptr, nullptr, &st);
-      edges[i] = (double)st.edges_count;
+      edges[i] = (double)search(ctx, roots[i], strategy, 0, false).edges;
     }
     struct Knob {
       uint32_t bfsx_params::*field;

@@ -344,9 +344,8 @@ bool coop_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool le
 // After a device loop (level0 = the level at its launch) the buffer is
 // `produced` flipped once per level it ran.
 void read_level_end(bfsx_ctx *ctx, uint32_t seq, uint32_t produced, uint32_t level0 = ~0u);
-void reached_summary(bfsx_ctx *ctx, unsigned long long *d_out);
-void level_histogram(bfsx_ctx *ctx, uint32_t max_levels, unsigned long long *d_counts,
-                     unsigned long long *d_edges);
+// d_out: 2 * max_levels + 1 entries (see k_level_hist)
+void level_histogram(bfsx_ctx *ctx, uint32_t max_levels, unsigned long long *d_out);
 void stream_copy(bfsx_ctx *ctx, const void *src, void *dst, uint64_t bytes);
 
 // ---- batched multi-source search (bfsx_msbfs.hip) -------------------------

@@ -1,0 +1,55 @@
+"""Kernel variants and dispatch rules at the sizes where they can go wrong
+(edges of tiles, remainders, escapes), against the CPU oracle.  Results are
+whole numbers: equal, no tolerance."""
+import numpy as np
+import pytest
+
+from graphs import csc_from_edges, path_graph, random_graph, star_graph, symmetrize
+from oracle import cpu
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def some_graph(name):
+    """(col_ptr, row_idx, n_rows, symmetric, root)"""
+    rng = np.random.default_rng(41)
+    if name == "one":
+        return np.zeros(2, np.uint32), np.zeros(0, np.uint32), 1, True, 0
+    if name == "path2500":
+        return (*path_graph(2500), 2500, True, 0)
+    if name == "star70001":
+        return (*star_graph(70001), 70001, True, 5)
+    if name == "directed4099":
+        cp, ri = random_graph(rng, 4099, 30000)
+        ri = ri[: int(cp[3000])]
+        cp = np.minimum(cp, cp[3000]).astype(np.uint64)
+        return cp, ri, 3000, False, int(np.flatnonzero(np.diff(cp.astype(np.int64)))[0])
+    n = int(name)
+    cp, ri = random_graph(rng, n, 3 * n, directed=False)
+    return cp, ri, n, True, int(np.argmax(np.diff(cp)))
+
+
+# a work-group of the histogram takes 4096 vertices, a lane four; tables of
+# more than 1024 levels are counted in global memory; degrees of 65535 and
+# more are not in the 16-bit array
+@pytest.mark.parametrize("name", ["one", "3", "4", "257", "4096", "4099", "20001", "path2500",
+                                  "star70001", "directed4099"])
+def test_level_histogram_edges(engine, name):
+    say("histogram", name)
+    cp, ri, n_rows, sym, root = some_graph(name)
+    engine.upload_csc(cp, ri, n_rows=n_rows, symmetric=sym)
+    want, ec, _ = cpu.bfs_queue(cp, ri, root, n_rows=n_rows)
+    deg = np.where(np.arange(len(want)) < n_rows, np.diff(cp.astype(np.int64)), 0)
+    hist = np.bincount(want[want >= 0])
+    lev, st = engine.run(root, "llb")
+    assert (lev == want).all()
+    assert [st[k] for k in ("edges_count", "reached", "max_level", "n_levels")] == [
+        ec, int(hist.sum()), len(hist) - 1, len(hist)]
+    for size in (8, 1024, 4096):
+        counts, edges = engine.level_histogram(size)
+        assert (counts == hist).all()
+        assert (edges == np.bincount(want[want >= 0], weights=deg[want >= 0])).all()
