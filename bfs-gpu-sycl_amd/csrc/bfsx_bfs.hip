@@ -1986,6 +1986,9 @@ __global__ void k_level_begin(LevelCtl *ctl) {
 struct LevelEndWords {
   uint32_t F, choice, done, level, seq;
   unsigned long long EF, VE;
+  uint32_t n_llb, n_slb;  // levels run as LLB, SLB
+  unsigned long long VV;  // visited vertices
+  uint32_t prev_F;        // the frontier that the level expanded
 };
 
 // Bookkeeping at the end of a level, by one work-group (every thread calls
@@ -1995,20 +1998,21 @@ struct LevelEndWords {
 // flag.  Returns false, having changed nothing, when `guard` says that a
 // speculative launch's guess failed.  With `words`, thread 0 also leaves
 // there what the control block holds afterwards for the host's words, so
-// that they need no second read of it.
+// that they need no second read of it.  staged: the weights, in LDS already.
 __device__ __forceinline__ bool level_end_body(LevelCtl *ctl, uint32_t consumed,
                                                uint32_t produced, int stamp, int kind,
                                                const float *Wg, uint64_t n_cols, uint64_t nnz,
                                                uint64_t n_iso, uint32_t allow, int reuse,
                                                const SpecGuard &guard,
-                                               LevelEndWords *words = nullptr) {
+                                               LevelEndWords *words = nullptr,
+                                               const float4 *staged = nullptr) {
   __shared__ int s_live, s_skip;
   __shared__ float4 s_W4[NPARAM / 4];
   // the network's weights, loaded while thread 0 reads the control block
   // (both are round trips to memory; one waits for the other otherwise)
   constexpr int WPT = (NPARAM / 4 + 63) / 64;
   float4 wr[WPT];
-  if (Wg && threadIdx.x < 64) {
+  if (Wg && !staged && threadIdx.x < 64) {
     const float4 *G4 = reinterpret_cast<const float4 *>(Wg);
 #pragma unroll
     for (int i = 0; i < WPT; i++) {
@@ -2039,11 +2043,13 @@ __device__ __forceinline__ bool level_end_body(LevelCtl *ctl, uint32_t consumed,
       // nothing to do
     } else if (fc == 0) {
       ctl->done = 1;
-      if (words) *words = LevelEndWords{n, choice, 1u, level, seq0, ef, ve};
+      if (words) *words = LevelEndWords{n, choice, 1u, level, seq0, ef, ve, kc0, kc2, vv, fc};
     } else {
-      if (words) *words = LevelEndWords{n, choice, n == 0 ? 1u : 0u, level + 1, seq0, ef, ve + ef};
-      if (stamp) ctl->t_end = (unsigned long long)wall_clock64();
       const uint32_t k = kind >= 0 ? (uint32_t)kind : choice;
+      if (words)
+        *words = LevelEndWords{n, choice, n == 0 ? 1u : 0u, level + 1, seq0, ef, ve + ef,
+                               kc0 + (k == BFSX_LLB), kc2 + (k == BFSX_SLB), vv + n, fc};
+      if (stamp) ctl->t_end = (unsigned long long)wall_clock64();
       if (k < 4) ctl->kind_count[k] = (k == 0 ? kc0 : k == 1 ? kc1 : k == 2 ? kc2 : kc3) + 1;
       ctl->discovered = n;
       ctl->visited_vertices = vv + n;
@@ -2079,15 +2085,18 @@ __device__ __forceinline__ bool level_end_body(LevelCtl *ctl, uint32_t consumed,
     // the learned scheduler picks the next level's step in the same launch
     // (a level that keeps the last decision skips the network)
     if (s_live) {
-      if (threadIdx.x < 64) {
+      if (!staged) {
+        if (threadIdx.x < 64) {
 #pragma unroll
-        for (int i = 0; i < WPT; i++) {
-          const int j = (int)threadIdx.x + 64 * i;
-          if (j < NPARAM / 4) s_W4[j] = wr[i];
+          for (int i = 0; i < WPT; i++) {
+            const int j = (int)threadIdx.x + 64 * i;
+            if (j < NPARAM / 4) s_W4[j] = wr[i];
+          }
         }
+        __syncthreads();
       }
-      __syncthreads();
-      const uint32_t picked = decide_compute(ctl, s_W4, produced, n_cols, nnz, n_iso, allow, 0);
+      const uint32_t picked = decide_compute(ctl, staged ? staged : s_W4, produced, n_cols, nnz,
+                                             n_iso, allow, 0);
       if (words && threadIdx.x == 0) words->choice = picked;
     }
   }
@@ -2114,13 +2123,19 @@ __device__ __forceinline__ void put_level_end(LevelCtl *ctl, const LevelEndWords
   mirror->w[2] = t16 | (v.VE & MIRROR_48);
   mirror->w[3] = t32 | (v.choice & 0xFFu) | ((unsigned long long)(v.done ? 1u : 0u) << 8) |
                  ((unsigned long long)(v.level & MIRROR_LEVEL_MASK) << 9);
+  mirror->w[4] = t16 | (unsigned long long)(v.n_slb & MIRROR_KIND_MASK) << 24 |
+                 (v.n_llb & MIRROR_KIND_MASK);
+  mirror->w[5] = t16 | (v.VV & MIRROR_48);
+  mirror->w[6] = t32 | v.prev_F;
 }
 
 __device__ __forceinline__ void write_level_end(LevelCtl *ctl, uint32_t produced,
-                                                LevelMirror *mirror) {
+                                                uint32_t prev_F, LevelMirror *mirror) {
   put_level_end(ctl,
                 LevelEndWords{ctl->q_count[produced], ctl->choice, ctl->done, ctl->level,
-                              ctl->seq, ctl->q_edges[produced], ctl->visited_edges},
+                              ctl->seq, ctl->q_edges[produced], ctl->visited_edges,
+                              ctl->kind_count[BFSX_LLB], ctl->kind_count[BFSX_SLB],
+                              ctl->visited_vertices, prev_F},
                 mirror);
 }
 
@@ -2227,7 +2242,211 @@ __global__ __launch_bounds__(WG) void k_coop_levels(KArgs base, LevelCtl *ctl, C
     });
     cur ^= 1;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) write_level_end(ctl, cur, c.mirror);
+  if (blockIdx.x == 0 && threadIdx.x == 0) write_level_end(ctl, cur, 0u, c.mirror);
+}
+
+// ---------------------------------------------------------------------------
+// solo loop: consecutive tiny levels in one launch of one work-group
+// ---------------------------------------------------------------------------
+// The first levels of a search and its tail hold a few edges each; as
+// launches of a step and a level end they cost about 20 us apiece, nearly
+// all of it dispatch gaps and the host's round trip.  Here one work-group
+// runs them back to back.  What bounds a level is its chain of dependent
+// reads, about 0.7 us each, so the chain is short: the control block and the
+// scheduler's weights are read into LDS once and written back once; a
+// discovered vertex keeps its list's start and length (read for the edge
+// count anyway) with its queue entry in LDS, so the next level begins with
+// its lists; an edge group's reads are issued together; the visited bits are
+// set with work-group-scope atomics, done in this XCD's L2 (no other group
+// runs).  Levels of more than SOLO_WG vertices read the rest from the queue,
+// which is written in full.  A single group makes LLB's and SLB's mappings of
+// entries to groups the same.
+//
+// The loop leaves, like the device loop's, at a level whose kind is neither
+// LLB nor SLB or that holds more than c.max_edges edges or vertices, at the
+// end of the search, or after max_levels, and writes one set of level-end
+// words.  With max_levels 0 it only writes them: the first state of a
+// search, instead of a copy of the control block and a synchronisation.
+constexpr int SOLO_WG = 1024;
+struct SoloArgs {
+  uint32_t *queue[2];
+  uint32_t cur;         // queue buffer holding the frontier at entry
+  int fixed;            // BFSX_LLB or BFSX_SLB, or -1: ctl->choice
+  uint32_t max_edges;
+  uint32_t max_levels;
+  const float *Wg;      // scheduler weights (learned) or null
+  uint64_t n_cols, nnz, n_iso;
+  uint32_t allow;       // kinds the scheduler may pick
+  LevelMirror *mirror;
+};
+
+template <typename PtrT>
+__global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl, SoloArgs c) {
+  __shared__ LevelCtl s_ctl;
+  __shared__ float4 s_W4[NPARAM / 4];
+  __shared__ PtrT s_nstart[SOLO_WG], s_start[SOLO_WG];       // next frontier's lists, this tile's
+  __shared__ uint32_t s_ndeg[SOLO_WG], s_nv[SOLO_WG], s_v[SOLO_WG];
+  __shared__ uint32_t s_scan[SOLO_WG], s_wave[SOLO_WG / 64 + 1];
+  __shared__ uint32_t s_count;
+  __shared__ unsigned long long s_edges;
+  constexpr uint32_t CTL_WORDS = sizeof(LevelCtl) / 4;
+  static_assert(CTL_WORDS <= SOLO_WG, "one word per thread");
+  const PtrT *col_ptr = static_cast<const PtrT *>(a.col_ptr);
+  const uint32_t t = threadIdx.x, lane = t & 63;
+  uint32_t cur = c.cur, prev_F = 0;
+  if (t < CTL_WORDS)
+    reinterpret_cast<uint32_t *>(&s_ctl)[t] = reinterpret_cast<const uint32_t *>(ctl)[t];
+  if (c.Wg)
+    for (uint32_t i = t; i < NPARAM / 4; i += SOLO_WG)
+      s_W4[i] = reinterpret_cast<const float4 *>(c.Wg)[i];
+  // (the queue holds n_cols + 1 entries: in bounds whatever the frontier)
+  uint32_t v = t < a.n_cols ? c.queue[cur][t] : 0u;
+  __syncthreads();
+  PtrT st = 0;
+  uint32_t deg = 0;
+  // this thread's entry of the frontier's first tile
+  if (c.max_levels && t < s_ctl.q_count[cur] && s_ctl.q_edges[cur] <= c.max_edges &&
+      v < a.n_rows) {
+    st = col_ptr[v];
+    deg = (uint32_t)(col_ptr[v + 1] - st);
+  }
+  for (uint32_t it = 0; it < c.max_levels; it++) {
+    const uint32_t F = s_ctl.q_count[cur];
+    const uint32_t choice = c.fixed >= 0 ? (uint32_t)c.fixed : s_ctl.choice;
+    // (uniform: every thread reads the same LDS words after a barrier)
+    if (F == 0 || F > c.max_edges || s_ctl.q_edges[cur] > c.max_edges ||
+        (choice != BFSX_LLB && choice != BFSX_SLB))
+      break;
+    const int32_t next_level = (int32_t)s_ctl.level + 1;
+    const uint32_t *q_in = c.queue[cur];
+    uint32_t *q_out = c.queue[cur ^ 1];
+    if (t == 0) {
+      s_count = 0;
+      s_edges = 0;
+    }
+    unsigned long long dacc = 0;
+    for (uint32_t e0 = 0; e0 < F; e0 += SOLO_WG) {
+      if (e0 > 0) {
+        deg = 0;
+        if (e0 + t < F) {
+          v = q_in[e0 + t];
+          if (v < a.n_rows) {
+            st = col_ptr[v];
+            deg = (uint32_t)(col_ptr[v + 1] - st);
+          }
+        }
+      }
+      uint32_t total;
+      const uint32_t ex = block_excl_scan<SOLO_WG>(deg, total, s_wave);
+      s_scan[t] = ex;
+      s_start[t] = st;
+      s_v[t] = v;
+      __syncthreads();
+      for (uint32_t r0 = 0; r0 < total; r0 += SOLO_WG * EPT) {
+        const uint32_t base = r0 + t * EPT;
+        uint32_t j = 0;
+#pragma unroll
+        for (uint32_t step = SOLO_WG / 2; step > 0; step >>= 1)
+          if (s_scan[j + step] <= base) j += step;
+        uint32_t from[EPT], n[EPT], word[EPT], bit[EPT];
+        PtrT at[EPT];
+        bool cand[EPT];
+#pragma unroll
+        for (int k = 0; k < EPT; k++) {
+          const uint32_t e = base + k;
+          cand[k] = e < total;
+          while (cand[k] && j + 1 < SOLO_WG && s_scan[j + 1] <= e) j++;
+          at[k] = cand[k] ? s_start[j] + (PtrT)(e - s_scan[j]) : PtrT(0);
+          from[k] = s_v[j];
+        }
+        // (past the end: entry 0's vertex, read and not used; no branch
+        // around a load, so that the four are in flight together)
+#pragma unroll
+        for (int k = 0; k < EPT; k++) n[k] = a.row_idx[at[k]];
+#pragma unroll
+        for (int k = 0; k < EPT; k++) word[k] = a.vis[n[k] >> 5];
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < EPT; k++) {
+          bit[k] = 1u << (n[k] & 31);
+          cand[k] = cand[k] && !(word[k] & bit[k]);
+          any = any || cand[k];
+        }
+        uint32_t cnt = 0;
+        uint32_t ndeg[EPT];
+        PtrT nstart[EPT];
+        if (any) {
+          uint32_t old[EPT];
+          PtrT end[EPT];
+          // two edges of one lane to one vertex stay exact-once: a thread's
+          // atomics on one address take effect in order
+#pragma unroll
+          for (int k = 0; k < EPT; k++)
+            old[k] = __hip_atomic_fetch_or(&a.vis[n[k] >> 5], cand[k] ? bit[k] : 0u,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+          for (int k = 0; k < EPT; k++) {
+            const uint32_t m = n[k] < a.n_rows ? n[k] : 0u;
+            nstart[k] = col_ptr[m];
+            end[k] = col_ptr[m + 1];
+          }
+#pragma unroll
+          for (int k = 0; k < EPT; k++) {
+            cand[k] = cand[k] && !(old[k] & bit[k]);
+            ndeg[k] = n[k] < a.n_rows ? (uint32_t)(end[k] - nstart[k]) : 0u;
+            if (cand[k]) {
+              a.levels[n[k]] = next_level;
+              if (a.parents) a.parents[n[k]] = from[k];
+              dacc += ndeg[k];
+              cnt++;
+            }
+          }
+        }
+        const uint32_t incl = wave_incl_scan(cnt);
+        uint32_t slot = 0;
+        if (lane == 63 && incl) slot = atomicAdd(&s_count, incl);
+        slot = __shfl(slot, 63, 64) + incl - cnt;
+        if (cnt) {
+#pragma unroll
+          for (int k = 0; k < EPT; k++)
+            if (cand[k]) {
+              q_out[slot] = n[k];
+              if (slot < SOLO_WG) {
+                s_nv[slot] = n[k];
+                s_nstart[slot] = nstart[k];
+                s_ndeg[slot] = ndeg[k];
+              }
+              slot++;
+            }
+        }
+      }
+      __syncthreads();  // this tile's arrays are no longer read
+    }
+    dacc = wave_sum(dacc);
+    if (lane == 0 && dacc) atomicAdd(&s_edges, dacc);
+    __syncthreads();
+    const uint32_t found = s_count;
+    deg = 0;
+    if (t < found) {
+      v = s_nv[t];
+      st = s_nstart[t];
+      deg = s_ndeg[t];
+    }
+    if (t == 0) {
+      s_ctl.q_count[cur ^ 1] = found;
+      s_ctl.q_edges[cur ^ 1] = s_edges;
+    }
+    level_end_body(&s_ctl, cur, cur ^ 1, 0, (int)choice, c.Wg, c.n_cols, c.nnz, c.n_iso, c.allow,
+                   1, SpecGuard{nullptr, 0, 0, NEVER_MARKS}, nullptr, s_W4);
+    __syncthreads();
+    prev_F = F;
+    cur ^= 1;
+  }
+  __syncthreads();
+  if (t == 0) write_level_end(&s_ctl, cur, prev_F, c.mirror);
+  __syncthreads();
+  if (t < CTL_WORDS)
+    reinterpret_cast<uint32_t *>(ctl)[t] = reinterpret_cast<const uint32_t *>(&s_ctl)[t];
 }
 
 // Vertex counts and out-degree sums per level: out[0] = deepest level + 1,
@@ -2900,6 +3119,37 @@ bool coop_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool le
   c.allow = allow;
   c.mirror = ctx->d_mirror;
   return ctx->ptr_bytes == 8 ? coop_levels_t<uint64_t>(ctx, a, c) : coop_levels_t<uint32_t>(ctx, a, c);
+}
+
+void solo_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool learned,
+                 uint32_t *parents, uint32_t max_levels) {
+  KArgs a{};
+  a.col_ptr = ctx->col_ptr.p;
+  a.row_idx = ctx->row_idx.as<uint32_t>();
+  a.n_rows = ctx->n_rows;
+  a.n_cols = ctx->n_cols;
+  a.vis = ctx->vis.as<uint32_t>();
+  a.levels = ctx->levels.as<int32_t>();
+  a.parents = parents;
+  SoloArgs c{};
+  c.queue[0] = ctx->queue[0].as<uint32_t>();
+  c.queue[1] = ctx->queue[1].as<uint32_t>();
+  c.cur = cur;
+  c.fixed = fixed;
+  c.max_edges = SOLO_EDGES;
+  c.max_levels = max_levels;
+  c.Wg = learned ? ctx->sched_w.as<float>() : nullptr;
+  c.n_cols = ctx->n_cols;
+  c.nnz = ctx->nnz;
+  c.n_iso = (ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols ? ctx->n_isolated : 0;
+  c.allow = allow;
+  c.mirror = ctx->d_mirror;
+  LevelCtl *ctl = ctx->ctl.as<LevelCtl>();
+  if (ctx->ptr_bytes == 8)
+    hipLaunchKernelGGL(k_solo_levels<uint64_t>, dim3(1), dim3(SOLO_WG), 0, ctx->stream, a, ctl, c);
+  else
+    hipLaunchKernelGGL(k_solo_levels<uint32_t>, dim3(1), dim3(SOLO_WG), 0, ctx->stream, a, ctl, c);
+  BFSX_HIP(hipGetLastError());
 }
 
 void level_histogram(bfsx_ctx *ctx, uint32_t max_levels, unsigned long long *d_out) {

@@ -174,12 +174,16 @@ static void view_from_ctl(bfsx_ctx *ctx, uint32_t produced) {
   ctx->view.choice = c.choice;
   ctx->view.done = c.done;
   ctx->view.level = c.level & MIRROR_LEVEL_MASK;
+  ctx->view.n_llb = c.kind_count[BFSX_LLB] & MIRROR_KIND_MASK;
+  ctx->view.n_slb = c.kind_count[BFSX_SLB] & MIRROR_KIND_MASK;
+  ctx->view.VV = c.visited_vertices;
+  ctx->view.prev_F = 0;  // (not kept in the block)
 }
 
 // After a launch that ends with k_level_end: that kernel writes the values
 // the host needs into the host-mapped mirror, every word tagged with its
 // sequence number, so the host polls the words (no copy, no stream
-// synchronisation) until all four carry `seq` -- a word of the previous
+// synchronisation) until all of them carry `seq` -- a word of the previous
 // level end next to a new one means the new ones have not all arrived.
 // After a second without them, the stream is synchronised, which reports any
 // device error, and the values come from a full copy of the control block.
@@ -188,8 +192,10 @@ void read_level_end(bfsx_ctx *ctx, uint32_t seq, uint32_t produced, uint32_t lev
   const unsigned long long t32 = seq, t16 = seq & 0xFFFFu;
   const auto t0 = std::chrono::steady_clock::now();
   auto take = [&]() {
-    const unsigned long long w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
-    if (!((w0 >> 32) == t32 && (w1 >> 48) == t16 && (w2 >> 48) == t16 && (w3 >> 32) == t32))
+    const unsigned long long w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3], w4 = w[4], w5 = w[5],
+                             w6 = w[6];
+    if (!((w0 >> 32) == t32 && (w1 >> 48) == t16 && (w2 >> 48) == t16 && (w3 >> 32) == t32 &&
+          (w4 >> 48) == t16 && (w5 >> 48) == t16 && (w6 >> 32) == t32))
       return false;
     ctx->view.F = (uint32_t)w0;
     ctx->view.EF = w1 & MIRROR_48;
@@ -197,6 +203,10 @@ void read_level_end(bfsx_ctx *ctx, uint32_t seq, uint32_t produced, uint32_t lev
     ctx->view.choice = (uint32_t)(w3 & 0xFFu);
     ctx->view.done = (uint32_t)((w3 >> 8) & 1u);
     ctx->view.level = (uint32_t)((w3 >> 9) & MIRROR_LEVEL_MASK);
+    ctx->view.n_llb = (uint32_t)w4 & MIRROR_KIND_MASK;
+    ctx->view.n_slb = (uint32_t)(w4 >> 24) & MIRROR_KIND_MASK;
+    ctx->view.VV = w5 & MIRROR_48;
+    ctx->view.prev_F = (uint32_t)w6;
     return true;
   };
   for (uint32_t spin = 0;; spin++) {
@@ -389,11 +399,13 @@ struct Walker {
 
 static uint32_t allow_mask(const Walker &w) { return 0x7u | (w.pull_possible ? 0x8u : 0u); }
 
-// Initial state of a search (levels, visited bitmap, queue, control block),
-// read back so that the root's degree is known; frontier degree sums are
-// always kept, since they decide between mark and exact-once discovery.
+// Initial state of a search (levels, visited bitmap, queue, control block);
+// frontier degree sums are always kept, since they decide between mark and
+// exact-once discovery.  With read, the control block is copied back, so
+// that the root's degree is known; otherwise the caller learns it from the
+// level-end words of the launch that follows (solo_levels).
 static Walker start_search(bfsx_ctx *ctx, uint32_t root, bool pull_possible, bool stamp,
-                           uint32_t *par) {
+                           uint32_t *par, bool read = true) {
   if (!ctx->has_graph) fail(BFSX_ERR_STATE, "no graph uploaded");
   if (root >= ctx->n_cols) fail(BFSX_ERR_ARG, "root out of range");
   hipStream_t s = ctx->stream;
@@ -403,8 +415,11 @@ static Walker start_search(bfsx_ctx *ctx, uint32_t root, bool pull_possible, boo
     ctx->mark_dirty = false;
   }
   init_search(ctx, root, graph_symmetric(ctx), par);
-  read_ctl(ctx);
-  view_from_ctl(ctx, 0);
+  if (read) {
+    ctx->seq_known = false;  // (until a search in the host loop ends)
+    read_ctl(ctx);
+    view_from_ctl(ctx, 0);
+  }
   Walker w;
   w.ctx = ctx;
   w.pull_possible = pull_possible;
@@ -544,17 +559,19 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
   }
   if (want_parents) ensure(ctx->parents, sizeof(uint32_t) * ctx->n_cols, s);
   uint32_t *par = want_parents ? ctx->parents.as<uint32_t>() : nullptr;
+  if (!ctx->seq_known) {
+    read_ctl(ctx);
+    ctx->seq = ctx->h_ctl->seq;
+  }
   // initial state outside the timer (host.cpp:113-121 / run_bfs_gpu.hpp:674-677)
   Walker w = start_search(ctx, root, fixed == BFSX_PULL || ((learned || beamer) && symmetric),
-                          false, par);
+                          false, par, timed);
   BeamerRule rule;
   w.count = timed;
-  BFSX_HIP(hipStreamSynchronize(s));
   ctx->trace.clear();
 
   RunOut out;
   out.reached = 1;  // the root
-  BFSX_HIP(hipEventRecord(ctx->ev0, s));
   uint64_t f_edges = 0, visited_v = 1, visited_e = 0, examined = 0;
   // The root level (one vertex) runs LLB, the choice k_init leaves in the
   // control block, with no network evaluation or extra round trip; every
@@ -562,18 +579,50 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
   w.decide_allow = learned ? allow_mask(w) : 0u;
   w.decide_reuse = true;
   if (trace) {
-    read_ctl(ctx);
     f_edges = ctx->h_ctl->q_edges[0];
     visited_e = ctx->h_ctl->visited_edges;
   }
-  uint32_t seq = ctx->h_ctl->seq;  // level ends so far (h_ctl: the block k_init wrote)
-  uint32_t decisions = ctx->h_ctl->decisions;
+  uint32_t seq = ctx->seq;  // level ends so far
+  ctx->seq_known = false;   // until this search has read its last one
+  uint32_t decisions = timed ? ctx->h_ctl->decisions : 0;
   const bool dev_loop = (flags & BFSX_RUN_DEVICE_LOOP) && ctx->coop_ok;
   const MarkRule mr = mark_rule(ctx);
   // speculative steps (see Walker::launch_speculative_pull / _td)
   const bool can_spec = ctx->params.speculate && learned && !timed;
   int spec = -1;  // the kind speculated for level w.level: BFSX_PULL, BFSX_LLB (LLB or SLB) or -1
   uint64_t prev_F = 1;  // the previous level's frontier size
+  // Tiny levels run in one work-group's loop on the device (not with
+  // per-level traces, for kinds that name another kernel, or where every
+  // level has to mark).  Its words are also how an untimed search learns its
+  // first state: the launch follows k_init without a host round trip, and
+  // has run the first levels when the host reads it.
+  const bool solo_ok = !timed && !dev_loop && ctx->params.mark_ratio_q10 != 0 &&
+                       (learned || (!beamer && (fixed == BFSX_LLB || fixed == BFSX_SLB)));
+  auto solo = [&](uint32_t max_levels) {
+    const uint32_t level0 = w.level;
+    solo_levels(ctx, w.cur, learned ? -1 : fixed, w.decide_allow, learned, par, max_levels);
+    read_level_end(ctx, ++seq, w.cur, level0);
+    const uint32_t ran = (ctx->view.level - level0) & MIRROR_LEVEL_MASK;
+    w.cur ^= ran & 1u;
+    w.level += ran;
+    w.F = ctx->view.F;
+    w.EF = ctx->view.EF;
+    w.VE = ctx->view.VE;
+    out.reached = ctx->view.VV;
+    out.n_levels += ran;
+    out.steps[BFSX_LLB] += (ctx->view.n_llb - out.steps[BFSX_LLB]) & MIRROR_KIND_MASK;
+    out.steps[BFSX_SLB] += (ctx->view.n_slb - out.steps[BFSX_SLB]) & MIRROR_KIND_MASK;
+    if (ran > 0) {
+      w.fbm_valid = false;
+      w.queue_valid = true;
+      w.last = BFSX_LLB;
+      prev_F = ctx->view.prev_F;
+    }
+  };
+  constexpr uint32_t SOLO_LEVELS = 4096;  // per launch
+  if (!timed && !solo_ok) solo(0);
+  BFSX_HIP(hipEventRecord(ctx->ev0, s));
+  if (solo_ok) solo(SOLO_LEVELS);
   while (w.F > 0) {
     // a search has at most n_cols levels; more means a broken invariant
     if (w.level > ctx->n_cols) fail(BFSX_ERR_DEVICE, "level loop did not terminate");
@@ -602,7 +651,21 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
         }
       }
     }
+    const bool spec_ran = (spec == BFSX_PULL && choice == BFSX_PULL) ||
+                          (spec == BFSX_LLB && (choice == BFSX_LLB || choice == BFSX_SLB) &&
+                           !mr.marks(w.EF, w.F));
+    if (solo_ok && !spec_ran && (choice == BFSX_LLB || choice == BFSX_SLB) &&
+        w.EF <= SOLO_EDGES && w.F <= SOLO_EDGES) {
+      // (a speculative step that was not picked exits without a write)
+      if (!w.queue_valid)
+        bitmap_to_queue(ctx, ctx->fbm[w.fbm_cur].as<uint32_t>(),
+                        ctx->queue[w.cur].as<uint32_t>());
+      spec = -1;
+      solo(SOLO_LEVELS);
+      continue;
+    }
     const uint32_t level = w.level, F = w.F, cur = w.cur;
+    const unsigned long long EF = w.EF;
     // the decision in force for this level (made at the previous level's end)
     bfsx_level_record r{};
     if (trace && learned) {
@@ -613,13 +676,10 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
     }
     if (timed) BFSX_HIP(hipEventRecord(ctx->ev_step0, s));
     bool new_fbm;
-    if (spec == BFSX_PULL && choice == BFSX_PULL) {
+    if (spec_ran) {
       // this level's step is the speculative one already in the stream
-      new_fbm = true;
-      w.last = BFSX_PULL;
-    } else if (spec == BFSX_LLB && (choice == BFSX_LLB || choice == BFSX_SLB) &&
-               !mr.marks(w.EF, w.F)) {
-      new_fbm = false;  // (the speculative top-down step writes the queue only)
+      // (a bottom-up one writes the bitmap, a top-down one only the queue)
+      new_fbm = choice == BFSX_PULL;
       w.last = choice;
     } else {
       // (a speculative step that was not picked exits without a write)
@@ -630,13 +690,15 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
     // or marking: heavy, and usually followed by bottom-up levels); a thin
     // top-down step after another top-down step whose frontier did not grow
     // more than twofold (the tail of a search, a grid), not while the
-    // frontier grows fast (a guess that fails costs its empty launches).
+    // frontier grows fast (a guess that fails costs its empty launches), nor
+    // where the next level is likely one for the solo loop, which then runs
+    // it and the rest of the search in one launch.
     spec = -1;
     if (can_spec && w.pull_possible && (choice == BFSX_PULL || new_fbm)) {
       w.launch_speculative_pull();
       spec = BFSX_PULL;
     } else if (can_spec && !dev_loop && choice != BFSX_PULL && !par && level > 0 &&
-               (uint64_t)F <= 2ull * prev_F) {
+               (uint64_t)F <= 2ull * prev_F && !(solo_ok && EF <= 2 * SOLO_EDGES)) {
       w.launch_speculative_td(mr);
       spec = BFSX_LLB;
     }
@@ -680,6 +742,8 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
   BFSX_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   out.ms = ms;
   out.edges = w.VE;
+  ctx->seq = seq;
+  ctx->seq_known = true;
   if (dev_loop) {  // the device loop's levels were counted on the device
     read_ctl(ctx);
     for (int k = 0; k < BFSX_N_STEP_KINDS; k++) out.steps[k] = ctx->h_ctl->kind_count[k];

@@ -60,26 +60,30 @@ static_assert(offsetof(LevelCtl, seq) + sizeof(uint32_t) == sizeof(LevelCtl),
               "seq is the last field: resets and restores cover the bytes before it");
 constexpr size_t CTL_RESET_BYTES = offsetof(LevelCtl, seq);
 
-// What the host reads at a level end without synchronising the stream: four
+// What the host reads at a level end without synchronising the stream:
 // 8-byte words in host-mapped memory, written by the level-end kernel.
 // Device writes to host memory can reach it out of order even across a
 // system-scope fence, so every word carries the level end's sequence number
-// and the host takes the words only once all four carry the number it waits
-// for (an 8-byte aligned store arrives whole).
+// and the host takes the words only once all of them carry the number it
+// waits for (an 8-byte aligned store arrives whole).
 //   w[0] = seq << 32 | frontier size (count of the produced queue)
 //   w[1] = (seq & 0xFFFF) << 48 | frontier edges (48 bits)
 //   w[2] = (seq & 0xFFFF) << 48 | edges of the visited vertices (48 bits)
 //   w[3] = seq << 32 | next step kind (8 bits) | done << 8 | level << 9
 //          (the level of the next frontier, 23 bits)
+//   w[4] = (seq & 0xFFFF) << 48 | levels run as SLB (24 bits) << 24 | as LLB
+//   w[5] = (seq & 0xFFFF) << 48 | vertices visited (48 bits)
+//   w[6] = seq << 32 | size of the frontier that the level expanded
 // Two such sets alternate by the parity of seq: a level end launched ahead
 // of the host's read of the previous one (a speculative step) writes the
 // other set, so it cannot overwrite words the host has not read yet.
 struct LevelMirror {
-  unsigned long long w[4];
+  unsigned long long w[8];  // (w[7] unused: a set is one 64-byte line)
 };
 constexpr int MIRROR_SLOTS = 2;
 constexpr unsigned long long MIRROR_48 = (1ull << 48) - 1;
 constexpr uint32_t MIRROR_LEVEL_MASK = (1u << 23) - 1;
+constexpr uint32_t MIRROR_KIND_MASK = (1u << 24) - 1;
 
 // Whether a top-down level marks and compacts or discovers exact-once.  A
 // level marks from hi_E frontier edges on, and from lo_E on when its
@@ -104,6 +108,9 @@ struct LevelView {
   unsigned long long EF = 0, VE = 0;
   uint32_t choice = 0, done = 0;
   uint32_t level = 0;  // level of the next frontier (23 bits)
+  uint32_t n_llb = 0, n_slb = 0;    // levels of those kinds so far (24 bits)
+  unsigned long long VV = 0;        // vertices visited
+  uint32_t prev_F = 0;              // size of the frontier last expanded
 };
 
 // Bitmaps hold whole 1024-vertex chunks (32 words) so that a wave can own a
@@ -189,6 +196,11 @@ struct bfsx_ctx {
   bfsx::LevelMirror *h_mirror = nullptr;  // pinned, host-mapped: tagged level-end words (2 sets)
   bfsx::LevelMirror *d_mirror = nullptr;  // device address of h_mirror (k_level_end writes it)
   bfsx::LevelView view;                   // the values of the last level end the host read
+  // level ends so far (LevelCtl::seq), while the host knows it: a search
+  // that ran to its end knows the next one's first sequence number without
+  // reading the control block
+  uint32_t seq = 0;
+  bool seq_known = false;
   bool mark_dirty = false;          // a mark step did not reach its compaction
 
   // learned scheduler weights and the snapshot used to time alternatives
@@ -338,6 +350,16 @@ void level_begin(bfsx_ctx *ctx);
 // False when the device cannot launch cooperatively.
 bool coop_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool learned,
                  MarkRule mark, uint32_t max_levels);
+// The same with one work-group and no barrier between groups, for frontiers
+// of at most SOLO_EDGES edges (max_levels 0: the level-end words only).  The
+// line: beyond about 2 K edges a launch over several work-groups is faster
+// although it costs its dispatch (a 512 x 512 grid, learned, whole search:
+// 2.60 ms at 512 edges, 2.48 at 2 K, 2.69 at 4 K, 3.45 at 8 K, 2.98 without
+// this loop; R-MAT 12 205 -> 135 us, R-MAT 16 251 -> 165 us).
+constexpr uint32_t SOLO_EDGES = 2048;
+void solo_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool learned,
+                 uint32_t *parents, uint32_t max_levels);
+
 // Waits for the level end with sequence number `seq` (the tagged host-mapped
 // words) and leaves its values in ctx->view; `produced` = the queue buffer
 // the level filled (for the synchronising fallback).

@@ -431,6 +431,8 @@ __global__ void k_ms_end(LevelCtl *ctl, uint32_t qi, LevelMirror *mirror) {
   mirror->w[1] = t16 | (ctl->q_edges[qo] & MIRROR_48);
   mirror->w[2] = t16 | (ctl->overflow ? 1ull : 0ull);
   mirror->w[3] = t32 | (ctl->choice & 0xFFu) | ((unsigned long long)(ctl->done ? 1u : 0u) << 8);
+  mirror->w[4] = mirror->w[5] = t16;  // (not used by a batch)
+  mirror->w[6] = t32;
   __threadfence_system();
 }
 
@@ -724,6 +726,7 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
     ctx->ms_key = key;
   }
 
+  ctx->seq_known = false;
   // the timed level loop: one graph launch per K levels, the termination
   // flag read from the tagged level-end words
   MsResult r;

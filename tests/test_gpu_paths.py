@@ -53,3 +53,42 @@ def test_level_histogram_edges(engine, name):
         counts, edges = engine.level_histogram(size)
         assert (counts == hist).all()
         assert (edges == np.bincount(want[want >= 0], weights=deg[want >= 0])).all()
+
+
+# tiny levels run in one work-group: tiles of 1024 frontier entries, up to
+# 2048 edges a level, 4096 levels a launch
+@pytest.mark.parametrize("name", ["one", "path2500", "path9001", "star70001", "directed4099",
+                                  "hub1023", "hub1025", "hub2045", "hub2048", "hub2049", "hub4097"])
+def test_tiny_levels_loop(engine, name):
+    say("tiny levels", name)
+    if name.startswith("hub"):
+        # a hub at the end of a path whose k leaves share one far vertex
+        k = int(name[3:])
+        src = np.concatenate([[0, 1], np.full(k, 2), np.arange(k) + 3])
+        dst = np.concatenate([[1, 2], np.arange(k) + 3, np.full(k, k + 3)])
+        cp, ri = csc_from_edges(k + 4, *symmetrize(src, dst))
+        n_rows, sym, root = k + 4, True, 0
+    elif name == "path9001":
+        cp, ri, n_rows, sym, root = *path_graph(9001), 9001, True, 4500
+    else:
+        cp, ri, n_rows, sym, root = some_graph(name)
+    engine.upload_csc(cp, ri, n_rows=n_rows, symmetric=sym)
+    want, ec, _ = cpu.bfs_queue(cp, ri, root, n_rows=n_rows)
+    engine.load_scheduler()
+    try:
+        for s, kw in [("llb", {}), ("slb", {}), ("learned", {}), ("llb", {"hub_degree": 512}),
+                      ("llb", {"mark_ratio_q10": 0}), ("slb", {"mark_ratio_q10": 0xFFFFFFFF})]:
+            before = engine.params
+            if kw:
+                engine.set_params(**kw)
+            lev, st, par = engine.run(root, s, parents=True)
+            engine.set_params(**before)
+            assert (lev == want).all(), (s, kw)
+            assert cpu.check_parents(cp, ri, root, want, par, n_rows=n_rows) == 0
+            assert [st[k] for k in ("edges_count", "reached", "max_level", "n_levels")] == [
+                ec, int((want >= 0).sum()), int(want.max()), int(want.max()) + 1]
+            assert sum(st["steps"].values()) == st["n_levels"]
+            if s != "learned":
+                assert st["steps"][s] == st["n_levels"]
+    finally:
+        engine.set_scheduler_weights(None)
