@@ -152,6 +152,7 @@ struct KArgs {
   int32_t next_level;
   uint32_t hub_degree;
   uint8_t *mark;      // non-null: mark-then-compact mode
+  bool mark_probe;    // mark mode: read a target's mark byte before storing it
   unsigned long long *examined;  // nullable: bottom-up adjacency entries read
   // mark mode only: row_idx is the hot copy; a flagged entry names hot
   // vertex hot_id[h], whose visited bit is bit h of hot_vis (null: plain ids)
@@ -329,12 +330,24 @@ __device__ __forceinline__ void expand_edges(const KArgs &a, const PtrT *col_ptr
         const uint32_t *p = probe_word<HOT>(a, n[k], idx[k]);
         w[k] = valid[k] ? *p : ~0u;
       }
+      uint32_t v[EPT];
+      uint8_t m[EPT];
+#pragma unroll
+      for (int k = 0; k < EPT; k++) {
+        valid[k] = valid[k] && !((w[k] >> (idx[k] & 31)) & 1u);
+        v[k] = valid[k] ? entry_vertex<HOT>(a, n[k]) : 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < EPT; k++) m[k] = 0;
+      if (a.mark_probe) {  // (uniform)
+#pragma unroll
+        for (int k = 0; k < EPT; k++) m[k] = a.mark[v[k]];
+      }
 #pragma unroll
       for (int k = 0; k < EPT; k++)
-        if (valid[k] && !((w[k] >> (idx[k] & 31)) & 1u)) {
-          const uint32_t v = entry_vertex<HOT>(a, n[k]);
-          a.mark[v] = 1;
-          if (a.parents) a.parents[v] = from[k];
+        if (valid[k] && !m[k]) {
+          a.mark[v[k]] = 1;
+          if (a.parents) a.parents[v[k]] = from[k];
         }
     } else {
 #pragma unroll
@@ -365,12 +378,34 @@ struct LlbShared {
   uint32_t hub[WG];
 };
 
+// Work-groups that share one tile of WG frontier entries: each scans the
+// tile's degrees again (5 KB of queue and col_ptr reads at WG 256) and
+// expands its slice of the edges.  With one group per tile a level's groups
+// are as few as its frontier is small: R-MAT 22's second level has 99 K
+// vertices, 387 tiles of 190 K edges each for 256 CUs, and a first level of
+// a dozen hubs is a single tile.  The line lies at LLB_ROUNDS rounds of a
+// group's edges on average, so that a level of thin tiles (a grid's) keeps
+// one group per tile.  Measured on the step kernel (frontier, edges): 214,
+// 160 K at R-MAT 16 229 -> 12 us; 7.6 K, 5.5 M at R-MAT 19 343 -> 39 us;
+// 78, 763 K at R-MAT 24 1507 -> 44 us; whole fixed-LLB searches of R-MAT 16 /
+// 19 / 22 / 24: 282 / 511 / 1855 / 8159 -> 112 / 180 / 1095 / 4661 us.
+constexpr uint32_t LLB_ROUNDS = 4, LLB_MAX_PARTS = 64;
+__host__ __device__ inline uint32_t llb_parts(unsigned long long EF, uint32_t n_tiles,
+                                              uint32_t wg) {
+  const unsigned long long per = (unsigned long long)wg * EPT * LLB_ROUNDS * n_tiles;
+  const unsigned long long p = per ? (EF + per - 1) / per : 1;
+  return p < 1 ? 1u : p > LLB_MAX_PARTS ? LLB_MAX_PARTS : (uint32_t)p;
+}
+
 // One LLB tile: WG frontier entries (contiguous, or strided by n_tiles for
-// SLB), block scan of their degrees, cooperative expansion of their edges.
+// SLB), block scan of their degrees, cooperative expansion of their edges
+// (of slice `part` of n_parts; a slice holds at least one round of edges, so
+// the later parts of a small tile have none).
 template <typename PtrT, int WG, bool HOT = false>
 __device__ __forceinline__ void llb_tile(const KArgs &a, LlbShared<PtrT, WG> &sh, uint32_t tile,
                                          uint32_t n_tiles, bool strided,
-                                         unsigned long long &dacc, bool have_v0 = false,
+                                         unsigned long long &dacc, uint32_t part = 0,
+                                         uint32_t n_parts = 1, bool have_v0 = false,
                                          uint32_t v0 = 0) {
   constexpr int NW = WG / 64;
   PtrT *s_start = sh.start;
@@ -407,27 +442,39 @@ __device__ __forceinline__ void llb_tile(const KArgs &a, LlbShared<PtrT, WG> &sh
   __syncthreads();
   // owner of edge i = last slot j with s_scan[j] <= i (empty slots tie with
   // the next one and are skipped by taking the last)
-  expand_edges<PtrT, WG, true, HOT>(a, col_ptr, s_scan, s_start, s_v, PtrT(0), total, dacc);
+  PtrT lo = 0, hi = total;
+  if (n_parts > 1) {
+    constexpr PtrT ROUND = (PtrT)WG * EPT;
+    PtrT per = total / n_parts + 1;  // (sums that fit PtrT whatever total is)
+    per = per < ROUND ? ROUND : (per + EPT - 1) / EPT * EPT;
+    lo = part < total / per + 1 ? (PtrT)part * per : total;
+    hi = total - lo > per ? lo + per : total;
+  }
+  expand_edges<PtrT, WG, true, HOT>(a, col_ptr, s_scan, s_start, s_v, lo, hi, dacc);
   if (a.hub_degree) {
     const uint32_t nh = s_hub_n;
     const uint32_t w = t >> 6, l = t & 63;
+    // (each of the tile's groups lists its hubs in an order of its own: the
+    // groups share every hub's edges, not the list)
     for (uint32_t h = w; h < nh; h += NW) {
       const uint32_t slot = s_hub[h];
       const PtrT b = s_start[slot];
-      const PtrT e1 = col_ptr[s_v[slot] + 1];
-      for (PtrT e = b + l; e < e1; e += 64)
-        discover<PtrT, HOT>(a, col_ptr, a.row_idx[e], s_v[slot], dacc);
+      const PtrT len = col_ptr[s_v[slot] + 1] - b;
+      for (PtrT e = l + 64 * part; e < len; e += 64 * n_parts)
+        discover<PtrT, HOT>(a, col_ptr, a.row_idx[b + e], s_v[slot], dacc);
     }
   }
 }
 
-// Host-sized launch: one tile per work-group, grid = ceil(F / WG).  The
-// degree sum of exact-once discoveries leaves with one atomic per group.
+// Host-sized launch: one part of a tile per work-group, grid =
+// ceil(F / WG) * parts.  The degree sum of exact-once discoveries leaves
+// with one atomic per group.
 template <typename PtrT, int WG, bool STRIDED, bool HOT>
-__global__ __launch_bounds__(WG) void k_llb(KArgs a) {
+__global__ __launch_bounds__(WG) void k_llb(KArgs a, uint32_t n_tiles, uint32_t n_parts) {
   __shared__ LlbShared<PtrT, WG> sh;
   unsigned long long dacc = 0;
-  llb_tile<PtrT, WG, HOT>(a, sh, blockIdx.x, gridDim.x, STRIDED, dacc);
+  llb_tile<PtrT, WG, HOT>(a, sh, blockIdx.x % n_tiles, n_tiles, STRIDED, dacc,
+                          blockIdx.x / n_tiles, n_parts);
   if (a.q_out_edges && !a.mark) block_atomic_add<WG>(dacc, a.q_out_edges);
 }
 
@@ -471,10 +518,14 @@ __global__ __launch_bounds__(WG) void k_td_dev(KArgs a, LevelCtl *ctl, DevStep d
   a.next_level = (int32_t)h0.z + 1;
   if (!marks) a.mark = nullptr;
   const uint32_t n_tiles = (F + WG - 1) / WG;
+  const uint32_t n_parts = llb_parts(c_edges, n_tiles, WG);
   const bool llb = choice == BFSX_LLB;
   unsigned long long dacc = 0;
-  for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x)
-    llb_tile<PtrT, WG>(a, sh, tile, n_tiles, !llb, dacc, llb && tile == blockIdx.x, v0);
+  for (uint64_t i = blockIdx.x; i < (uint64_t)n_tiles * n_parts; i += gridDim.x) {
+    const uint32_t tile = (uint32_t)(i % n_tiles);
+    llb_tile<PtrT, WG>(a, sh, tile, n_tiles, !llb, dacc, (uint32_t)(i / n_tiles), n_parts,
+                       llb && tile == blockIdx.x, v0);
+  }
   if (a.q_out_edges && !a.mark) block_atomic_add<WG>(dacc, a.q_out_edges);
 }
 
@@ -2232,9 +2283,11 @@ __global__ __launch_bounds__(WG) void k_coop_levels(KArgs base, LevelCtl *ctl, C
     a.next_level = (int32_t)ctl->level + 1;
     a.mark = nullptr;
     const uint32_t n_tiles = (F + WG - 1) / WG;
+    const uint32_t n_parts = llb_parts(EF, n_tiles, WG);
     unsigned long long dacc = 0;
-    for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x)
-      llb_tile<PtrT, WG>(a, sh, tile, n_tiles, choice == BFSX_SLB, dacc);
+    for (uint64_t i = blockIdx.x; i < (uint64_t)n_tiles * n_parts; i += gridDim.x)
+      llb_tile<PtrT, WG>(a, sh, (uint32_t)(i % n_tiles), n_tiles, choice == BFSX_SLB, dacc,
+                         (uint32_t)(i / n_tiles), n_parts);
     block_atomic_add<WG>(dacc, a.q_out_edges);
     grid_barrier_last(ctl, gridDim.x, [&] {
       level_end_body(ctl, cur, cur ^ 1, 0, choice, c.Wg, c.n_cols, c.nnz, c.n_iso, c.allow, 1,
@@ -2593,6 +2646,15 @@ static KArgs kargs(const StepArgs &s, uint32_t hub) {
   a.next_level = s.next_level;
   a.hub_degree = hub;
   a.mark = s.mark;
+  // Where many edges lead to each new vertex and the marks do not stay in an
+  // XCD's L2 (4 MB), a read of the mark byte (mostly a line this XCD already
+  // holds) saves the store, which the L2 has to write back line by line in
+  // all eight XCDs: R-MAT 22's second level (62 M edges, 2 M new vertices)
+  // 758 -> 555 us, R-MAT 24's (339 M, 7.6 M) 4715 -> 3763 us.  With fewer
+  // edges per new vertex the extra read costs more than the stores it saves
+  // (16 M edges, 0.75 M new of 1.5 M: 102 -> 137 us), as on levels whose
+  // targets are mostly visited already (R-MAT 22's third: 342 -> 360 us).
+  a.mark_probe = s.mark && s.n_cols >= (1u << 21) && s.EF >= 8ull * s.n_cols && !s.hot_ok;
   a.examined = s.count_examined ? &s.ctl->examined : nullptr;
   a.hot_vis = nullptr;
   a.hot_id = nullptr;
@@ -2614,16 +2676,18 @@ __global__ void k_hot_bits(const uint32_t *vis, const uint32_t *hot_id, uint32_t
 }
 
 template <typename PtrT, bool STRIDED, bool HOT>
-static void launch_llb_t(bfsx_ctx *ctx, const KArgs &a) {
+static void launch_llb_t(bfsx_ctx *ctx, const KArgs &a, unsigned long long EF) {
   const uint32_t wg = ctx->params.llb_wg;
-  const unsigned grid = (unsigned)((a.F + wg - 1) / wg);
+  const uint32_t tiles = (uint32_t)(((uint64_t)a.F + wg - 1) / wg);
+  const uint32_t parts = llb_parts(EF, tiles, wg);
+  const dim3 grid(tiles * parts);  // (below 2^26 tiles of 64; parts follow the edges)
   hipStream_t s = ctx->stream;
   switch (wg) {
-    case 64: hipLaunchKernelGGL((k_llb<PtrT, 64, STRIDED, HOT>), dim3(grid), dim3(64), 0, s, a); break;
-    case 128: hipLaunchKernelGGL((k_llb<PtrT, 128, STRIDED, HOT>), dim3(grid), dim3(128), 0, s, a); break;
-    case 256: hipLaunchKernelGGL((k_llb<PtrT, 256, STRIDED, HOT>), dim3(grid), dim3(256), 0, s, a); break;
-    case 512: hipLaunchKernelGGL((k_llb<PtrT, 512, STRIDED, HOT>), dim3(grid), dim3(512), 0, s, a); break;
-    case 1024: hipLaunchKernelGGL((k_llb<PtrT, 1024, STRIDED, HOT>), dim3(grid), dim3(1024), 0, s, a); break;
+    case 64: hipLaunchKernelGGL((k_llb<PtrT, 64, STRIDED, HOT>), grid, dim3(64), 0, s, a, tiles, parts); break;
+    case 128: hipLaunchKernelGGL((k_llb<PtrT, 128, STRIDED, HOT>), grid, dim3(128), 0, s, a, tiles, parts); break;
+    case 256: hipLaunchKernelGGL((k_llb<PtrT, 256, STRIDED, HOT>), grid, dim3(256), 0, s, a, tiles, parts); break;
+    case 512: hipLaunchKernelGGL((k_llb<PtrT, 512, STRIDED, HOT>), grid, dim3(512), 0, s, a, tiles, parts); break;
+    case 1024: hipLaunchKernelGGL((k_llb<PtrT, 1024, STRIDED, HOT>), grid, dim3(1024), 0, s, a, tiles, parts); break;
     default: fail(BFSX_ERR_ARG, "llb_wg must be 64, 128, 256, 512 or 1024");
   }
 }
@@ -2647,19 +2711,19 @@ void step_llb(bfsx_ctx *ctx, const StepArgs &s, bool strided) {
   const bool hot = a.hot_vis != nullptr;
   if (ctx->ptr_bytes == 8) {
     if (hot) {
-      if (strided) launch_llb_t<uint64_t, true, true>(ctx, a);
-      else launch_llb_t<uint64_t, false, true>(ctx, a);
+      if (strided) launch_llb_t<uint64_t, true, true>(ctx, a, s.EF);
+      else launch_llb_t<uint64_t, false, true>(ctx, a, s.EF);
     } else {
-      if (strided) launch_llb_t<uint64_t, true, false>(ctx, a);
-      else launch_llb_t<uint64_t, false, false>(ctx, a);
+      if (strided) launch_llb_t<uint64_t, true, false>(ctx, a, s.EF);
+      else launch_llb_t<uint64_t, false, false>(ctx, a, s.EF);
     }
   } else {
     if (hot) {
-      if (strided) launch_llb_t<uint32_t, true, true>(ctx, a);
-      else launch_llb_t<uint32_t, false, true>(ctx, a);
+      if (strided) launch_llb_t<uint32_t, true, true>(ctx, a, s.EF);
+      else launch_llb_t<uint32_t, false, true>(ctx, a, s.EF);
     } else {
-      if (strided) launch_llb_t<uint32_t, true, false>(ctx, a);
-      else launch_llb_t<uint32_t, false, false>(ctx, a);
+      if (strided) launch_llb_t<uint32_t, true, false>(ctx, a, s.EF);
+      else launch_llb_t<uint32_t, false, false>(ctx, a, s.EF);
     }
   }
   BFSX_HIP(hipGetLastError());

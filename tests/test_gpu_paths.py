@@ -92,3 +92,36 @@ def test_tiny_levels_loop(engine, name):
                 assert st["steps"][s] == st["n_levels"]
     finally:
         engine.set_scheduler_weights(None)
+
+
+# several work-groups share a tile of frontier entries: tiles of one hub, of
+# hubs beside empty lists, totals that are no multiple of a round or a part
+@pytest.mark.parametrize("leaves", [4096, 4097, 20011, 150001])
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+def test_tiles_shared_by_groups(engine, leaves, ptr):
+    say("shared tiles", leaves, ptr.__name__)
+    rng = np.random.default_rng(leaves)
+    k, n = 29, leaves + 400
+    # root -> k hubs (far apart), each hub -> a random tenth of the leaves
+    hubs = 1 + 13 * np.arange(k)
+    src, dst = [np.zeros(k, np.int64)], [hubs]
+    for h in hubs:
+        to = rng.permutation(np.arange(400, n))[: leaves // 10 + h]
+        src.append(np.full(len(to), h))
+        dst.append(to)
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    for sym in (False, True):
+        e = symmetrize(src, dst) if sym else (src, dst)
+        cp, ri = csc_from_edges(n, *e, dtype=ptr)
+        engine.upload_csc(cp, ri, n_rows=n if sym else n - 7, symmetric=sym)
+        want, ec, _ = cpu.bfs_queue(cp, ri, 0, n_rows=n if sym else n - 7)
+        before = engine.params
+        for kw in ({}, {"llb_wg": 64}, {"llb_wg": 1024}, {"hub_degree": 1024},
+                   {"hub_degree": 16, "llb_wg": 128},
+                   {"mark_ratio_q10": 0}, {"mark_ratio_q10": 0xFFFFFFFF}):
+            engine.set_params(**kw)
+            for s in ("llb", "slb"):
+                for loop in ({}, {"parents": True}, {"graph_loop": True}, {"device_loop": True}):
+                    lev, st = engine.run(0, s, **loop)[:2]
+                    assert (lev == want).all() and st["edges_count"] == ec, (kw, s, loop)
+            engine.set_params(**before)
