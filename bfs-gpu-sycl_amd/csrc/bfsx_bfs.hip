@@ -2646,15 +2646,7 @@ static KArgs kargs(const StepArgs &s, uint32_t hub) {
   a.next_level = s.next_level;
   a.hub_degree = hub;
   a.mark = s.mark;
-  // Where many edges lead to each new vertex and the marks do not stay in an
-  // XCD's L2 (4 MB), a read of the mark byte (mostly a line this XCD already
-  // holds) saves the store, which the L2 has to write back line by line in
-  // all eight XCDs: R-MAT 22's second level (62 M edges, 2 M new vertices)
-  // 758 -> 555 us, R-MAT 24's (339 M, 7.6 M) 4715 -> 3763 us.  With fewer
-  // edges per new vertex the extra read costs more than the stores it saves
-  // (16 M edges, 0.75 M new of 1.5 M: 102 -> 137 us), as on levels whose
-  // targets are mostly visited already (R-MAT 22's third: 342 -> 360 us).
-  a.mark_probe = s.mark && s.n_cols >= (1u << 21) && s.EF >= 8ull * s.n_cols && !s.hot_ok;
+  a.mark_probe = s.mark_probe;
   a.examined = s.count_examined ? &s.ctl->examined : nullptr;
   a.hot_vis = nullptr;
   a.hot_id = nullptr;

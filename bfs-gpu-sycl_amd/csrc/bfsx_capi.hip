@@ -298,6 +298,17 @@ struct Walker {
     a.bucket_ok = br != 0xFFFFFFFFu && (double)UE * 1024.0 >= (double)ctx->nnz * br &&
                   (use_mark || EF * 256 >= ctx->n_cols) && mr.lo_E != ~0ull;
     a.mark = use_mark ? ctx->mark.as<uint8_t>() : nullptr;
+    // Where many edges lead to each new vertex and the marks do not stay in
+    // an XCD's L2 (4 MB), a read of the mark byte (mostly a line this XCD
+    // already holds) saves the store, which the L2s of all eight XCDs write
+    // back line by line: R-MAT 22's second level (62 M edges, 2 M new
+    // vertices) 758 -> 555 us, R-MAT 24's (339 M, 7.6 M) 4715 -> 3763 us.
+    // With fewer edges per vertex the extra read costs more than the stores
+    // it saves (16 M edges, 0.75 M new of 1.5 M: 102 -> 137 us), as on levels
+    // whose targets are mostly visited already, i.e. once the levels before
+    // this one hold a quarter of the edges (R-MAT 22's third: 342 -> 360 us).
+    a.mark_probe = use_mark && ctx->n_cols >= (1u << 21) && EF >= 8ull * ctx->n_cols &&
+                   (VE - EF) * 4 < ctx->nnz;
     // the hot copy pays once the visited vertices hold half the edges
     a.hot_ok = VE * 2 >= ctx->nnz;
     // next frontier bitmap of a top-down step (kept for bottom-up steps)

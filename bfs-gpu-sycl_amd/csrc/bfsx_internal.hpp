@@ -306,6 +306,7 @@ struct StepArgs {
   int32_t next_level;
   bool track_degrees;      // accumulate degree sum of discovered vertices
   uint8_t *mark;           // non-null: mark-then-compact step
+  bool mark_probe;         // a marking step reads a target's mark byte before storing it
   bool count_examined;     // bottom-up: add adjacency entries read to ctl->examined
   hipEvent_t ev_k0, ev_k1; // non-null: recorded around the step's main kernel
   unsigned long long EF;   // frontier edges (out-degree sum of q_in)

@@ -125,3 +125,74 @@ def test_tiles_shared_by_groups(engine, leaves, ptr):
                     lev, st = engine.run(0, s, **loop)[:2]
                     assert (lev == want).all() and st["edges_count"] == ec, (kw, s, loop)
             engine.set_params(**before)
+
+
+# the allocation-free search: tiny levels in one work-group (up to 2048 edges),
+# exact-once and marking levels, tiles shared by groups, compaction of 8192
+# vertices per group, level arrays at any 4-byte alignment
+@pytest.mark.parametrize("name", ["one", "3", "257", "8191", "8193", "20001", "path9001",
+                                  "star70001", "directed4099", "hub2047", "hub2049", "hub20011",
+                                  "rmat15", "wide4194304"])
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_noalloc_edges(engine, name, ptr, shift):
+    import ctypes as C
+
+    import bfsx
+    from test_zz_no_alloc import Dev, hip
+    say("noalloc", name, ptr.__name__, shift)
+    h = hip()
+    if name.startswith("hub"):
+        k = int(name[3:])
+        src = np.concatenate([[0, 1], np.full(k, 2), np.arange(k) + 3])
+        dst = np.concatenate([[1, 2], np.arange(k) + 3, np.full(k, k + 3)])
+        cp, ri = csc_from_edges(k + 4, *symmetrize(src, dst))
+        n_rows, root = k + 4, 0
+    elif name.startswith("wide"):
+        # one level of nearly every vertex, which fills the queue's buffer up
+        # to the marks, then 200000 leaves of which share one more vertex
+        n_rows = int(name[4:])
+        leaf = np.arange(1, n_rows - 3)
+        src = np.concatenate([np.zeros(len(leaf), np.int64), leaf[-200000:], [n_rows - 3]])
+        dst = np.concatenate([leaf, np.full(200000, n_rows - 3), [n_rows - 2]])
+        cp, ri = csc_from_edges(n_rows, *symmetrize(src, dst))
+        root = 7
+    elif name == "rmat15":
+        engine.generate_rmat(15, 16, 0.57, 0.19, 0.19, 3, 4, 4)
+        cp, ri = engine.download_csc()
+        n_rows, root = 1 << 15, int(engine.pick_roots(1, 5)[0])
+    elif name == "path9001":
+        cp, ri, n_rows, root = *path_graph(9001), 9001, 4500
+    else:
+        cp, ri, n_rows, _, root = some_graph(name)
+    cp, n = cp.astype(ptr), len(cp) - 1
+    want, _, _ = cpu.bfs_queue(cp, ri, root, n_rows=n_rows)
+    d_cp, d_ri, d_lev = Dev.of(h, cp), Dev.of(h, ri), Dev(h, 4 * (n + 2))
+    try:
+        def run(row_idx, col_ptr):
+            nl = C.c_uint32(0)
+            rc = bfsx.lib().bfsx_run_noalloc(0, None, col_ptr.p, cp.itemsize, row_idx.p, n, n_rows,
+                                             len(ri), root, d_lev.p.value + 4 * shift, C.byref(nl))
+            return rc, nl.value, d_lev.get(np.int32, n + 2)[shift:shift + n]
+        for _ in range(2):
+            rc, nl, lev = run(d_ri, d_cp)
+            assert rc == 0 and (lev == want).all() and nl == int(want.max()) + 1
+        # entries past the graph are skipped and reported, in lists and offsets
+        if len(ri) > 100:
+            bad = ri.copy()
+            bad[len(ri) // 2] = n + 1000
+            used = np.searchsorted(cp.astype(np.int64), len(ri) // 2, side="right") - 1
+            d_bad = Dev.of(h, bad)
+            rc, _, lev = run(d_bad, d_cp)
+            d_bad.free()
+            assert rc == (1 if used < n_rows and want[used] >= 0 else 0)
+            assert ((lev >= 0) <= (want >= 0)).all() and (lev[lev >= 0] >= want[lev >= 0]).all()
+            cut = cp.copy()
+            cut[root + 1] = len(ri) + 5  # the root's list runs past the end
+            d_cut = Dev.of(h, cut)
+            rc, _, lev = run(d_ri, d_cut)
+            d_cut.free()
+            assert rc == 1 and lev[root] == 0
+    finally:
+        for d in (d_cp, d_ri, d_lev):
+            d.free()
