@@ -871,7 +871,6 @@ static uint32_t record(bfsx_ctx *ctx, const uint32_t *roots, uint32_t n_roots, u
 
 static void finish_run(bfsx_ctx *ctx, const RunOut &r, int32_t *levels_out,
                        uint32_t *parents_out, bfsx_run_stats *stats) {
-  hipStream_t s = ctx->stream;
   if (stats) {
     // The counts come from the level ends, which keep them exactly (they
     // decide each level's step).  A pass over levels and col_ptr after the
@@ -886,12 +885,8 @@ static void finish_run(bfsx_ctx *ctx, const RunOut &r, int32_t *levels_out,
     for (int i = 0; i < BFSX_N_STEP_KINDS; i++) stats->steps[i] = r.steps[i];
   }
   if (levels_out)
-    BFSX_HIP(hipMemcpyAsync(levels_out, ctx->levels.p, sizeof(int32_t) * ctx->n_cols,
-                            hipMemcpyDeviceToHost, s));
-  if (parents_out)
-    BFSX_HIP(hipMemcpyAsync(parents_out, ctx->parents.p, sizeof(uint32_t) * ctx->n_cols,
-                            hipMemcpyDeviceToHost, s));
-  BFSX_HIP(hipStreamSynchronize(s));
+    copy_levels_out(ctx, levels_out, ctx->levels.as<int32_t>(), ctx->n_cols, r.n_levels - 1);
+  if (parents_out) copy_out(ctx, parents_out, ctx->parents.p, sizeof(uint32_t) * (size_t)ctx->n_cols);
 }
 
 }  // namespace bfsx
@@ -985,6 +980,10 @@ int bfsx_create(int device, bfsx_ctx **out) {
                            hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(ctx->h_mirror, 0, sizeof(LevelMirror) * MIRROR_SLOTS);
     BFSX_HIP(hipHostGetDevicePointer((void **)&ctx->d_mirror, ctx->h_mirror, 0));
+    BFSX_HIP(hipHostMalloc((void **)&ctx->ring, RING_PIECE_BYTES * RING_SLOTS, hipHostMallocMapped));
+    BFSX_HIP(hipHostGetDevicePointer((void **)&ctx->ring_dev, ctx->ring, 0));
+    for (hipEvent_t &e : ctx->ring_ev)
+      BFSX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     ctx->params = default_params();
   });
   if (rc != BFSX_OK) {
@@ -1012,6 +1011,9 @@ void bfsx_destroy(bfsx_ctx *ctx) {
     release(*b);
   if (ctx->h_ctl) (void)hipHostFree(ctx->h_ctl);
   if (ctx->h_mirror) (void)hipHostFree(ctx->h_mirror);
+  if (ctx->ring) (void)hipHostFree(ctx->ring);
+  for (hipEvent_t e : ctx->ring_ev)
+    if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : {ctx->ev0, ctx->ev1, ctx->ev_step0, ctx->ev_step1, ctx->ev_k0, ctx->ev_k1})
     if (e) (void)hipEventDestroy(e);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -1056,12 +1058,8 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
     release(ctx->row_idx);
     ensure(ctx->col_ptr, (size_t)col_ptr_bytes * n1, ctx->stream);
     ensure(ctx->row_idx, sizeof(uint32_t) * (nnz ? nnz : 1), ctx->stream);
-    BFSX_HIP(hipMemcpyAsync(ctx->col_ptr.p, col_ptr, (size_t)col_ptr_bytes * n1,
-                            hipMemcpyHostToDevice, ctx->stream));
-    if (nnz)
-      BFSX_HIP(hipMemcpyAsync(ctx->row_idx.p, row_idx, sizeof(uint32_t) * nnz,
-                              hipMemcpyHostToDevice, ctx->stream));
-    BFSX_HIP(hipStreamSynchronize(ctx->stream));
+    copy_in(ctx, ctx->col_ptr.p, col_ptr, (size_t)col_ptr_bytes * n1);
+    copy_in(ctx, ctx->row_idx.p, row_idx, sizeof(uint32_t) * nnz);
     ctx->n_cols = n_cols;
     ctx->n_rows = n_rows;
     ctx->nnz = nnz;
@@ -1187,13 +1185,8 @@ int bfsx_download_csc(bfsx_ctx *ctx, void *col_ptr, uint32_t *row_idx) {
     set_device(ctx);
     if (!ctx->has_graph) fail(BFSX_ERR_STATE, "no graph uploaded");
     if (col_ptr)
-      BFSX_HIP(hipMemcpyAsync(col_ptr, ctx->col_ptr.p,
-                              (size_t)ctx->ptr_bytes * ((uint64_t)ctx->n_cols + 1),
-                              hipMemcpyDeviceToHost, ctx->stream));
-    if (row_idx && ctx->nnz)
-      BFSX_HIP(hipMemcpyAsync(row_idx, ctx->row_idx.p, sizeof(uint32_t) * ctx->nnz,
-                              hipMemcpyDeviceToHost, ctx->stream));
-    BFSX_HIP(hipStreamSynchronize(ctx->stream));
+      copy_out(ctx, col_ptr, ctx->col_ptr.p, (size_t)ctx->ptr_bytes * ((uint64_t)ctx->n_cols + 1));
+    if (row_idx) copy_out(ctx, row_idx, ctx->row_idx.p, sizeof(uint32_t) * ctx->nnz);
   });
 }
 

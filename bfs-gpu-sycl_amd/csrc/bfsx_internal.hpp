@@ -129,6 +129,11 @@ constexpr uint32_t PULL_HUB_FLAG = 0x80000000u;
 constexpr uint32_t PULL_HUBS_MAX = 1u << 18;
 __host__ __device__ inline uint64_t mark_bytes(uint64_t n) { return ((n + 1023) / 1024) * 1024; }
 
+// The ring of pinned host buffers that copies from and to pageable host
+// memory go through.
+constexpr size_t RING_PIECE_BYTES = 2u << 20;
+constexpr int RING_SLOTS = 8;
+
 // Growable device allocation.
 struct DevBuf {
   void *p = nullptr;
@@ -201,6 +206,9 @@ struct bfsx_ctx {
   // reading the control block
   uint32_t seq = 0;
   bool seq_known = false;
+  uint8_t *ring = nullptr;      // pinned: RING_SLOTS pieces of RING_PIECE_BYTES
+  uint8_t *ring_dev = nullptr;  // its device address
+  hipEvent_t ring_ev[bfsx::RING_SLOTS] = {};  // a piece's copy has finished
   bool mark_dirty = false;          // a mark step did not reach its compaction
 
   // learned scheduler weights and the snapshot used to time alternatives
@@ -383,6 +391,15 @@ void ms_drop(bfsx_ctx *ctx);  // the relabelled graph and the captured loop
 void gen_rmat_pairs_offset(bfsx_ctx *ctx, int scale, uint64_t m, uint32_t tA, uint32_t tAB,
                            uint32_t tABC, uint64_t seed_graph, uint64_t seed_perm,
                            uint32_t offset, uint32_t *d_u, uint32_t *d_v);
+
+// ---- host transfers (bfsx_transfer.hip) ------------------------------------
+// Copies between the card and the caller's memory, after all work queued on
+// the context's stream; they return when the copy is done.
+void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes);
+void copy_in(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes);
+// n levels, none above max_level
+void copy_levels_out(bfsx_ctx *ctx, int32_t *dst, const int32_t *levels, uint32_t n,
+                     uint32_t max_level);
 
 // ---- allocation-free search (bfsx_noalloc.hip) ----------------------------
 const char *noalloc_last_error();  // the calling thread's last failure message

@@ -777,8 +777,7 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
     hipLaunchKernelGGL(k_ms_transpose, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, rows, NB,
                        n_bits, (uint32_t)n, out.as<uint8_t>());
     BFSX_HIP(hipGetLastError());
-    BFSX_HIP(hipMemcpyAsync(levels_out, out.p, (size_t)n_bits * n, hipMemcpyDeviceToHost, s));
-    BFSX_HIP(hipStreamSynchronize(s));
+    copy_out(ctx, levels_out, out.p, (size_t)n_bits * n);
     release(out);
     release(plain);
   }

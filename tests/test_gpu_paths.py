@@ -196,3 +196,31 @@ def test_noalloc_edges(engine, name, ptr, shift):
     finally:
         for d in (d_cp, d_ri, d_lev):
             d.free()
+
+
+# levels cross as 1, 2 or 4 bytes each (up to 254, 65534 or more levels) in
+# pieces of 1 MB through four pinned buffers, a piece's slices by up to four
+# threads; graphs cross as bytes the same way
+@pytest.mark.parametrize("depth", [254, 255, 256, 65535, 65536])
+@pytest.mark.parametrize("n", [70001, 1 << 20, (1 << 20) + 1, 5 * (1 << 20) + 13])
+def test_levels_and_graphs_to_pageable_memory(engine, depth, n):
+    say("transfer", depth, n)
+    # a path of depth + 1 vertices; the other vertices hang off its first one
+    # (a third of them) or are isolated
+    rng = np.random.default_rng(n)
+    other = np.arange(depth + 1, n)
+    leaf = other[rng.random(len(other)) < 0.33]
+    src = np.concatenate([np.arange(depth), np.zeros(len(leaf), np.int64)])
+    dst = np.concatenate([np.arange(depth) + 1, leaf])
+    cp, ri = csc_from_edges(n, *symmetrize(src, dst), dtype=np.uint64)
+    engine.upload_csc(cp, ri, symmetric=True)
+    got_cp, got_ri = engine.download_csc()
+    assert (got_cp == cp).all() and (got_ri == ri).all()
+    want = np.full(n, -1, np.int32)
+    want[: depth + 1] = np.arange(depth + 1)
+    want[leaf] = 1
+    lev, st, par = engine.run(0, "llb", parents=True)
+    assert st["max_level"] == depth and (lev == want).all()
+    ok = par[1:depth + 1] == np.arange(depth)
+    assert ok.all() and (par[leaf] == 0).all() and par[0] == 0
+    assert (par[want < 0] == 0xFFFFFFFF).all()
