@@ -2728,10 +2728,10 @@ static void glb_bucketed(bfsx_ctx *ctx, const StepArgs &s, const KArgs &a, const
   hipStream_t st = ctx->stream;
   // the frontier's edge count (kept exactly by every step) bounds the targets
   const uint64_t cap = s.EF ? s.EF : 1;
-  ensure(ctx->bkt, sizeof(uint16_t) * cap, st);
-  ensure(ctx->bkt_cnt, sizeof(uint32_t) * (size_t)grid * n_slices, st);
-  ensure(ctx->bkt_tot, sizeof(uint64_t) * n_slices, st);
-  ensure(ctx->bkt_base, sizeof(uint64_t) * (n_slices + 1), st);
+  ensure(ctx->bkt, sizeof(uint16_t) * cap, ctx);
+  ensure(ctx->bkt_cnt, sizeof(uint32_t) * (size_t)grid * n_slices, ctx);
+  ensure(ctx->bkt_tot, sizeof(uint64_t) * n_slices, ctx);
+  ensure(ctx->bkt_base, sizeof(uint64_t) * (n_slices + 1), ctx);
   uint32_t *cnt = ctx->bkt_cnt.as<uint32_t>();
   uint64_t *tot = ctx->bkt_tot.as<uint64_t>();
   uint64_t *base = ctx->bkt_base.as<uint64_t>();
@@ -2851,10 +2851,10 @@ bool step_glb(bfsx_ctx *ctx, const StepArgs &s) {
   if (s.F == 0) return false;
   const uint64_t pw = ctx->ptr_bytes;
   // scratch: local + global scans, starts, tile sums, chunk table
-  ensure(ctx->glb_scan, pw * 2 * ((uint64_t)ctx->n_cols + 1), ctx->stream);
-  ensure(ctx->glb_start, pw * ((uint64_t)ctx->n_cols + 1), ctx->stream);
-  ensure(ctx->glb_tile, pw * ((uint64_t)ctx->n_cols / GLB_TILE + 4), ctx->stream);
-  ensure(ctx->glb_chunk_lo, sizeof(uint32_t) * (ctx->nnz / GLB_MIN_CHUNK + 2), ctx->stream);
+  ensure(ctx->glb_scan, pw * 2 * ((uint64_t)ctx->n_cols + 1), ctx);
+  ensure(ctx->glb_start, pw * ((uint64_t)ctx->n_cols + 1), ctx);
+  ensure(ctx->glb_tile, pw * ((uint64_t)ctx->n_cols / GLB_TILE + 4), ctx);
+  ensure(ctx->glb_chunk_lo, sizeof(uint32_t) * (ctx->nnz / GLB_MIN_CHUNK + 2), ctx);
   const bool bucketed =
       ctx->ptr_bytes == 8 ? step_glb_t<uint64_t>(ctx, s) : step_glb_t<uint32_t>(ctx, s);
   BFSX_HIP(hipGetLastError());
@@ -2916,7 +2916,7 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   const SpecGuard guard{speculative ? s.ctl : nullptr, s.q_in_idx, 1u << BFSX_PULL, NEVER_MARKS};
   const uint32_t *g_sum = nullptr;
   if (use_sum) {
-    ensure(ctx->fsum, sizeof(uint32_t) * PULL_SUM_WORDS_MAX, st);
+    ensure(ctx->fsum, sizeof(uint32_t) * PULL_SUM_WORDS_MAX, ctx);
     const uint32_t n_words = (uint32_t)bitmap_words(s.n_cols);
     const unsigned sgrid = cap_grid(((uint64_t)sum_bits + 255) / 256, (unsigned)ctx->cu_count * 4);
     hipLaunchKernelGGL(k_fbm_summary, dim3(sgrid), dim3(256), 0, st, s.fbm_cur, n_words, shift,

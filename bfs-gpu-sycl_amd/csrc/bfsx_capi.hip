@@ -25,23 +25,74 @@ void check_hip(hipError_t e, const char *what) {
   fail(st, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-void ensure(DevBuf &b, size_t bytes, hipStream_t s) {
-  (void)s;
+// A context's released device buffers, kept for its next ensure(): a graph
+// that replaces another (and every sort on the way to its orders) otherwise
+// allocates and frees some twenty buffers, 2.5 ms of the 11.5 ms that loading
+// 16 M edges took.  All users of a context work on its one stream, so a buffer
+// taken over is used after its last user.  Bounded (single buffers and in
+// all), emptied when an allocation fails and with the context.
+static constexpr size_t SPARE_BUF_MAX = 256u << 20, SPARE_MAX = 1u << 30;
+
+void DevPool::drop() {
+  for (const DevBuf &b : spare) (void)hipFree(b.p);
+  spare.clear();
+  bytes = 0;
+}
+
+void ensure(DevBuf &b, size_t bytes, bfsx_ctx *ctx) {
   if (bytes == 0) bytes = 1;
   if (b.p && b.bytes >= bytes) return;
-  if (b.p) {
-    BFSX_HIP(hipFree(b.p));
-    b.p = nullptr;
-    b.bytes = 0;
+  release(b);
+  if (bytes <= SPARE_BUF_MAX) {
+    // sixteenths of a power of two, so that graphs of nearly one size share
+    size_t unit = 4096;
+    while (unit * 32 <= bytes) unit *= 2;
+    bytes = (bytes + unit - 1) / unit * unit;
   }
-  BFSX_HIP(hipMalloc(&b.p, bytes));
+  DevPool &pool = ctx->pool;
+  size_t best = pool.spare.size();
+  for (size_t i = 0; i < pool.spare.size(); i++) {
+    const size_t have = pool.spare[i].bytes;
+    if (have >= bytes && have <= bytes * 2 &&
+        (best == pool.spare.size() || have < pool.spare[best].bytes))
+      best = i;
+  }
+  if (best < pool.spare.size()) {
+    b = pool.spare[best];
+    pool.spare[best] = pool.spare.back();
+    pool.spare.pop_back();
+    pool.bytes -= b.bytes;
+    return;
+  }
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipErrorOutOfMemory && !pool.spare.empty()) {
+    (void)hipGetLastError();
+    BFSX_HIP(hipStreamSynchronize(ctx->stream));
+    pool.drop();
+    e = hipMalloc(&p, bytes);
+  }
+  check_hip(e, "hipMalloc");
+  b.p = p;
   b.bytes = bytes;
+  b.pool = &pool;
 }
 
 void release(DevBuf &b) {
-  if (b.p) (void)hipFree(b.p);
-  b.p = nullptr;
-  b.bytes = 0;
+  if (b.p) {
+    DevPool *pool = b.pool;
+    if (b.bytes <= SPARE_BUF_MAX && pool->bytes + b.bytes <= SPARE_MAX) {
+      try {
+        pool->spare.push_back(b);
+        pool->bytes += b.bytes;
+      } catch (...) {  // (no host memory for the list)
+        (void)hipFree(b.p);
+      }
+    } else {
+      (void)hipFree(b.p);
+    }
+  }
+  b = DevBuf{};
 }
 
 static void set_device(bfsx_ctx *ctx) { BFSX_HIP(hipSetDevice(ctx->device)); }
@@ -63,20 +114,20 @@ static void free_search_state(bfsx_ctx *ctx) {
 static void alloc_search_state(bfsx_ctx *ctx) {
   hipStream_t s = ctx->stream;
   const uint64_t n = ctx->n_cols;
-  ensure(ctx->levels, sizeof(int32_t) * n, s);
-  ensure(ctx->vis, sizeof(uint32_t) * bitmap_words(n), s);
-  ensure(ctx->queue[0], sizeof(uint32_t) * (n + 1), s);
-  ensure(ctx->queue[1], sizeof(uint32_t) * (n + 1), s);
-  ensure(ctx->mark, mark_bytes(n), s);
+  ensure(ctx->levels, sizeof(int32_t) * n, ctx);
+  ensure(ctx->vis, sizeof(uint32_t) * bitmap_words(n), ctx);
+  ensure(ctx->queue[0], sizeof(uint32_t) * (n + 1), ctx);
+  ensure(ctx->queue[1], sizeof(uint32_t) * (n + 1), ctx);
+  ensure(ctx->mark, mark_bytes(n), ctx);
   BFSX_HIP(hipMemsetAsync(ctx->mark.p, 0, mark_bytes(n), s));
   BFSX_HIP(hipStreamSynchronize(s));
 }
 
 static void ensure_pull_state(bfsx_ctx *ctx) {
   const uint64_t w = bitmap_words(ctx->n_cols);
-  ensure(ctx->fbm[0], sizeof(uint32_t) * w, ctx->stream);
-  ensure(ctx->fbm[1], sizeof(uint32_t) * w, ctx->stream);
-  ensure(ctx->fsum, sizeof(uint32_t) * bfsx::PULL_SUM_WORDS_MAX, ctx->stream);
+  ensure(ctx->fbm[0], sizeof(uint32_t) * w, ctx);
+  ensure(ctx->fbm[1], sizeof(uint32_t) * w, ctx);
+  ensure(ctx->fsum, sizeof(uint32_t) * bfsx::PULL_SUM_WORDS_MAX, ctx);
 }
 
 // the {first neighbour, degree} array and its hub index, and the top-down
@@ -568,7 +619,7 @@ static RunOut search(bfsx_ctx *ctx, uint32_t root, int strategy, uint32_t flags,
       fail(BFSX_ERR_UNSUPPORTED, "the captured level loop has no per-level trace or parents");
     return search_graph_loop(ctx, root, strategy == BFSX_LEARNED ? -1 : fixed, learned);
   }
-  if (want_parents) ensure(ctx->parents, sizeof(uint32_t) * ctx->n_cols, s);
+  if (want_parents) ensure(ctx->parents, sizeof(uint32_t) * ctx->n_cols, ctx);
   uint32_t *par = want_parents ? ctx->parents.as<uint32_t>() : nullptr;
   if (!ctx->seq_known) {
     read_ctl(ctx);
@@ -770,9 +821,9 @@ static void snapshot(bfsx_ctx *ctx, bool save) {
   hipStream_t s = ctx->stream;
   const size_t lb = sizeof(int32_t) * ctx->n_cols;
   const size_t vb = sizeof(uint32_t) * bitmap_words(ctx->n_cols);
-  ensure(ctx->snap_levels, lb, s);
-  ensure(ctx->snap_vis, vb, s);
-  ensure(ctx->snap_ctl, sizeof(LevelCtl), s);
+  ensure(ctx->snap_levels, lb, ctx);
+  ensure(ctx->snap_vis, vb, ctx);
+  ensure(ctx->snap_ctl, sizeof(LevelCtl), ctx);
   if (save) {
     BFSX_HIP(hipMemcpyAsync(ctx->snap_levels.p, ctx->levels.p, lb, hipMemcpyDeviceToDevice, s));
     BFSX_HIP(hipMemcpyAsync(ctx->snap_vis.p, ctx->vis.p, vb, hipMemcpyDeviceToDevice, s));
@@ -799,7 +850,7 @@ static uint32_t record(bfsx_ctx *ctx, const uint32_t *roots, uint32_t n_roots, u
   const bool symmetric = graph_symmetric(ctx);
   // scheduler inputs come from the same kernel as at inference; the
   // network's outputs are not used here
-  ensure(ctx->sched_w, sizeof(float) * BFSX_SCHED_PARAMS, ctx->stream);
+  ensure(ctx->sched_w, sizeof(float) * BFSX_SCHED_PARAMS, ctx);
   if (!ctx->sched_loaded)
     BFSX_HIP(hipMemsetAsync(ctx->sched_w.p, 0, sizeof(float) * BFSX_SCHED_PARAMS, ctx->stream));
   uint64_t rng = seed * 0x9E3779B97F4A7C15ull + 1;
@@ -972,7 +1023,7 @@ int bfsx_create(int device, bfsx_ctx **out) {
     BFSX_HIP(hipEventCreate(&ctx->ev_step1));
     BFSX_HIP(hipEventCreate(&ctx->ev_k0));
     BFSX_HIP(hipEventCreate(&ctx->ev_k1));
-    ensure(ctx->ctl, sizeof(LevelCtl), ctx->stream);
+    ensure(ctx->ctl, sizeof(LevelCtl), ctx);
     BFSX_HIP(hipMemsetAsync(ctx->ctl.p, 0, sizeof(LevelCtl), ctx->stream));  // level-end counter 0
     BFSX_HIP(hipStreamSynchronize(ctx->stream));
     BFSX_HIP(hipHostMalloc((void **)&ctx->h_ctl, sizeof(LevelCtl), hipHostMallocDefault));
@@ -1009,6 +1060,7 @@ void bfsx_destroy(bfsx_ctx *ctx) {
   release(ctx->scratch);
   for (DevBuf *b : {&ctx->sched_w, &ctx->snap_levels, &ctx->snap_vis, &ctx->snap_ctl})
     release(*b);
+  ctx->pool.drop();
   if (ctx->h_ctl) (void)hipHostFree(ctx->h_ctl);
   if (ctx->h_mirror) (void)hipHostFree(ctx->h_mirror);
   if (ctx->ring) (void)hipHostFree(ctx->ring);
@@ -1040,26 +1092,59 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
     if (col_ptr_bytes != 4 && col_ptr_bytes != 8) fail(BFSX_ERR_ARG, "col_ptr_bytes must be 4 or 8");
     if (n_rows > n_cols) fail(BFSX_ERR_ARG, "n_rows > n_cols");
     if (!col_ptr || (nnz && !row_idx)) fail(BFSX_ERR_ARG, "null graph pointer");
-    // validate col_ptr on the host: monotone, starts at 0, ends at nnz
     const uint64_t n1 = (uint64_t)n_cols + 1;
     auto at = [&](uint64_t i) -> uint64_t {
       return col_ptr_bytes == 8 ? static_cast<const uint64_t *>(col_ptr)[i]
                                 : static_cast<const uint32_t *>(col_ptr)[i];
     };
     if (at(0) != 0) fail(BFSX_ERR_ARG, "col_ptr[0] != 0");
-    for (uint64_t i = 1; i < n1; i++)
-      if (at(i) < at(i - 1)) fail(BFSX_ERR_ARG, "col_ptr is not monotone");
-    if (at(n_rows) > nnz || at(n_cols) != nnz)
-      fail(BFSX_ERR_ARG, "col_ptr end does not match nnz");
-    for (uint64_t i = 0; i < nnz; i++)
-      if (row_idx[i] >= n_cols) fail(BFSX_ERR_ARG, "row_idx entry >= n_cols");
+    auto refuse = [&](bool falls, bool outside) {
+      if (falls) fail(BFSX_ERR_ARG, "col_ptr is not monotone");
+      if (at(n_rows) > nnz || at(n_cols) != nnz)
+        fail(BFSX_ERR_ARG, "col_ptr end does not match nnz");
+      if (outside) fail(BFSX_ERR_ARG, "row_idx entry >= n_cols");
+    };
+    // The arrays go into buffers of their own and are checked on the card (a
+    // pass over 64 MB took the host 3.5 ms, as long as their transfer): a
+    // graph that is refused leaves the resident one as it was.
+    DevBuf cp, ri;
+    struct Releaser {
+      DevBuf *b[2];
+      ~Releaser() {
+        for (DevBuf *x : b) release(*x);
+      }
+    } releaser{{&cp, &ri}};
+    bool beside = true;
+    try {
+      ensure(cp, (size_t)col_ptr_bytes * n1, ctx);
+      ensure(ri, sizeof(uint32_t) * (nnz ? nnz : 1), ctx);
+    } catch (const Error &e) {
+      if (e.status != BFSX_ERR_NOMEM) throw;
+      beside = false;
+    }
+    if (!beside) {  // no room for both graphs: checked on the host first
+      (void)hipGetLastError();
+      release(cp);
+      release(ri);
+      bool falls = false, outside = false;
+      for (uint64_t i = 1; i < n1; i++) falls |= at(i) < at(i - 1);
+      for (uint64_t i = 0; i < nnz; i++) outside |= row_idx[i] >= n_cols;
+      refuse(falls, outside);
+      ctx->has_graph = false;
+      release(ctx->col_ptr);
+      release(ctx->row_idx);
+      ensure(cp, (size_t)col_ptr_bytes * n1, ctx);
+      ensure(ri, sizeof(uint32_t) * (nnz ? nnz : 1), ctx);
+    }
+    copy_in(ctx, cp.p, col_ptr, (size_t)col_ptr_bytes * n1);
+    copy_in(ctx, ri.p, row_idx, sizeof(uint32_t) * nnz);
+    if (beside) {
+      const uint32_t bad = check_csc(ctx, cp.p, col_ptr_bytes, n_cols, ri.as<uint32_t>(), nnz);
+      refuse(bad & 1u, bad & 2u);
+    }
     ctx->has_graph = false;
-    release(ctx->col_ptr);
-    release(ctx->row_idx);
-    ensure(ctx->col_ptr, (size_t)col_ptr_bytes * n1, ctx->stream);
-    ensure(ctx->row_idx, sizeof(uint32_t) * (nnz ? nnz : 1), ctx->stream);
-    copy_in(ctx, ctx->col_ptr.p, col_ptr, (size_t)col_ptr_bytes * n1);
-    copy_in(ctx, ctx->row_idx.p, row_idx, sizeof(uint32_t) * nnz);
+    std::swap(ctx->col_ptr, cp);
+    std::swap(ctx->row_idx, ri);
     ctx->n_cols = n_cols;
     ctx->n_rows = n_rows;
     ctx->nnz = nnz;
@@ -1094,8 +1179,8 @@ int bfsx_generate_rmat(bfsx_ctx *ctx, int scale, int edge_factor, double a, doub
     release(ctx->col_ptr);
     release(ctx->row_idx);
     DevBuf du, dv;
-    ensure(du, sizeof(uint32_t) * m, ctx->stream);
-    ensure(dv, sizeof(uint32_t) * m, ctx->stream);
+    ensure(du, sizeof(uint32_t) * m, ctx);
+    ensure(dv, sizeof(uint32_t) * m, ctx);
     gen_rmat_pairs(ctx, scale, m, thresh32(a), thresh32(a + b), thresh32(a + b + c), seed_graph,
                    seed_perm, du.as<uint32_t>(), dv.as<uint32_t>());
     build_symmetric_csc(ctx, n, du.as<uint32_t>(), dv.as<uint32_t>(), m, col_ptr_bytes);
@@ -1121,8 +1206,8 @@ int bfsx_generate_grid(bfsx_ctx *ctx, uint32_t side, double drop_prob, uint32_t 
     release(ctx->col_ptr);
     release(ctx->row_idx);
     DevBuf du, dv;
-    ensure(du, sizeof(uint32_t) * m, ctx->stream);
-    ensure(dv, sizeof(uint32_t) * m, ctx->stream);
+    ensure(du, sizeof(uint32_t) * m, ctx);
+    ensure(dv, sizeof(uint32_t) * m, ctx);
     gen_grid_pairs(ctx, side, thresh32(drop_prob), n_long, seed, du.as<uint32_t>(), dv.as<uint32_t>());
     build_symmetric_csc(ctx, (uint32_t)V, du.as<uint32_t>(), dv.as<uint32_t>(), m, col_ptr_bytes);
     release(du);
@@ -1158,15 +1243,20 @@ int bfsx_order_adjacency(bfsx_ctx *ctx, int order) {
       fail(BFSX_ERR_ARG,
            "order must be BFSX_ORDER_ID, BFSX_ORDER_HUB_FIRST or BFSX_ORDER_PULL_HUB_FIRST");
     if (order == BFSX_ORDER_PULL_HUB_FIRST) {
-      ensure(ctx->row_idx_pull, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), ctx->stream);
-      order_adjacency(ctx, true, ctx->row_idx_pull.as<uint32_t>());
+      ensure(ctx->row_idx_pull, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), ctx);
+      DevBuf by_degree;  // the vertices, largest degree first
+      struct Releaser {
+        DevBuf &b;
+        ~Releaser() { release(b); }
+      } releaser{by_degree};
+      order_adjacency(ctx, true, ctx->row_idx_pull.as<uint32_t>(), &by_degree);
       if (ctx->max_degree < 0xFFFFFFFFull) {  // degrees fit the array's 32 bits
-        ensure(ctx->pull_fd, sizeof(uint2) * std::max<uint64_t>(ctx->n_rows, 1), ctx->stream);
+        ensure(ctx->pull_fd, sizeof(uint2) * std::max<uint64_t>(ctx->n_rows, 1), ctx);
         first_neighbours(ctx, ctx->row_idx_pull.as<uint32_t>(), ctx->pull_fd.as<uint2>());
-        index_hub_neighbours(ctx);
+        index_hub_neighbours(ctx, by_degree.as<uint32_t>());
         compact_first_neighbours(ctx);
       }
-      build_hot_copy(ctx);
+      build_hot_copy(ctx, by_degree.as<uint32_t>());
       ctx->gflags |= BFSX_GRAPH_PULL_COPY;
       return;
     }
@@ -1202,7 +1292,7 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
     if (mode == 2) {
       const uint32_t k = std::min(n_roots, ctx->n_rows);
       DevBuf dv;
-      ensure(dv, sizeof(uint32_t) * std::max(k, 1u), s);
+      ensure(dv, sizeof(uint32_t) * std::max(k, 1u), ctx);
       top_degree_vertices(ctx, k, dv.as<uint32_t>());
       if (k) {
         BFSX_HIP(hipMemcpyAsync(roots_out, dv.p, sizeof(uint32_t) * k, hipMemcpyDeviceToHost, s));
@@ -1221,8 +1311,8 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
       const uint32_t probe_batch = 64;
       std::vector<uint32_t> cand(probe_batch);
       DevBuf dv, dok;
-      ensure(dv, sizeof(uint32_t) * probe_batch, s);
-      ensure(dok, probe_batch, s);
+      ensure(dv, sizeof(uint32_t) * probe_batch, ctx);
+      ensure(dok, probe_batch, ctx);
       std::vector<uint8_t> ok(probe_batch);
       bool found = false;
       for (uint64_t first = 0; first < 64ull * probe_batch && !found; first += probe_batch) {
@@ -1243,8 +1333,8 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
     }
     const uint32_t batch = 1u << 16;
     DevBuf dv, dok;
-    ensure(dv, sizeof(uint32_t) * batch, s);
-    ensure(dok, batch, s);
+    ensure(dv, sizeof(uint32_t) * batch, ctx);
+    ensure(dok, batch, ctx);
     std::vector<uint32_t> cand(batch);
     std::vector<uint8_t> ok(batch);
     std::vector<uint32_t> got;
@@ -1306,7 +1396,7 @@ int bfsx_level_histogram(bfsx_ctx *ctx, uint64_t *counts, uint64_t *edges, uint3
     if (!ctx->has_graph || !ctx->levels.p) fail(BFSX_ERR_STATE, "no search has run");
     if (max_levels == 0 || max_levels > (1u << 24)) fail(BFSX_ERR_ARG, "max_levels out of range");
     hipStream_t s = ctx->stream;
-    ensure(ctx->scratch, sizeof(unsigned long long) * (2 * (size_t)max_levels + 1), s);
+    ensure(ctx->scratch, sizeof(unsigned long long) * (2 * (size_t)max_levels + 1), ctx);
     unsigned long long *d = ctx->scratch.as<unsigned long long>();
     level_histogram(ctx, max_levels, d);
     std::vector<unsigned long long> h(2 * (size_t)max_levels + 1);
@@ -1330,8 +1420,8 @@ int bfsx_stream_copy(bfsx_ctx *ctx, uint64_t bytes, int repeats, double *ms) {
     if (bytes < 16 || repeats < 1) fail(BFSX_ERR_ARG, "bytes >= 16 and repeats >= 1 required");
     bytes &= ~15ull;
     DevBuf a, b;
-    ensure(a, bytes, ctx->stream);
-    ensure(b, bytes, ctx->stream);
+    ensure(a, bytes, ctx);
+    ensure(b, bytes, ctx);
     BFSX_HIP(hipMemsetAsync(a.p, 1, bytes, ctx->stream));
     stream_copy(ctx, a.p, b.p, bytes);  // warm-up
     BFSX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
@@ -1391,8 +1481,8 @@ int bfsx_generate_rmat_union(bfsx_ctx *ctx, uint32_t n_graphs, const int *scales
     release(ctx->col_ptr);
     release(ctx->row_idx);
     DevBuf du, dv;
-    ensure(du, sizeof(uint32_t) * M, ctx->stream);
-    ensure(dv, sizeof(uint32_t) * M, ctx->stream);
+    ensure(du, sizeof(uint32_t) * M, ctx);
+    ensure(dv, sizeof(uint32_t) * M, ctx);
     for (uint32_t g = 0; g < n_graphs; g++)
       gen_rmat_pairs_offset(ctx, scales[g], eoff[g + 1] - eoff[g], thresh32(0.57),
                             thresh32(0.57 + 0.19), thresh32(0.57 + 0.19 + 0.19),
@@ -1420,7 +1510,7 @@ int bfsx_sched_set_weights(bfsx_ctx *ctx, const float *w, uint32_t n) {
     if (n != BFSX_SCHED_PARAMS) fail(BFSX_ERR_ARG, "scheduler needs 1476 parameters");
     for (uint32_t i = 0; i < n; i++)
       if (!std::isfinite(w[i])) fail(BFSX_ERR_ARG, "scheduler weight is not finite");
-    ensure(ctx->sched_w, sizeof(float) * n, ctx->stream);
+    ensure(ctx->sched_w, sizeof(float) * n, ctx);
     BFSX_HIP(hipMemcpyAsync(ctx->sched_w.p, w, sizeof(float) * n, hipMemcpyHostToDevice,
                             ctx->stream));
     BFSX_HIP(hipStreamSynchronize(ctx->stream));

@@ -135,15 +135,24 @@ constexpr size_t RING_PIECE_BYTES = 2u << 20;
 constexpr int RING_SLOTS = 8;
 
 // Growable device allocation.
+struct DevPool;
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
+  DevPool *pool = nullptr;  // where it goes when released
   template <class T> T *as() const { return static_cast<T *>(p); }
+};
+
+struct DevPool {
+  std::vector<DevBuf> spare;
+  size_t bytes = 0;
+  void drop();
 };
 
 }  // namespace bfsx
 
 struct bfsx_ctx {
+  bfsx::DevPool pool;  // released device buffers
   int device = 0;
   hipStream_t stream = nullptr;
   int cu_count = 0;
@@ -248,7 +257,7 @@ struct Error {
 void check_hip(hipError_t e, const char *what);
 #define BFSX_HIP(call) ::bfsx::check_hip((call), #call)
 
-void ensure(DevBuf &b, size_t bytes, hipStream_t s);
+void ensure(DevBuf &b, size_t bytes, bfsx_ctx *ctx);
 void release(DevBuf &b);
 
 // ---- graph construction (bfsx_gen.hip) -----------------------------------
@@ -263,17 +272,23 @@ uint64_t gen_grid_pairs(bfsx_ctx *ctx, uint32_t side, uint32_t t_drop,
                         uint32_t n_long, uint64_t seed, uint32_t *d_u,
                         uint32_t *d_v);
 void graph_summary(bfsx_ctx *ctx);  // max degree, isolated bitmap/count
+// Bit 0: col_ptr falls somewhere; bit 1: a row_idx entry is >= n_cols.
+uint32_t check_csc(bfsx_ctx *ctx, const void *col_ptr, int col_ptr_bytes, uint32_t n_cols,
+                   const uint32_t *row_idx, uint64_t nnz);
 // re-sorts every adjacency list by neighbour id or hub first (needs graph_summary)
 // Sorts every adjacency list (id order, or hub first) into `out`, which is
-// ctx->row_idx (in place) or a copy of the same size.
-void order_adjacency(bfsx_ctx *ctx, bool hub_first, uint32_t *out);
+// ctx->row_idx (in place) or a copy of the same size.  With hub_first,
+// *by_degree (optional) receives the n_cols vertices in rank order: degree
+// descending, ties by id.
+void order_adjacency(bfsx_ctx *ctx, bool hub_first, uint32_t *out, DevBuf *by_degree = nullptr);
 // fd[v] = {row_idx[col_ptr[v]] (~0u without neighbours), degree} for v < n_rows
 // (degrees below 2^32).
 void first_neighbours(bfsx_ctx *ctx, const uint32_t *row_idx, uint2 *fd);
 // Names the first neighbours that are among the graph's top-degree vertices
 // by their index in ctx->pull_hub (sets pull_hub, pull_hbm, pull_hubs); needs
-// ctx->pull_fd (one entry per vertex) and n_cols < 2^31.
-void index_hub_neighbours(bfsx_ctx *ctx);
+// ctx->pull_fd (one entry per vertex) and n_cols < 2^31; by_degree: the
+// vertices in degree order (order_adjacency).
+void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree);
 // Drops the isolated vertices' entries from ctx->pull_fd (one uint2 entry per
 // vertex before), splits it into ctx->pull_fd (first neighbours) and
 // ctx->pull_fdd (16-bit degrees), and builds ctx->pull_crank (needs the
@@ -282,7 +297,7 @@ void compact_first_neighbours(bfsx_ctx *ctx);
 // Builds row_idx_hot / hot_id / hot_vis / hot_n for graphs of
 // HOT_MIN_VERTICES to 2^31 vertices (otherwise leaves hot_n = 0).
 constexpr uint32_t HOT_MIN_VERTICES = 1u << 24;
-void build_hot_copy(bfsx_ctx *ctx);
+void build_hot_copy(bfsx_ctx *ctx, const uint32_t *by_degree);
 // The graph with vertices renamed by (degree descending, id ascending):
 // rank[v] = new id of v, order[i] = old id of new vertex i, new_cp / new_ri
 // the relabelled CSC (lists ascending in new ids), col_ptr of the graph's

@@ -576,12 +576,11 @@ static MsGraph ms_graph_of(bfsx_ctx *ctx, bool symmetric) {
   if (ctx->row_idx_pull.p) g.row_idx_pull = ctx->row_idx_pull.as<uint32_t>();
   if (!symmetric || !ctx->params.ms_relabel) return g;
   if (!ctx->ms_relabelled) {
-    hipStream_t s = ctx->stream;
     const uint64_t n = ctx->n_cols;
-    ensure(ctx->ms_rank, sizeof(uint32_t) * std::max<uint64_t>(n, 1), s);
-    ensure(ctx->ms_order, sizeof(uint32_t) * std::max<uint64_t>(n, 1), s);
-    ensure(ctx->ms_rcp, (size_t)ctx->ptr_bytes * (n + 1), s);
-    ensure(ctx->ms_rri, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), s);
+    ensure(ctx->ms_rank, sizeof(uint32_t) * std::max<uint64_t>(n, 1), ctx);
+    ensure(ctx->ms_order, sizeof(uint32_t) * std::max<uint64_t>(n, 1), ctx);
+    ensure(ctx->ms_rcp, (size_t)ctx->ptr_bytes * (n + 1), ctx);
+    ensure(ctx->ms_rri, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), ctx);
     relabel_by_degree(ctx, ctx->ms_rank.as<uint32_t>(), ctx->ms_order.as<uint32_t>(),
                       ctx->ms_rcp.p, ctx->ms_rri.as<uint32_t>());
     ctx->ms_relabelled = true;
@@ -605,14 +604,14 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
   const bool symmetric = (ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols;
   const MsGraph G = ms_graph_of(ctx, symmetric);
   const PtrT *gcp = static_cast<const PtrT *>(G.col_ptr);
-  ensure(ctx->ms_seen, sizeof(uint32_t) * n * W, s);
-  ensure(ctx->ms_cur, sizeof(uint32_t) * n * W, s);
-  ensure(ctx->ms_nxt, sizeof(uint32_t) * n * W, s);
-  ensure(ctx->ms_lv, (size_t)n * NB, s);
-  ensure(ctx->ms_hubs, sizeof(uint32_t) * (n + 1), s);
+  ensure(ctx->ms_seen, sizeof(uint32_t) * n * W, ctx);
+  ensure(ctx->ms_cur, sizeof(uint32_t) * n * W, ctx);
+  ensure(ctx->ms_nxt, sizeof(uint32_t) * n * W, ctx);
+  ensure(ctx->ms_lv, (size_t)n * NB, ctx);
+  ensure(ctx->ms_hubs, sizeof(uint32_t) * (n + 1), ctx);
   const size_t act_words = n / 32 + 2;
-  ensure(ctx->ms_act, sizeof(uint32_t) * 2 * act_words, s);
-  ensure(ctx->scratch, 64, s);
+  ensure(ctx->ms_act, sizeof(uint32_t) * 2 * act_words, ctx);
+  ensure(ctx->scratch, 64, ctx);
   uint32_t *seen = ctx->ms_seen.as<uint32_t>();
   uint32_t *buf[2] = {ctx->ms_cur.as<uint32_t>(), ctx->ms_nxt.as<uint32_t>()};
   uint32_t *act[2] = {ctx->ms_act.as<uint32_t>(), ctx->ms_act.as<uint32_t>() + act_words};
@@ -646,7 +645,7 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
   // vertices that bottom-up levels hand to k_ms_pull_hubs
   uint32_t n_phubs = 0;
   if (symmetric) {
-    ensure(ctx->ms_phubs, sizeof(uint32_t) * ((uint64_t)ctx->n_rows + 1), s);
+    ensure(ctx->ms_phubs, sizeof(uint32_t) * ((uint64_t)ctx->n_rows + 1), ctx);
     uint32_t *d_np = ctx->scratch.as<uint32_t>() + 12;
     BFSX_HIP(hipMemsetAsync(d_np, 0, sizeof(uint32_t), s));
     hipLaunchKernelGGL(k_ms_hub_list<PtrT>, dim3(ms_grid(ctx->n_rows, 256, cap)), dim3(256), 0, s,
@@ -767,13 +766,13 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
     DevBuf out, plain;
     const uint8_t *rows = lv;
     if (G.rank) {  // back to the caller's vertex ids
-      ensure(plain, (size_t)n * NB, s);
+      ensure(plain, (size_t)n * NB, ctx);
       hipLaunchKernelGGL(k_ms_unrename, dim3(ms_grid(n * (NB / 16), 256, cap)), dim3(256), 0, s,
                          reinterpret_cast<const uint4 *>(lv), NB / 16, (uint32_t)n, G.rank,
                          plain.as<uint4>());
       rows = plain.as<uint8_t>();
     }
-    ensure(out, (size_t)n_bits * n, s);
+    ensure(out, (size_t)n_bits * n, ctx);
     hipLaunchKernelGGL(k_ms_transpose, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, rows, NB,
                        n_bits, (uint32_t)n, out.as<uint8_t>());
     BFSX_HIP(hipGetLastError());
@@ -800,8 +799,8 @@ MsResult ms_run(bfsx_ctx *ctx, const uint32_t *sources, const uint16_t *bits, ui
   distinct.erase(std::unique(distinct.begin(), distinct.end()), distinct.end());
   hipStream_t s = ctx->stream;
   DevBuf ds, db;
-  ensure(ds, sizeof(uint32_t) * n_src, s);
-  ensure(db, sizeof(uint16_t) * n_src, s);
+  ensure(ds, sizeof(uint32_t) * n_src, ctx);
+  ensure(db, sizeof(uint16_t) * n_src, ctx);
   BFSX_HIP(hipMemcpyAsync(ds.p, sources, sizeof(uint32_t) * n_src, hipMemcpyHostToDevice, s));
   BFSX_HIP(hipMemcpyAsync(db.p, bits, sizeof(uint16_t) * n_src, hipMemcpyHostToDevice, s));
   const int W = n_bits <= 32 ? 1 : n_bits <= 64 ? 2 : n_bits <= 128 ? 4 : 8;

@@ -198,20 +198,20 @@ struct TrainBufs {
 static void upload_batch(bfsx_ctx *ctx, TrainBufs &b, const float *X, const float *T,
                          const float *M, uint32_t n, const float *W) {
   hipStream_t s = ctx->stream;
-  ensure(b.X, sizeof(float) * IN * (size_t)n, s);
-  ensure(b.W, sizeof(float) * NPARAM, s);
+  ensure(b.X, sizeof(float) * IN * (size_t)n, ctx);
+  ensure(b.W, sizeof(float) * NPARAM, ctx);
   BFSX_HIP(hipMemcpyAsync(b.X.p, X, sizeof(float) * IN * (size_t)n, hipMemcpyHostToDevice, s));
   BFSX_HIP(hipMemcpyAsync(b.W.p, W, sizeof(float) * NPARAM, hipMemcpyHostToDevice, s));
   if (T) {
-    ensure(b.T, sizeof(float) * OUT * (size_t)n, s);
-    ensure(b.M, sizeof(float) * OUT * (size_t)n, s);
+    ensure(b.T, sizeof(float) * OUT * (size_t)n, ctx);
+    ensure(b.M, sizeof(float) * OUT * (size_t)n, ctx);
     BFSX_HIP(hipMemcpyAsync(b.T.p, T, sizeof(float) * OUT * (size_t)n, hipMemcpyHostToDevice, s));
     BFSX_HIP(hipMemcpyAsync(b.M.p, M, sizeof(float) * OUT * (size_t)n, hipMemcpyHostToDevice, s));
     for (DevBuf *d : {&b.A1, &b.A2, &b.D1, &b.D2})
-      ensure(*d, sizeof(float) * 32 * (size_t)n, s);
-    ensure(b.D3, sizeof(float) * OUT * (size_t)n, s);
-    ensure(b.L, sizeof(float) * (size_t)n, s);
-    ensure(b.G, sizeof(float) * NPARAM, s);
+      ensure(*d, sizeof(float) * 32 * (size_t)n, ctx);
+    ensure(b.D3, sizeof(float) * OUT * (size_t)n, ctx);
+    ensure(b.L, sizeof(float) * (size_t)n, ctx);
+    ensure(b.G, sizeof(float) * NPARAM, ctx);
   }
 }
 
@@ -245,7 +245,7 @@ void mlp_forward(bfsx_ctx *ctx, const float *X, uint32_t n, const float *W, floa
   try {
     upload_batch(ctx, b, X, nullptr, nullptr, n, W);
     DevBuf y;
-    ensure(y, sizeof(float) * OUT * (size_t)n, ctx->stream);
+    ensure(y, sizeof(float) * OUT * (size_t)n, ctx);
     hipLaunchKernelGGL(k_mlp_forward, dim3((n + 255) / 256), dim3(256), 0, ctx->stream,
                        b.X.as<float>(), n, b.W.as<float>(), y.as<float>());
     BFSX_HIP(hipGetLastError());
@@ -266,7 +266,7 @@ void mlp_loss_grad(bfsx_ctx *ctx, const float *X, const float *T, const float *M
   try {
     const float inv = mask_inv_count(M, n);
     upload_batch(ctx, b, X, T, M, n, W);
-    ensure(b.loss, sizeof(float), ctx->stream);
+    ensure(b.loss, sizeof(float), ctx);
     grad_pass(ctx, b, n, inv, b.loss.as<float>());
     BFSX_HIP(hipMemcpyAsync(grad, b.G.p, sizeof(float) * NPARAM, hipMemcpyDeviceToHost,
                             ctx->stream));
@@ -286,9 +286,9 @@ void mlp_train(bfsx_ctx *ctx, const float *X, const float *T, const float *M, ui
     const float inv = mask_inv_count(M, n);
     upload_batch(ctx, b, X, T, M, n, W);
     hipStream_t s = ctx->stream;
-    ensure(b.m, sizeof(float) * NPARAM, s);
-    ensure(b.v, sizeof(float) * NPARAM, s);
-    ensure(b.loss, sizeof(float) * (epochs ? epochs : 1), s);
+    ensure(b.m, sizeof(float) * NPARAM, ctx);
+    ensure(b.v, sizeof(float) * NPARAM, ctx);
+    ensure(b.loss, sizeof(float) * (epochs ? epochs : 1), ctx);
     BFSX_HIP(hipMemsetAsync(b.m.p, 0, sizeof(float) * NPARAM, s));
     BFSX_HIP(hipMemsetAsync(b.v.p, 0, sizeof(float) * NPARAM, s));
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;

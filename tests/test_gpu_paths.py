@@ -224,3 +224,85 @@ def test_levels_and_graphs_to_pageable_memory(engine, depth, n):
     ok = par[1:depth + 1] == np.arange(depth)
     assert ok.all() and (par[leaf] == 0).all() and par[0] == 0
     assert (par[want < 0] == 0xFFFFFFFF).all()
+
+
+# a graph is checked on the card beside the resident one: refused graphs leave
+# that as it was, wherever the bad entry is
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+@pytest.mark.parametrize("nnz", [4, 7, 1023, 400001])
+def test_refused_graphs(engine, ptr, nnz):
+    import bfsx
+    say("refused", ptr.__name__, nnz)
+    cp0, ri0 = path_graph(100)
+    engine.upload_csc(cp0, ri0, symmetric=True)
+    rng = np.random.default_rng(nnz)
+    n = max(3, nnz // 5)
+    src = np.sort(rng.integers(0, n, nnz))
+    cp = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(ptr)
+    ri = rng.integers(0, n, nnz).astype(np.uint32)
+
+    def refused(cp, ri, text, n_rows=None):
+        with pytest.raises(bfsx.BfsxError) as e:
+            engine.upload_csc(cp, ri, n_rows=n_rows)
+        assert e.value.status == 1 and text in e.value.msg
+        lev, _ = engine.run(99, "llb")
+        assert (lev == 99 - np.arange(100)).all()
+
+    for at in sorted({0, 1, nnz // 2, nnz - 1}):
+        bad = ri.copy()
+        bad[at] = n
+        refused(cp, bad, "row_idx entry >= n_cols")
+        bad[at] = 0xFFFFFFFF
+        refused(cp, bad, "row_idx entry >= n_cols")
+    for at in sorted({1, n // 2, n - 1}):
+        bad = cp.copy()
+        bad[at] = nnz + 9
+        refused(bad, ri, "not monotone")
+    refused(cp + ptr(1), ri, "col_ptr[0] != 0")
+    refused(cp, ri[:-1], "end does not match")
+    engine.upload_csc(cp, ri)
+    got_cp, got_ri = engine.download_csc()
+    assert (got_cp == cp).all() and (got_ri == ri).all()
+
+
+# runs of 4096 edges find their columns: a list longer than a run, more than
+# 4096 empty columns inside one, lists behind n_rows; chunks of 2048 vertices
+@pytest.mark.parametrize("shape", ["hub", "gaps", "tail", "small"])
+@pytest.mark.parametrize("order", ["hub_first", "id", "pull_hub_first"])
+def test_order_adjacency_runs(engine, shape, order):
+    say("order", shape, order)
+    rng = np.random.default_rng(len(shape))
+    n = {"hub": 30011, "gaps": 70001, "tail": 5000, "small": 3}[shape]
+    if shape == "hub":
+        src = np.concatenate([np.full(20000, 7), rng.integers(0, n, 30000)])
+    elif shape == "gaps":
+        src = np.concatenate([rng.integers(0, 50, 9000), np.full(3, 20000), np.full(9000, n - 2)])
+    else:
+        src = rng.integers(0, n, 4 * n)
+    dst = rng.integers(0, n, len(src))
+    sym = shape != "tail"
+    e = symmetrize(src, dst) if sym else (src, dst)
+    cp, ri = csc_from_edges(n, *e)
+    ri = ri.copy()
+    for v in range(n):  # any order: the lists are sorted by the engine
+        rng.shuffle(ri[cp[v]:cp[v + 1]])
+    n_rows = n if sym else n - 1000
+    engine.upload_csc(cp, ri, n_rows=n_rows, symmetric=sym)
+    engine.order_adjacency(order)
+    got_cp, got = engine.download_csc()
+    deg = np.diff(cp.astype(np.int64)) * (np.arange(n) < n_rows)
+    rank = np.empty(n, np.int64)
+    rank[np.lexsort((np.arange(n), -deg))] = np.arange(n)
+    col = np.repeat(np.arange(n), np.diff(cp.astype(np.int64)))
+    assert (got_cp == cp).all()
+    if order == "pull_hub_first":
+        assert (got == ri).all()
+    else:
+        key = ri.astype(np.int64) if order == "id" else rank[ri]
+        want = ri[np.lexsort((key, col))]
+        rows = slice(0, int(cp[n_rows]))
+        assert (got[rows] == want[rows]).all()
+    for root in rng.integers(0, n_rows, 3):
+        want, _, _ = cpu.bfs_queue(cp, ri, int(root), n_rows=n_rows)
+        for s in ["llb", "glb"] + (["pull"] if sym else []):
+            assert (engine.run(int(root), s)[0] == want).all(), (s, root)
