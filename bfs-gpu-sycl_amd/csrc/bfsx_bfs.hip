@@ -1639,8 +1639,12 @@ __global__ __launch_bounds__(WG) void k_pull(KArgs a, const uint32_t *fbm_cur,
 // two phases per chunk.  Phase 1 decides every candidate it can from its
 // first (highest-degree) neighbour alone: fd entry, one probe (of the hub
 // bitmap for a hub); candidates left undecided with more neighbours get a
-// bit in an LDS mask.  Phase 2 takes those 64 * PULL_SLOTS at a time: their
-// col_ptr pair, then the rest of the list (scan_rest).
+// bit in an LDS mask.  Phase 2 takes those 64 * PULL_SLOTS at a time: the
+// next three neighbours from a 16-byte entry beside fd (in the order of the
+// vertices with neighbours, so a dense level reads whole lines of it), three
+// probes in flight, and only the fifth neighbour on from the list
+// (scan_rest).  Through col_ptr and the list, two lines of a candidate's own,
+// R-MAT 26's second levels took 510 and 360 us, now 430 and 330.
 // Separating them keeps the short rounds of phase 1 from waiting for the
 // long chain (col_ptr, list line, probes) of a few undecided lanes.
 // Otherwise as k_pull: found vertices set bits in 64 LDS words the wave then
@@ -1651,7 +1655,7 @@ __global__ __launch_bounds__(WG) void k_pull2(KArgs a, const uint32_t *fbm_cur,
                                               uint32_t *fbm_next, const uint32_t *g_sum,
                                               uint32_t sum_words, uint32_t shift,
                                               const uint32_t *fd, const uint16_t *fdd,
-                                              const uint32_t *iso,
+                                              const uint4 *fn, const uint32_t *iso,
                                               const uint32_t *crank, const uint32_t *hbm,
                                               const uint32_t *hub, SpecGuard guard) {
   if (guard.skip()) return;
@@ -1760,34 +1764,56 @@ __global__ __launch_bounds__(WG) void k_pull2(KArgs a, const uint32_t *fbm_cur,
       const uint32_t incl2 = wave_incl_scan(cnt2);
       const uint32_t total2 = __shfl(incl2, 63, 64);
       const uint32_t excl2 = incl2 - cnt2;
+      const PtrT cfirst = col_ptr[c * PULL_CHUNK];
       for (uint32_t r = 0; r < total2; r += 64 * PULL_SLOTS) {
         bool cand[PULL_SLOTS];
-        uint32_t off[PULL_SLOTS];
+        uint32_t off[PULL_SLOTS], fi[PULL_SLOTS];
 #pragma unroll
         for (int sl = 0; sl < PULL_SLOTS; sl++) {
           const uint32_t idx = r + 64 * sl + lane;
           cand[sl] = idx < total2;
-          uint32_t o = 0, bit = 0;
-          if (r + 64 * sl < total2) wave_kth_bit(um, excl2, idx, o, bit);
+          uint32_t o = 0, bit = 0, rk = lbase;
+          if (r + 64 * sl < total2) {
+            wave_kth_bit(um, excl2, idx, o, bit);
+            rk = rank_of(o, bit);
+          }
           off[sl] = cand[sl] ? o * 32 + bit : 0u;
+          fi[sl] = cand[sl] ? rk : lbase;
         }
-        // (u is a vertex of this chunk below n_rows for every lane)
-        PtrT cb[PULL_SLOTS], ce[PULL_SLOTS];
+        uint4 nb[PULL_SLOTS];
+        uint32_t d16[PULL_SLOTS];
 #pragma unroll
         for (int sl = 0; sl < PULL_SLOTS; sl++) {
-          cb[sl] = col_ptr[c * PULL_CHUNK + off[sl]];
-          ce[sl] = col_ptr[c * PULL_CHUNK + off[sl] + 1];
+          nb[sl] = fn[fi[sl]];
+          d16[sl] = fdd[fi[sl]];
+        }
+        bool h[PULL_SLOTS][3];
+#pragma unroll
+        for (int sl = 0; sl < PULL_SLOTS; sl++) {
+          h[sl][0] = in_frontier_fd<SUM>(fbm_cur, hbm, s_sum, shift, cand[sl] ? nb[sl].x : 0u);
+          h[sl][1] = in_frontier_fd<SUM>(fbm_cur, hbm, s_sum, shift, cand[sl] ? nb[sl].y : 0u);
+          h[sl][2] = in_frontier_fd<SUM>(fbm_cur, hbm, s_sum, shift, cand[sl] ? nb[sl].z : 0u);
         }
 #pragma unroll
         for (int sl = 0; sl < PULL_SLOTS; sl++) {
-          const PtrT deg = cand[sl] ? ce[sl] - cb[sl] : PtrT(0);
-          bool found = false;
-          uint32_t par = 0;
-          // (the first neighbour is done; not a candidate: an empty range)
-          scan_rest<PtrT, SUM>(a, fbm_cur, s_sum, shift, cand[sl], found, par, cb[sl] + 1,
-                               cand[sl] ? cb[sl] + deg : cb[sl] + 1, scanned);
+          const uint32_t u = c * PULL_CHUNK + off[sl];
+          bool found = cand[sl] && (h[sl][0] | h[sl][1] | h[sl][2]);
+          const uint32_t nm = h[sl][0] ? nb[sl].x : h[sl][1] ? nb[sl].y : nb[sl].z;
+          uint32_t par = nm;
+          if (a.parents && found && hbm && (nm & PULL_HUB_FLAG)) par = hub[nm & ~PULL_HUB_FLAG];
+          PtrT deg = d16[sl];
+          if (cand[sl] && d16[sl] == DEG16_ESCAPE) deg = col_ptr[u + 1] - col_ptr[u];
+          if (a.examined && cand[sl]) scanned += deg < 4 ? (uint32_t)deg - 1 : 3u;
+          // the fifth neighbour on, from the list
+          const bool more = cand[sl] && !found && deg > 4;
+          if (__ballot(more)) {  // (wave-uniform: scan_rest is collective)
+            PtrT b = 0;
+            if (more)
+              b = (nb[sl].w != 0xFFFFFFFFu ? cfirst + (PtrT)nb[sl].w : col_ptr[u]) + 4;
+            scan_rest<PtrT, SUM>(a, fbm_cur, s_sum, shift, more, found, par, b,
+                                 more ? b + (deg - 4) : b, scanned);
+          }
           if (found) {
-            const uint32_t u = c * PULL_CHUNK + off[sl];
             a.levels[u] = a.next_level;
             if (a.parents) a.parents[u] = par;
             atomicOr(&fw[off[sl] >> 5], 1u << (off[sl] & 31));
@@ -2874,16 +2900,16 @@ template <typename PtrT, int WG>
 static void launch_pull(unsigned grid, size_t lds, hipStream_t st, const KArgs &a,
                         const StepArgs &s, const uint32_t *g_sum, uint32_t sum_words,
                         uint32_t shift, const uint32_t *fd, const uint16_t *fdd,
-                        const uint32_t *iso,
+                        const uint4 *fn, const uint32_t *iso,
                         const uint32_t *crank, const uint32_t *hbm, const uint32_t *hub,
                         SpecGuard guard) {
   if (fd) {
     if (g_sum)
       hipLaunchKernelGGL((k_pull2<PtrT, WG, true>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
-                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, iso, crank, hbm, hub, guard);
+                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard);
     else
       hipLaunchKernelGGL((k_pull2<PtrT, WG, false>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
-                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, iso, crank, hbm, hub, guard);
+                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard);
   } else {
     if (g_sum)
       hipLaunchKernelGGL((k_pull<PtrT, WG, true>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
@@ -2936,6 +2962,7 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
                            ? ctx->pull_fd.as<uint32_t>()
                            : nullptr;
   const uint16_t *fdd = fd ? ctx->pull_fdd.as<uint16_t>() : nullptr;
+  const uint4 *fn = fd ? ctx->pull_fn.as<uint4>() : nullptr;
   // (its entries exist for the vertices with neighbours: the others must
   // start visited, which a search does on a symmetric graph)
   if (fd && !((ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols))
@@ -2953,10 +2980,10 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   }
   KernelTimer kt(s, st);
   switch (wg) {
-    case 64: launch_pull<PtrT, 64>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, iso, crank, hbm, hub, guard); break;
-    case 128: launch_pull<PtrT, 128>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, iso, crank, hbm, hub, guard); break;
-    case 256: launch_pull<PtrT, 256>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, iso, crank, hbm, hub, guard); break;
-    case 512: launch_pull<PtrT, 512>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, iso, crank, hbm, hub, guard); break;
+    case 64: launch_pull<PtrT, 64>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
+    case 128: launch_pull<PtrT, 128>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
+    case 256: launch_pull<PtrT, 256>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
+    case 512: launch_pull<PtrT, 512>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
     default: fail(BFSX_ERR_ARG, "pull_wg must be 64, 128, 256 or 512");
   }
 }

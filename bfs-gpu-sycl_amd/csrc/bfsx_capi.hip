@@ -135,6 +135,7 @@ static void ensure_pull_state(bfsx_ctx *ctx) {
 static void drop_pull_fd(bfsx_ctx *ctx) {
   release(ctx->pull_fd);
   release(ctx->pull_fdd);
+  release(ctx->pull_fn);
   release(ctx->pull_crank);
   release(ctx->pull_hub);
   release(ctx->pull_hbm);
@@ -1244,17 +1245,19 @@ int bfsx_order_adjacency(bfsx_ctx *ctx, int order) {
            "order must be BFSX_ORDER_ID, BFSX_ORDER_HUB_FIRST or BFSX_ORDER_PULL_HUB_FIRST");
     if (order == BFSX_ORDER_PULL_HUB_FIRST) {
       ensure(ctx->row_idx_pull, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), ctx);
-      DevBuf by_degree;  // the vertices, largest degree first
+      DevBuf by_degree, hrank;  // the vertices, largest degree first; hub indexes
       struct Releaser {
-        DevBuf &b;
-        ~Releaser() { release(b); }
-      } releaser{by_degree};
+        DevBuf *b[2];
+        ~Releaser() {
+          for (DevBuf *x : b) release(*x);
+        }
+      } releaser{{&by_degree, &hrank}};
       order_adjacency(ctx, true, ctx->row_idx_pull.as<uint32_t>(), &by_degree);
       if (ctx->max_degree < 0xFFFFFFFFull) {  // degrees fit the array's 32 bits
         ensure(ctx->pull_fd, sizeof(uint2) * std::max<uint64_t>(ctx->n_rows, 1), ctx);
         first_neighbours(ctx, ctx->row_idx_pull.as<uint32_t>(), ctx->pull_fd.as<uint2>());
-        index_hub_neighbours(ctx, by_degree.as<uint32_t>());
-        compact_first_neighbours(ctx);
+        index_hub_neighbours(ctx, by_degree.as<uint32_t>(), hrank);
+        compact_first_neighbours(ctx, hrank.as<uint32_t>());
       }
       build_hot_copy(ctx, by_degree.as<uint32_t>());
       ctx->gflags |= BFSX_GRAPH_PULL_COPY;

@@ -618,7 +618,7 @@ __global__ void k_fd_hub_index(uint2 *fd, uint32_t n_rows, const uint32_t *hrank
   }
 }
 
-void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree) {
+void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree, DevBuf &hrank) {
   release(ctx->pull_hub);
   release(ctx->pull_hbm);
   ctx->pull_hubs = 0;
@@ -633,7 +633,6 @@ void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree) {
   ensure(ctx->pull_hbm, sizeof(uint32_t) * (H / 32), ctx);
   BFSX_HIP(hipMemcpyAsync(ctx->pull_hub.p, by_degree, sizeof(uint32_t) * H,
                           hipMemcpyDeviceToDevice, s));
-  DevBuf hrank;
   ensure(hrank, sizeof(uint32_t) * ctx->n_cols, ctx);
   BFSX_HIP(hipMemsetAsync(hrank.p, 0xFF, sizeof(uint32_t) * ctx->n_cols, s));
   hipLaunchKernelGGL(k_hub_rank, dim3(grid_for(H)), dim3(256), 0, s,
@@ -641,8 +640,6 @@ void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree) {
   hipLaunchKernelGGL(k_fd_hub_index, dim3(grid_for(n)), dim3(256), 0, s,
                      ctx->pull_fd.as<uint2>(), n, hrank.as<uint32_t>());
   BFSX_HIP(hipGetLastError());
-  BFSX_HIP(hipStreamSynchronize(s));
-  release(hrank);
   ctx->pull_hubs = (uint32_t)H;
 }
 
@@ -693,17 +690,29 @@ __global__ __launch_bounds__(1024) void k_scan_runs(uint32_t *cnt, uint32_t n) {
   }
 }
 
-// out[crank[c] + k] = fd[v].x and outd[...] = min(fd[v].y, DEG16_ESCAPE) for
-// the k-th vertex v with neighbours of chunk c: a wave per chunk, 64 vertices
-// at a time, slots by the lanes below.  (A thread per chunk walked its 2048
-// vertices alone: 1027 us for 1 M vertices, 15 now.)
+// For the k-th vertex v with neighbours of chunk c, at r = crank[c] + k:
+// out[r] = fd[v].x, outd[r] = min(fd[v].y, DEG16_ESCAPE), and outn[r] = its
+// second to fourth neighbours (named as in fd: hubs by index; the second
+// repeated past the list's end) and where its list starts, counted from the
+// chunk's first list (~0u: that does not fit, see col_ptr).  A wave per
+// chunk, 64 vertices at a time, slots by the lanes below.  (A thread per
+// chunk walked its 2048 vertices alone: 1027 us for 1 M vertices without
+// outn, 15 by waves.)
+template <typename PtrT>
 __global__ __launch_bounds__(256) void k_fd_compact(const uint2 *fd, const uint32_t *iso,
                                                     uint32_t n_rows, uint32_t n_chunks,
-                                                    const uint32_t *crank, uint32_t *out,
-                                                    uint16_t *outd) {
+                                                    const uint32_t *crank, const PtrT *col_ptr,
+                                                    const uint32_t *row_idx,
+                                                    const uint32_t *hrank, uint32_t *out,
+                                                    uint16_t *outd, uint4 *outn) {
   const uint32_t lane = threadIdx.x & 63;
+  auto name = [&](uint32_t x) {
+    const uint32_t h = hrank ? hrank[x] : ~0u;
+    return h != ~0u ? PULL_HUB_FLAG | h : x;
+  };
   for (uint32_t c = blockIdx.x * 4 + (threadIdx.x >> 6); c < n_chunks; c += gridDim.x * 4) {
     uint32_t pos = crank[c];
+    const PtrT first = col_ptr[(uint64_t)c * PULL_CHUNK];
     const uint32_t word = linked_word(iso, c * 64 + lane, n_rows);
 #pragma unroll 4
     for (uint32_t i = 0; i < 32; i++) {
@@ -711,21 +720,29 @@ __global__ __launch_bounds__(256) void k_fd_compact(const uint2 *fd, const uint3
       const bool in = (w >> (lane & 31)) & 1u;
       const unsigned long long m = __ballot(in);
       if (in) {
-        const uint2 x = fd[(uint64_t)c * PULL_CHUNK + i * 64 + lane];
+        const uint64_t v = (uint64_t)c * PULL_CHUNK + i * 64 + lane;
+        const uint2 x = fd[v];
         const uint32_t p = pos + __builtin_amdgcn_mbcnt_hi(
                                      (uint32_t)(m >> 32),
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
         out[p] = x.x;
         outd[p] = (uint16_t)(x.y < DEG16_ESCAPE ? x.y : DEG16_ESCAPE);
+        const PtrT b = col_ptr[v];
+        const uint64_t rel = (uint64_t)(b - first);
+        const uint32_t n2 = x.y > 1 ? name(row_idx[b + 1]) : 0u;
+        outn[p] = make_uint4(n2, x.y > 2 ? name(row_idx[b + 2]) : n2,
+                             x.y > 3 ? name(row_idx[b + 3]) : n2,
+                             rel < 0xFFFFFFFFull ? (uint32_t)rel : 0xFFFFFFFFu);
       }
       pos += (uint32_t)__popcll(m);
     }
   }
 }
 
-void compact_first_neighbours(bfsx_ctx *ctx) {
+void compact_first_neighbours(bfsx_ctx *ctx, const uint32_t *hrank) {
   release(ctx->pull_crank);
   release(ctx->pull_fdd);
+  release(ctx->pull_fn);
   if (!ctx->pull_fd.p) return;
   hipStream_t s = ctx->stream;
   const uint32_t n = ctx->n_rows;
@@ -733,8 +750,8 @@ void compact_first_neighbours(bfsx_ctx *ctx) {
   ensure(ctx->pull_crank, sizeof(uint32_t) * ((uint64_t)n_chunks + 1), ctx);
   uint32_t *crank = ctx->pull_crank.as<uint32_t>();
   const uint32_t *iso = ctx->iso_bm.as<uint32_t>();
-  hipLaunchKernelGGL(k_chunk_linked, dim3(grid_for((uint64_t)n_chunks * 64)), dim3(256), 0, s, iso, n,
-                     n_chunks, crank);
+  hipLaunchKernelGGL(k_chunk_linked, dim3(grid_for((uint64_t)n_chunks * 64)), dim3(256), 0, s, iso,
+                     n, n_chunks, crank);
   hipLaunchKernelGGL(k_scan_runs, dim3(1), dim3(1024), 0, s, crank, n_chunks);
   BFSX_HIP(hipGetLastError());
   uint32_t linked = 0;
@@ -742,18 +759,31 @@ void compact_first_neighbours(bfsx_ctx *ctx) {
   BFSX_HIP(hipStreamSynchronize(s));
   if (linked != n - ctx->n_isolated) fail(BFSX_ERR_DEVICE, "isolated-vertex count mismatch");
   DevBuf out;
+  struct Releaser {
+    DevBuf &b;
+    ~Releaser() { release(b); }
+  } releaser{out};
   ensure(out, sizeof(uint32_t) * ((uint64_t)linked + 1), ctx);
   ensure(ctx->pull_fdd, sizeof(uint16_t) * ((uint64_t)linked + 1), ctx);
+  ensure(ctx->pull_fn, sizeof(uint4) * ((uint64_t)linked + 1), ctx);
   // the padding entry: a vertex with no neighbours (read, never used)
   BFSX_HIP(hipMemsetAsync(out.as<uint32_t>() + linked, 0, sizeof(uint32_t), s));
   BFSX_HIP(hipMemsetAsync(ctx->pull_fdd.as<uint16_t>() + linked, 0, sizeof(uint16_t), s));
-  hipLaunchKernelGGL(k_fd_compact, dim3(grid_for((uint64_t)n_chunks * 64)), dim3(256), 0, s,
-                     ctx->pull_fd.as<uint2>(), iso, n, n_chunks, crank, out.as<uint32_t>(),
-                     ctx->pull_fdd.as<uint16_t>());
+  BFSX_HIP(hipMemsetAsync(ctx->pull_fn.as<uint4>() + linked, 0, sizeof(uint4), s));
+  const dim3 grid(grid_for((uint64_t)n_chunks * 64));
+  if (ctx->ptr_bytes == 8)
+    hipLaunchKernelGGL(k_fd_compact<uint64_t>, grid, dim3(256), 0, s, ctx->pull_fd.as<uint2>(), iso,
+                       n, n_chunks, crank, ctx->col_ptr.as<uint64_t>(),
+                       ctx->row_idx_pull.as<uint32_t>(), hrank, out.as<uint32_t>(),
+                       ctx->pull_fdd.as<uint16_t>(), ctx->pull_fn.as<uint4>());
+  else
+    hipLaunchKernelGGL(k_fd_compact<uint32_t>, grid, dim3(256), 0, s, ctx->pull_fd.as<uint2>(), iso,
+                       n, n_chunks, crank, ctx->col_ptr.as<uint32_t>(),
+                       ctx->row_idx_pull.as<uint32_t>(), hrank, out.as<uint32_t>(),
+                       ctx->pull_fdd.as<uint16_t>(), ctx->pull_fn.as<uint4>());
   BFSX_HIP(hipGetLastError());
   BFSX_HIP(hipStreamSynchronize(s));
   std::swap(ctx->pull_fd, out);
-  release(out);
 }
 
 // out[k] = PULL_HUB_FLAG | hrank[x] for hot x = row_idx[k], else x

@@ -185,7 +185,11 @@ struct bfsx_ctx {
   // the vertices with neighbours before v in its PULL_CHUNK-vertex chunk
   // (from the isolated-vertex bitmap); one padding entry follows.  While the
   // arrays are built, pull_fd holds uint2 {first neighbour, degree} per vertex.
-  bfsx::DevBuf pull_fd, pull_fdd, pull_crank;
+  // pull_fn (uint4, at the same positions): the second to fourth neighbours,
+  // named as in pull_fd, and the list's start counted from the chunk's first
+  // list, so that a candidate with up to four neighbours needs neither its
+  // col_ptr entries nor its list (16 bytes instead of two cache lines).
+  bfsx::DevBuf pull_fd, pull_fdd, pull_crank, pull_fn;
   // The pull_hubs vertices of largest degree ("hubs") are named in pull_fd by
   // their index: fd[v].x = PULL_HUB_FLAG | h for the hub pull_hub[h].  Before
   // every bottom-up step their frontier bits are gathered into pull_hbm
@@ -287,13 +291,15 @@ void first_neighbours(bfsx_ctx *ctx, const uint32_t *row_idx, uint2 *fd);
 // Names the first neighbours that are among the graph's top-degree vertices
 // by their index in ctx->pull_hub (sets pull_hub, pull_hbm, pull_hubs); needs
 // ctx->pull_fd (one entry per vertex) and n_cols < 2^31; by_degree: the
-// vertices in degree order (order_adjacency).
-void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree);
+// vertices in degree order (order_adjacency).  hrank receives every vertex's
+// index among them (~0u: none), or stays empty without hubs.
+void index_hub_neighbours(bfsx_ctx *ctx, const uint32_t *by_degree, DevBuf &hrank);
 // Drops the isolated vertices' entries from ctx->pull_fd (one uint2 entry per
 // vertex before), splits it into ctx->pull_fd (first neighbours) and
-// ctx->pull_fdd (16-bit degrees), and builds ctx->pull_crank (needs the
-// isolated bitmap).
-void compact_first_neighbours(bfsx_ctx *ctx);
+// ctx->pull_fdd (16-bit degrees), and builds ctx->pull_fn (the next three
+// neighbours, hubs named by hrank if given) and ctx->pull_crank (needs the
+// isolated bitmap and row_idx_pull).
+void compact_first_neighbours(bfsx_ctx *ctx, const uint32_t *hrank);
 // Builds row_idx_hot / hot_id / hot_vis / hot_n for graphs of
 // HOT_MIN_VERTICES to 2^31 vertices (otherwise leaves hot_n = 0).
 constexpr uint32_t HOT_MIN_VERTICES = 1u << 24;

@@ -306,3 +306,35 @@ def test_order_adjacency_runs(engine, shape, order):
         want, _, _ = cpu.bfs_queue(cp, ri, int(root), n_rows=n_rows)
         for s in ["llb", "glb"] + (["pull"] if sym else []):
             assert (engine.run(int(root), s)[0] == want).all(), (s, root)
+
+
+# bottom-up with the hub-first copy: candidates of one to six neighbours (the
+# first four beside the list), degrees that the 16-bit array does not hold,
+# chunks of 2048 vertices, no hubs below 64 vertices
+@pytest.mark.parametrize("n", [5, 63, 64, 2047, 2048, 2049, 6000, 140001])
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+def test_bottom_up_short_lists(engine, n, ptr):
+    say("bottom-up", n, ptr.__name__)
+    rng = np.random.default_rng(n)
+    # vertex v picks v % 4 earlier neighbours; the largest graph's vertex 0 is
+    # next to every second vertex (degree 70000)
+    src = np.repeat(np.arange(n), np.arange(n) % 4)
+    dst = (rng.random(len(src)) * np.maximum(src, 1)).astype(np.int64)
+    if n > 100000:
+        even = np.arange(2, n, 2)
+        src, dst = np.concatenate([src, even]), np.concatenate([dst, np.zeros(len(even), np.int64)])
+    keep = src != dst
+    cp, ri = csc_from_edges(n, *symmetrize(src[keep], dst[keep]), dtype=ptr)
+    engine.upload_csc(cp, ri, symmetric=True)
+    engine.order_adjacency("pull_hub_first")
+    deg = np.diff(cp.astype(np.int64))
+    for root in {0, int(np.flatnonzero(deg)[-1]), int(np.argmin(np.where(deg > 0, deg, 9999999)))}:
+        want, ec, _ = cpu.bfs_queue(cp, ri, root)
+        lev, st, par = engine.run(root, "pull", parents=True)
+        assert (lev == want).all() and st["edges_count"] == ec
+        assert cpu.check_parents(cp, ri, root, want, par) == 0
+        engine.run(root, "pull", levels=False, step_times=True)
+        later = lambda k: (want > k) | (want < 0)
+        for t in engine.last_trace():
+            lo = int(deg[later(t["level"] + 1)].sum()) + int((want == t["level"] + 1).sum())
+            assert lo <= t["pull_scanned"] <= int(deg[later(t["level"])].sum())
