@@ -107,7 +107,7 @@ static void free_search_state(bfsx_ctx *ctx) {
                     &ctx->glb_tile, &ctx->glb_chunk_lo, &ctx->mark, &ctx->fsum, &ctx->bkt,
                     &ctx->bkt_cnt, &ctx->bkt_tot, &ctx->bkt_base, &ctx->ms_seen,
                     &ctx->ms_cur, &ctx->ms_nxt, &ctx->ms_lv, &ctx->ms_hubs, &ctx->ms_phubs,
-                    &ctx->ms_act})
+                    &ctx->ms_act, &ctx->ms_part})
     release(*b);
 }
 
@@ -209,8 +209,7 @@ struct RunOut {
   unsigned long long reached = 0, edges = 0;
 };
 
-// Full copy of the control block into h_ctl (stream synchronised).
-static void read_ctl(bfsx_ctx *ctx) {
+void read_ctl(bfsx_ctx *ctx) {
   BFSX_HIP(hipMemcpyAsync(ctx->h_ctl, ctx->ctl.p, sizeof(LevelCtl), hipMemcpyDeviceToHost,
                           ctx->stream));
   BFSX_HIP(hipStreamSynchronize(ctx->stream));

@@ -235,7 +235,7 @@ struct bfsx_ctx {
   hipEvent_t ev_k0 = nullptr, ev_k1 = nullptr;  // main kernel of a timed step
 
   // batched multi-source search state
-  bfsx::DevBuf ms_seen, ms_cur, ms_nxt, ms_lv, ms_hubs, ms_phubs, ms_act;
+  bfsx::DevBuf ms_seen, ms_cur, ms_nxt, ms_lv, ms_hubs, ms_phubs, ms_act, ms_part;
   // the graph relabelled by degree for batched searches (made on first use)
   bfsx::DevBuf ms_rcp, ms_rri, ms_rank, ms_order;
   bool ms_relabelled = false;
@@ -315,6 +315,9 @@ void top_degree_vertices(bfsx_ctx *ctx, uint32_t k, uint32_t *d_out);
 void root_candidates(bfsx_ctx *ctx, uint64_t seed, uint64_t first,
                      uint32_t count, const int32_t *d_component_levels,
                      uint32_t *d_out_vertex, uint8_t *d_out_ok);
+
+// Full copy of the control block into h_ctl (stream synchronised).
+void read_ctl(bfsx_ctx *ctx);
 
 // ---- search kernels (bfsx_bfs.hip) ---------------------------------------
 struct StepArgs {

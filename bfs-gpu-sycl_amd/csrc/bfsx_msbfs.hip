@@ -12,14 +12,15 @@
 // finalize pass keeps only unseen bits) or bottom-up (many: a group of W
 // lanes owns a vertex and ORs its neighbours' frontier words, word j in lane
 // j, stopping as soon as every search has reached the vertex).  Both write
-// levels for the new bits and append vertices with new bits to the active
-// queue with one atomic per wave.  A source set may hold several vertices
-// for one bit; the result is then the distance to the nearest of them, which
-// is how disjoint graphs packed into one CSC run in the same launch.
+// levels for the new bits and set the bit of every vertex with new bits in a
+// map, from which a top-down level lists its active vertices.  A source set
+// may hold several vertices for one bit; the result is then the distance to
+// the nearest of them, which is how disjoint graphs packed into one CSC run
+// in the same launch.
 //
 // The level loop is device-driven: K levels are captured once into a
 // hipGraph and replayed.  Each level's kernels read the frontier size, the
-// level and the direction from the control block; a one-wave kernel at the
+// level and the direction from the control block; a one-group kernel at the
 // start of a level picks the direction (top-down while the frontier's edges
 // times ms_push_divisor stay below nnz), one at the end counts, sets the
 // termination flag and writes the level-end words the host polls once per
@@ -39,31 +40,43 @@ namespace bfsx {
 
 namespace {
 
-__device__ __forceinline__ uint32_t ms_lanes_below(unsigned long long m) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                   __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// Appends u once per group (the group's first lane) with one atomic per wave.
-__device__ __forceinline__ void ms_append(bool leader_with_new, uint32_t u, uint32_t *q,
-                                          uint32_t *qc) {
-  const unsigned long long m = __ballot(leader_with_new);
-  if (!m) return;
-  const int first = __ffsll((unsigned long long)m) - 1;
-  uint32_t base = 0;
-  if ((int)__lane_id() == first) base = atomicAdd(qc, (uint32_t)__popcll(m));
-  base = __shfl(base, first, 64);
-  if (leader_with_new) q[base + ms_lanes_below(m)] = u;
-}
-
-// Writes level L for the set bits of `bits` (word j of vertex u).
+// Writes level L for the set bits of `bits` (word j of vertex u): the 32
+// bytes of a word belong to one lane, so beyond a few bits they are read,
+// blended four at a time and written back as two 16-byte words (a byte store
+// per bit is up to 32 stores of a lane).
 __device__ __forceinline__ void ms_write_levels(uint8_t *lv, uint32_t NB, uint32_t u, uint32_t j,
                                                 uint32_t bits, uint8_t L) {
   uint8_t *p = lv + (size_t)u * NB + 32 * j;
-  for (uint32_t b = bits; b; b &= b - 1) p[__ffs(b) - 1] = L;
+  if (__popc(bits) <= 3) {
+    for (uint32_t b = bits; b; b &= b - 1) p[__ffs(b) - 1] = L;
+    return;
+  }
+  uint4 *q = reinterpret_cast<uint4 *>(p);
+  uint4 x[2] = {q[0], q[1]};
+  uint32_t *w = reinterpret_cast<uint32_t *>(x);
+  const uint32_t L4 = 0x01010101u * L;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    // one byte of ones per set bit of the nibble
+    const uint32_t m = ((((bits >> (4 * i)) & 15u) * 0x00204081u) & 0x01010101u) * 255u;
+    w[i] = (w[i] & ~m) | (L4 & m);
+  }
+  q[0] = x[0];
+  q[1] = x[1];
 }
 
 }  // namespace
+
+// A level's totals (vertices with new bits, their out-degree sum) in
+// MS_PARTS parts, a cache line each: the work-groups add to part (group mod
+// MS_PARTS) and k_ms_end adds the parts up.  Atomics on one line take 12 ns
+// each; one per wave for the queue and one for the edges were three quarters
+// of a bottom-up level on R-MAT 18 (504 us, 65 K atomics).
+constexpr uint32_t MS_PARTS = 256;
+struct alignas(64) MsPart {
+  unsigned long long edges;
+  uint32_t count;
+};
 
 struct MsArgs {
   const void *col_ptr;
@@ -72,12 +85,12 @@ struct MsArgs {
   uint32_t n_rows, n_cols;
   uint32_t *seen, *cur, *nxt;
   uint8_t *lv;
-  uint32_t *q_in, *q_out, *q_count_out;
-  uint32_t qi;     // queue buffer holding this level's active vertices
+  const uint32_t *q_in;  // this level's active vertices (top-down levels)
+  uint32_t qi;     // which counters of the control block describe them
   uint32_t F;      // (set from the control block at kernel start)
   uint32_t level;  // level being written (the new bits' level), likewise
   uint32_t *overflow;
-  unsigned long long *q_edges_out;  // out-degree sum of the next active queue
+  MsPart *part;    // totals of the vertices with new bits
   uint32_t pull_hub;  // bottom-up: longer lists go to k_ms_pull_hubs
   LevelCtl *ctl;
   // one bit per vertex: in some search's frontier (cur != 0); not used on
@@ -150,19 +163,38 @@ __device__ __forceinline__ uint32_t ms_gather8(const MsArgs &a, const uint32_t (
   return part;
 }
 
-// Adds deg(u) of each group leader that appended u, one atomic per wave.
-template <typename PtrT>
-__device__ __forceinline__ void ms_track(const PtrT *col_ptr, uint32_t n_rows, bool appended,
-                                         uint32_t u, unsigned long long *acc) {
-  unsigned long long d = (appended && u < n_rows) ? (unsigned long long)(col_ptr[u + 1] - col_ptr[u]) : 0ull;
-  for (int k = 32; k > 0; k >>= 1) d += __shfl_xor(d, k, 64);
-  if ((threadIdx.x & 63) == 0 && d) atomicAdd(acc, d);
+// Adds a work-group's totals to its part; every thread calls it.
+__device__ __forceinline__ void ms_add_totals(const MsArgs &a, uint32_t cnt,
+                                              unsigned long long deg) {
+  __shared__ uint32_t s_cnt;
+  __shared__ unsigned long long s_deg;
+  if (threadIdx.x == 0) {
+    s_cnt = 0;
+    s_deg = 0;
+  }
+  for (int k = 32; k > 0; k >>= 1) {
+    cnt += __shfl_xor(cnt, k, 64);
+    deg += __shfl_xor(deg, k, 64);
+  }
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0 && cnt) {
+    atomicAdd(&s_cnt, cnt);
+    atomicAdd(&s_deg, deg);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_cnt) {
+    MsPart *p = &a.part[blockIdx.x % MS_PARTS];
+    atomicAdd(&p->count, s_cnt);
+    atomicAdd(&p->edges, s_deg);
+  }
 }
 
 // ---- top-down: expand active vertices, atomicOr frontier words into nxt ----
-// Active vertices with more than MS_HUB edges go to a list that every wave
-// then splits (k_ms_push_hubs); the rest are expanded by one wave each.
-constexpr uint32_t MS_HUB = 2048;
+// Active vertices with more than MS_HUB edges go to a list whose edges
+// k_ms_push_hubs shares out in MS_HUB_SLICES slices each; the rest are
+// expanded by one wave each (256 sources of up to 2048 edges each held their
+// waves for 117 us on R-MAT 18).
+constexpr uint32_t MS_HUB = 256, MS_HUB_SLICES = 128;
 // Bottom-up levels hand vertices with more neighbours than a.pull_hub to
 // k_ms_pull_hubs (a work-group each): a W-lane group scanning a long list
 // alone would hold its wave for hundreds of rounds.
@@ -211,12 +243,13 @@ __global__ __launch_bounds__(256) void k_ms_push_hubs(MsArgs a, const uint32_t *
   const uint32_t grp = (threadIdx.x & 63) / W;
   const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
   const uint32_t nwaves = gridDim.x * 4;
-  const uint32_t nh = a.ctl->ms_hub_count;
-  for (uint32_t h = 0; h < nh; h++)
-    ms_push_edges<PtrT, W>(a, col_ptr, hubs[h], (PtrT)(wave * G + grp), (PtrT)nwaves * G);
+  const uint64_t items = (uint64_t)a.ctl->ms_hub_count * MS_HUB_SLICES;
+  for (uint64_t i = wave; i < items; i += nwaves)
+    ms_push_edges<PtrT, W>(a, col_ptr, hubs[i / MS_HUB_SLICES],
+                           (PtrT)((i % MS_HUB_SLICES) * G + grp), (PtrT)(MS_HUB_SLICES * G));
 }
 
-// ---- after a top-down level: keep unseen bits, levels, next active queue ----
+// ---- after a top-down level: keep unseen bits, levels, next active map --------
 // Also clears this level's frontier words (cur), which become the next
 // level's nxt: a following top-down level finds them zero.
 template <typename PtrT, int W>
@@ -227,6 +260,8 @@ __global__ __launch_bounds__(256) void k_ms_finalize(MsArgs a, uint32_t n_groups
   const uint32_t lane = threadIdx.x & 63, j = lane % W, grp = lane / W;
   const uint32_t NB = 32 * W;
   const uint32_t nwaves = gridDim.x * 4;
+  uint32_t cnt = 0;
+  unsigned long long deg = 0;
   for (uint32_t wv = blockIdx.x * 4 + (threadIdx.x >> 6); wv < n_groups_total; wv += nwaves) {
     const uint32_t u = wv * G + grp;
     uint32_t nb = 0;
@@ -247,11 +282,13 @@ __global__ __launch_bounds__(256) void k_ms_finalize(MsArgs a, uint32_t n_groups
     }
     const unsigned long long m = __ballot(nb != 0);
     const bool group_new = (m >> (grp * W)) & ((W == 64) ? ~0ull : ((1ull << W) - 1));
-    const bool app = group_new && j == 0 && u < a.n_cols;
-    ms_append(app, u, a.q_out, a.q_count_out);
-    ms_track<PtrT>(col_ptr, a.n_rows, app, u, a.q_edges_out);
+    if (group_new && j == 0) {  // (new bits: u < n_cols)
+      cnt++;
+      if (u < a.n_rows) deg += (unsigned long long)(col_ptr[u + 1] - col_ptr[u]);
+    }
     ms_mark_active<W>(a.act_next, wv * G, m);
   }
+  ms_add_totals(a, cnt, deg);
 }
 
 // ---- bottom-up: every vertex with unseen bits ORs its neighbours' frontier ----
@@ -265,6 +302,8 @@ __global__ __launch_bounds__(256) void k_ms_pull(MsArgs a, uint32_t n_groups_tot
   const uint32_t NB = 32 * W;
   const uint32_t nwaves = gridDim.x * 4;
   const unsigned long long gmask = ((W == 64) ? ~0ull : ((1ull << W) - 1)) << (grp * W);
+  uint32_t cnt = 0;
+  unsigned long long deg = 0;
   for (uint32_t wv = blockIdx.x * 4 + (threadIdx.x >> 6); wv < n_groups_total; wv += nwaves) {
     const uint32_t u = wv * G + grp;
     const bool valid = u < a.n_cols;
@@ -307,11 +346,13 @@ __global__ __launch_bounds__(256) void k_ms_pull(MsArgs a, uint32_t n_groups_tot
       else ms_write_levels(a.lv, NB, u, j, nb, (uint8_t)a.level);
     }
     const unsigned long long m = __ballot(nb != 0);
-    const bool app = (m & gmask) != 0 && j == 0 && valid;
-    ms_append(app, u, a.q_out, a.q_count_out);
-    ms_track<PtrT>(col_ptr, a.n_rows, app, u, a.q_edges_out);
+    if ((m & gmask) != 0 && j == 0 && valid) {
+      cnt++;
+      deg += (unsigned long long)(e - b);
+    }
     ms_mark_active<W>(a.act_next, wv * G, m);
   }
+  ms_add_totals(a, cnt, deg);
 }
 
 // Bottom-up for the vertices with more than MS_PULL_HUB neighbours: a work-group
@@ -370,8 +411,9 @@ __global__ __launch_bounds__(256) void k_ms_pull_hubs(MsArgs a, const uint32_t *
     bool any = false;
     for (int w = 0; w < W; w++) any = any || s_acc[w] != 0;
     if (any) {
-      a.q_out[atomicAdd(a.q_count_out, 1u)] = u;
-      atomicAdd(a.q_edges_out, (unsigned long long)(col_ptr[u + 1] - col_ptr[u]));
+      MsPart *p = &a.part[blockIdx.x % MS_PARTS];
+      atomicAdd(&p->count, 1u);
+      atomicAdd(&p->edges, (unsigned long long)(col_ptr[u + 1] - col_ptr[u]));
       atomicOr(&a.act_next[u >> 5], 1u << (u & 31));
     }
   }
@@ -386,41 +428,80 @@ __global__ void k_ms_hub_list(const PtrT *col_ptr, uint32_t n_rows, uint32_t pul
     if ((uint64_t)(col_ptr[u + 1] - col_ptr[u]) > pull_hub) hubs[atomicAdd(n_hubs, 1u)] = u;
 }
 
-// ---- level start and end (one wave each) -------------------------------------
-// Direction of the level, reset of the output queue's counters.
-__global__ void k_ms_begin(LevelCtl *ctl, uint32_t qi, uint64_t nnz, uint32_t divisor,
-                           int symmetric) {
-  if (threadIdx.x != 0 || ctl->done) return;
-  const uint32_t qo = qi ^ 1;
+// ---- level start and end (one work-group each) ----------------------------------
+// Direction of the level, reset of the totals (one part per thread).
+__global__ __launch_bounds__(MS_PARTS) void k_ms_begin(LevelCtl *ctl, uint32_t qi, uint64_t nnz,
+                                                       uint32_t divisor, int symmetric,
+                                                       MsPart *part) {
+  if (ctl->done) return;
+  part[threadIdx.x].count = 0;
+  part[threadIdx.x].edges = 0;
+  if (threadIdx.x != 0) return;
   const bool push = !symmetric || ctl->q_edges[qi] * (unsigned long long)divisor < nnz;
   ctl->ms_prev_pull = ctl->choice;
   ctl->choice = push ? 0u : 1u;
   ctl->ms_hub_count = 0;
-  ctl->q_count[qo] = 0;
-  ctl->q_edges[qo] = 0;
+  ctl->conv = 0;
 }
 
 // Clears the next-active map, and the nxt words when a top-down level
 // follows a bottom-up one (a bottom-up level writes every nxt word; a
 // top-down level's finalize leaves the next top-down level's nxt zero).
-__global__ void k_ms_clear(const LevelCtl *ctl, uint32_t *act_next, size_t act_words,
-                           uint32_t *nxt, size_t nxt_words) {
+// For a top-down level after the first, lists the active vertices from their
+// map (a word per thread, one atomic per work-group and step).
+__global__ __launch_bounds__(256) void k_ms_clear(LevelCtl *ctl, const uint32_t *act_cur,
+                                                  uint32_t *act_next, size_t act_words,
+                                                  uint32_t *nxt, size_t nxt_words, uint32_t *q) {
   if (ctl->done) return;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   const size_t i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   for (size_t i = i0; i < act_words; i += stride) act_next[i] = 0u;
-  if (ctl->choice == 0 && ctl->ms_prev_pull)
+  if (ctl->choice != 0) return;
+  if (ctl->ms_prev_pull)
     for (size_t i = i0; i < nxt_words; i += stride) nxt[i] = 0u;
+  if (ctl->level == 0) return;  // (the sources are listed by the host)
+  __shared__ uint32_t s_n, s_base;
+  for (size_t g = blockIdx.x * (size_t)blockDim.x; g < act_words; g += stride) {  // (uniform)
+    const size_t i = g + threadIdx.x;
+    const uint32_t bits = i < act_words ? act_cur[i] : 0u;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    uint32_t at = bits ? atomicAdd(&s_n, (uint32_t)__popc(bits)) : 0u;
+    __syncthreads();
+    if (threadIdx.x == 0 && s_n) s_base = atomicAdd(&ctl->conv, s_n);
+    __syncthreads();
+    if (bits) at += s_base;
+    for (uint32_t b = bits; b; b &= b - 1) q[at++] = (uint32_t)(i * 32) + (__ffs(b) - 1);
+    __syncthreads();  // s_n and s_base are rewritten by the next step
+  }
 }
 
-// Counts, termination, and the tagged level-end words for the host.
-__global__ void k_ms_end(LevelCtl *ctl, uint32_t qi, LevelMirror *mirror) {
-  if (threadIdx.x != 0) return;
+// Totals, termination, and the tagged level-end words for the host.
+__global__ __launch_bounds__(MS_PARTS) void k_ms_end(LevelCtl *ctl, uint32_t qi,
+                                                     const MsPart *part, LevelMirror *mirror) {
+  __shared__ uint32_t s_cnt;
+  __shared__ unsigned long long s_deg;
   const uint32_t qo = qi ^ 1;
+  if (threadIdx.x == 0) {
+    s_cnt = 0;
+    s_deg = 0;
+  }
+  __syncthreads();
+  if (!ctl->done) {  // (uniform)
+    const uint32_t c = part[threadIdx.x].count;
+    if (c) {
+      atomicAdd(&s_cnt, c);
+      atomicAdd(&s_deg, part[threadIdx.x].edges);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
   if (!ctl->done) {
     ctl->kind_count[ctl->choice ? 1 : 0]++;
     ctl->level += 1;
-    ctl->done = ctl->q_count[qo] == 0;
+    ctl->q_count[qo] = s_cnt;
+    ctl->q_edges[qo] = s_deg;
+    ctl->done = s_cnt == 0;
   }
   const uint32_t seq = ctl->seq + 1;
   ctl->seq = seq;
@@ -474,20 +555,57 @@ __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v) {
 }
 
 // ---- output: vertex-major [V][NB] -> one row per search [n_bits][V] -----------
-__global__ __launch_bounds__(256) void k_ms_transpose(const uint8_t *lv, uint32_t NB,
-                                                      uint32_t n_bits, uint32_t n_cols,
-                                                      uint8_t *out) {
-  __shared__ uint8_t tile[64][257];
-  const uint32_t v0 = blockIdx.x * 64;
-  // load 64 vertices x NB bytes
-  for (uint32_t i = threadIdx.x; i < 64 * NB; i += 256) {
-    const uint32_t dv = i / NB, b = i % NB;
-    tile[dv][b] = (v0 + dv < n_cols) ? lv[(size_t)(v0 + dv) * NB + b] : 0xFF;
+// A work-group takes MS_TV vertices (the searched ids rank[v] of MS_TV
+// consecutive caller's ids, so that renamed vertices need no pass of their
+// own): their levels go to LDS as 32-bit words in 16-byte reads, and a lane
+// turns the words of four vertices into four rows' words with byte
+// permutes.  Rows are written four bytes at a time where they are aligned
+// (quad: n_cols a multiple of 4).
+constexpr uint32_t MS_TV = 128;
+template <int W>
+__global__ __launch_bounds__(256) void k_ms_transpose(const uint8_t *lv, uint32_t n_bits,
+                                                      uint32_t n_cols, const uint32_t *rank,
+                                                      int quad, uint8_t *out) {
+  constexpr uint32_t NW = 8 * W;  // words per vertex
+  __shared__ uint32_t tile[MS_TV][NW + 1];
+  const uint64_t v0 = blockIdx.x * (uint64_t)MS_TV;
+  for (uint32_t i = threadIdx.x; i < MS_TV * (NW / 4); i += 256) {
+    const uint32_t dv = i / (NW / 4), k = i % (NW / 4);
+    const uint64_t v = v0 + dv;
+    if (v < n_cols) {
+      const uint32_t u = rank ? rank[v] : (uint32_t)v;
+      const uint4 x = reinterpret_cast<const uint4 *>(lv + (size_t)u * (32 * W))[k];
+      tile[dv][4 * k] = x.x;
+      tile[dv][4 * k + 1] = x.y;
+      tile[dv][4 * k + 2] = x.z;
+      tile[dv][4 * k + 3] = x.w;
+    }
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < 64 * n_bits; i += 256) {
-    const uint32_t b = i / 64, dv = i % 64;
-    if (v0 + dv < n_cols) out[(size_t)b * n_cols + v0 + dv] = tile[dv][b];
+  for (uint32_t i = threadIdx.x; i < (MS_TV / 4) * NW; i += 256) {
+    const uint32_t q = i % (MS_TV / 4), k = i / (MS_TV / 4);  // vertices 4q.., rows 4k..
+    const uint64_t v = v0 + 4 * q;
+    if (v >= n_cols) continue;
+    const uint32_t a = tile[4 * q][k], b = tile[4 * q + 1][k], c = tile[4 * q + 2][k],
+                   d = tile[4 * q + 3][k];
+    // byte r of a, b, c, d -> word r
+    const uint32_t ab_lo = __builtin_amdgcn_perm(b, a, 0x05010400u);  // a0 b0 a1 b1
+    const uint32_t ab_hi = __builtin_amdgcn_perm(b, a, 0x07030602u);  // a2 b2 a3 b3
+    const uint32_t cd_lo = __builtin_amdgcn_perm(d, c, 0x05010400u);
+    const uint32_t cd_hi = __builtin_amdgcn_perm(d, c, 0x07030602u);
+    const uint32_t r[4] = {(ab_lo & 0xFFFFu) | cd_lo << 16, ab_lo >> 16 | (cd_lo & 0xFFFF0000u),
+                           (ab_hi & 0xFFFFu) | cd_hi << 16, ab_hi >> 16 | (cd_hi & 0xFFFF0000u)};
+#pragma unroll
+    for (uint32_t t = 0; t < 4; t++) {
+      const uint32_t row = 4 * k + t;
+      if (row >= n_bits) break;
+      uint8_t *p = out + (size_t)row * n_cols + v;
+      if (quad) {
+        *reinterpret_cast<uint32_t *>(p) = r[t];
+      } else {
+        for (uint32_t y = 0; y < 4 && v + y < n_cols; y++) p[y] = (uint8_t)(r[t] >> (8 * y));
+      }
+    }
   }
 }
 
@@ -508,25 +626,19 @@ __global__ void k_ms_edges(const PtrT *col_ptr, const uint32_t *seen, uint32_t n
     }
     if (c) acc += (unsigned long long)c * (unsigned long long)(col_ptr[u + 1] - col_ptr[u]);
   }
+  __shared__ unsigned long long s_acc;
+  if (threadIdx.x == 0) s_acc = 0;
+  __syncthreads();
   for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
-  if ((threadIdx.x & 63) == 0 && acc) atomicAdd(out, acc);
+  if ((threadIdx.x & 63) == 0 && acc) atomicAdd(&s_acc, acc);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_acc) atomicAdd(out, s_acc);
 }
 
 // ---- renaming sources and levels ---------------------------------------------
 __global__ void k_ms_map(uint32_t *v, uint32_t n, const uint32_t *rank) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) v[i] = rank[v[i]];
-}
-
-// lv_out[v] = lv[rank[v]] (NB bytes per vertex, as 16-byte words)
-__global__ void k_ms_unrename(const uint4 *lv, uint32_t words_per_vertex, uint32_t n,
-                              const uint32_t *rank, uint4 *lv_out) {
-  const uint64_t total = (uint64_t)n * words_per_vertex;
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < total;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t v = i / words_per_vertex, k = i % words_per_vertex;
-    lv_out[i] = lv[(uint64_t)rank[v] * words_per_vertex + k];
-  }
 }
 
 // sum of out-degree of the distinct sources (the first level's frontier edges)
@@ -611,6 +723,7 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
   ensure(ctx->ms_hubs, sizeof(uint32_t) * (n + 1), ctx);
   const size_t act_words = n / 32 + 2;
   ensure(ctx->ms_act, sizeof(uint32_t) * 2 * act_words, ctx);
+  ensure(ctx->ms_part, sizeof(MsPart) * MS_PARTS, ctx);
   ensure(ctx->scratch, 64, ctx);
   uint32_t *seen = ctx->ms_seen.as<uint32_t>();
   uint32_t *buf[2] = {ctx->ms_cur.as<uint32_t>(), ctx->ms_nxt.as<uint32_t>()};
@@ -654,7 +767,8 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
     BFSX_HIP(hipMemcpyAsync(&n_phubs, d_np, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   }
   BFSX_HIP(hipGetLastError());
-  BFSX_HIP(hipStreamSynchronize(s));
+  ctx->seq_known = false;
+  read_ctl(ctx);  // (its level-end counter; synchronises: n_phubs is there too)
 
   // K device-driven levels, captured once per shape
   const uint32_t K = ctx->params.ms_graph_levels;
@@ -667,7 +781,8 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
                      (uint64_t)(uintptr_t)buf[0], (uint64_t)(uintptr_t)buf[1],
                      (uint64_t)(uintptr_t)lv, (uint64_t)(uintptr_t)act[0],
                      (uint64_t)(uintptr_t)ctx->ms_hubs.p, (uint64_t)(uintptr_t)ctx->ms_phubs.p,
-                     (uint64_t)(uintptr_t)ctx->queue[0].p, (uint64_t)(uintptr_t)ctx->queue[1].p})
+                     (uint64_t)(uintptr_t)ctx->queue[0].p, (uint64_t)(uintptr_t)ctx->queue[1].p,
+                     (uint64_t)(uintptr_t)ctx->ms_part.p})
     key = (key ^ v) * 1099511628211ull;
   if (!ctx->ms_exec || ctx->ms_key != key) {
     ms_drop_loop(ctx);
@@ -687,18 +802,17 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
         a.lv = lv;
         a.qi = p;
         a.q_in = ctx->queue[p].as<uint32_t>();
-        a.q_out = ctx->queue[p ^ 1].as<uint32_t>();
-        a.q_count_out = &ctl->q_count[p ^ 1];
-        a.q_edges_out = &ctl->q_edges[p ^ 1];
+        a.part = ctx->ms_part.as<MsPart>();
         a.overflow = &ctl->overflow;
         a.pull_hub = pull_hub;
         a.ctl = ctl;
         a.act_cur = act[p ^ 1];
         a.act_next = act[p];
-        hipLaunchKernelGGL(k_ms_begin, dim3(1), dim3(64), 0, s, ctl, p, (uint64_t)ctx->nnz,
-                           ctx->params.ms_push_divisor, symmetric ? 1 : 0);
-        hipLaunchKernelGGL(k_ms_clear, dim3(cap), dim3(256), 0, s, (const LevelCtl *)ctl, act[p],
-                           act_words, buf[p ^ 1], (size_t)(n * W));
+        hipLaunchKernelGGL(k_ms_begin, dim3(1), dim3(MS_PARTS), 0, s, ctl, p, (uint64_t)ctx->nnz,
+                           ctx->params.ms_push_divisor, symmetric ? 1 : 0, a.part);
+        hipLaunchKernelGGL(k_ms_clear, dim3(ms_grid(n * W, 1024, cap)), dim3(256), 0, s, ctl,
+                           (const uint32_t *)act[p ^ 1], act[p], act_words, buf[p ^ 1],
+                           (size_t)(n * W), ctx->queue[p].as<uint32_t>());
         hipLaunchKernelGGL((k_ms_push<PtrT, W>), dim3(cap), dim3(256), 0, s, a,
                            ctx->ms_hubs.as<uint32_t>());
         hipLaunchKernelGGL((k_ms_push_hubs<PtrT, W>), dim3(cap), dim3(256), 0, s, a,
@@ -712,7 +826,8 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
             hipLaunchKernelGGL((k_ms_pull_hubs<PtrT, W>), dim3(n_phubs), dim3(256), 0, s, a,
                                (const uint32_t *)ctx->ms_phubs.as<uint32_t>());
         }
-        hipLaunchKernelGGL(k_ms_end, dim3(1), dim3(64), 0, s, ctl, p, ctx->d_mirror);
+        hipLaunchKernelGGL(k_ms_end, dim3(1), dim3(MS_PARTS), 0, s, ctl, p,
+                           (const MsPart *)a.part, ctx->d_mirror);
       }
     } catch (...) {
       hipGraph_t g = nullptr;
@@ -725,12 +840,9 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
     ctx->ms_key = key;
   }
 
-  ctx->seq_known = false;
   // the timed level loop: one graph launch per K levels, the termination
   // flag read from the tagged level-end words
   MsResult r;
-  BFSX_HIP(hipMemcpyAsync(ctx->h_ctl, ctl, sizeof(LevelCtl), hipMemcpyDeviceToHost, s));
-  BFSX_HIP(hipStreamSynchronize(s));
   uint32_t seq = ctx->h_ctl->seq;
   BFSX_HIP(hipEventRecord(ctx->ev0, s));
   const uint64_t max_launches = n / K + 4;  // a search has at most n levels
@@ -746,39 +858,30 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
   float ms = 0;
   BFSX_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   r.ms = ms;
-  BFSX_HIP(hipMemcpyAsync(ctx->h_ctl, ctl, sizeof(LevelCtl), hipMemcpyDeviceToHost, s));
-  BFSX_HIP(hipStreamSynchronize(s));
+  // edges summed over searches
+  unsigned long long *d_e = ctx->scratch.as<unsigned long long>();
+  BFSX_HIP(hipMemsetAsync(d_e, 0, sizeof(unsigned long long), s));
+  hipLaunchKernelGGL((k_ms_edges<PtrT, W>), dim3(ms_grid(ctx->n_rows, 256, (unsigned)ctx->cu_count * 2)),
+                     dim3(256), 0, s, gcp, seen, ctx->n_rows, n_bits, d_e);
+  unsigned long long edges = 0;
+  BFSX_HIP(hipMemcpyAsync(&edges, d_e, sizeof(edges), hipMemcpyDeviceToHost, s));
+  read_ctl(ctx);  // (synchronises)
   if (ctx->h_ctl->overflow) fail(BFSX_ERR_OVERFLOW, "a level above 254 does not fit uint8 levels");
   r.push_levels = ctx->h_ctl->kind_count[0];
   r.pull_levels = ctx->h_ctl->kind_count[1];
   r.n_levels = r.push_levels + r.pull_levels;
-
-  // edges summed over searches, then the per-search level rows
-  unsigned long long *d_e = ctx->scratch.as<unsigned long long>();
-  BFSX_HIP(hipMemsetAsync(d_e, 0, sizeof(unsigned long long), s));
-  hipLaunchKernelGGL((k_ms_edges<PtrT, W>), dim3(ms_grid(ctx->n_rows, 256, cap)), dim3(256), 0, s,
-                     gcp, seen, ctx->n_rows, n_bits, d_e);
-  unsigned long long edges = 0;
-  BFSX_HIP(hipMemcpyAsync(&edges, d_e, sizeof(edges), hipMemcpyDeviceToHost, s));
-  BFSX_HIP(hipStreamSynchronize(s));
   r.edges = edges;
-  if (levels_out) {
-    DevBuf out, plain;
-    const uint8_t *rows = lv;
-    if (G.rank) {  // back to the caller's vertex ids
-      ensure(plain, (size_t)n * NB, ctx);
-      hipLaunchKernelGGL(k_ms_unrename, dim3(ms_grid(n * (NB / 16), 256, cap)), dim3(256), 0, s,
-                         reinterpret_cast<const uint4 *>(lv), NB / 16, (uint32_t)n, G.rank,
-                         plain.as<uint4>());
-      rows = plain.as<uint8_t>();
-    }
+  if (levels_out) {  // the per-search level rows, in the caller's vertex ids
+    DevBuf out;
+    struct Releaser {
+      DevBuf &b;
+      ~Releaser() { release(b); }
+    } releaser{out};
     ensure(out, (size_t)n_bits * n, ctx);
-    hipLaunchKernelGGL(k_ms_transpose, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, rows, NB,
-                       n_bits, (uint32_t)n, out.as<uint8_t>());
+    hipLaunchKernelGGL((k_ms_transpose<W>), dim3((unsigned)((n + MS_TV - 1) / MS_TV)), dim3(256), 0,
+                       s, lv, n_bits, (uint32_t)n, G.rank, n % 4 == 0 ? 1 : 0, out.as<uint8_t>());
     BFSX_HIP(hipGetLastError());
     copy_out(ctx, levels_out, out.p, (size_t)n_bits * n);
-    release(out);
-    release(plain);
   }
   return r;
 }

@@ -338,3 +338,31 @@ def test_bottom_up_short_lists(engine, n, ptr):
         for t in engine.last_trace():
             lo = int(deg[later(t["level"] + 1)].sum()) + int((want == t["level"] + 1).sum())
             assert lo <= t["pull_scanned"] <= int(deg[later(t["level"])].sum())
+
+
+# batches: level rows of any length (128 vertices per group, four per word),
+# every bitset width, lists beyond 256 edges shared by waves, active vertices
+# listed again after bottom-up levels, more vertices than the totals have parts
+@pytest.mark.parametrize("n", [1, 2, 5, 127, 128, 129, 4099, 70002])
+@pytest.mark.parametrize("n_bits", [1, 33, 128, 250])
+def test_batch_edges(engine, n, n_bits):
+    say("batch", n, n_bits)
+    rng = np.random.default_rng(n + n_bits)
+    m = 3 * n
+    src = (rng.random(m) ** 3 * n).astype(np.int64)
+    dst = rng.integers(0, n, m)
+    for sym in (True, False):
+        cp, ri = csc_from_edges(n, *(symmetrize(src, dst) if sym else (src, dst)))
+        n_rows = n if sym else n - n // 10
+        engine.upload_csc(cp, ri, n_rows=n_rows, symmetric=sym)
+        sources = rng.integers(0, n, n_bits + 3)
+        bits = np.concatenate([np.arange(n_bits), rng.integers(0, n_bits, 3)])
+        want = cpu.msbfs_u8(cp, ri, sources, bits, n_bits, n_rows=n_rows)
+        deg = np.diff(cp.astype(np.int64))[:n_rows]
+        ec = int(((want[:, :n_rows] != 0xFF) * deg).sum())
+        before = engine.params
+        for kw in ({}, {"ms_relabel": 0, "ms_push_divisor": 1}, {"ms_push_divisor": 1024}):
+            engine.set_params(**kw)
+            lev, st = engine.run_multi(sources, bits, n_bits)
+            engine.set_params(**before)
+            assert (lev == want).all() and st["edges_count"] == ec, kw
