@@ -1509,7 +1509,7 @@ __device__ __forceinline__ void scan_rest(const KArgs &a, const uint32_t *fbm_cu
 
 // Bottom-up step over plain lists (without the hub-first copy and its
 // first-neighbour array; k_pull2 below is the step with them).  A wave owns
-// 2048-vertex chunks (grid-stride): lane l
+// 2048-vertex chunks (grid-stride), or 1 / 2^cut of one: lane l
 // reads visited word l of the chunk (one coalesced load) and holds its
 // unvisited bits.  The unvisited vertices are then checked 64 at a time,
 // one per lane: a wave prefix sum of the per-word counts and a shuffle
@@ -1525,7 +1525,7 @@ template <typename PtrT, int WG, bool SUM>
 __global__ __launch_bounds__(WG) void k_pull(KArgs a, const uint32_t *fbm_cur,
                                              uint32_t *fbm_next, const uint32_t *g_sum,
                                              uint32_t sum_words, uint32_t shift,
-                                             SpecGuard guard) {
+                                             uint32_t cut, SpecGuard guard) {
   if (guard.skip()) return;
   constexpr int NW = WG / 64;
   extern __shared__ uint32_t s_sum_mem[];  // sum_words entries when g_sum is set
@@ -1544,11 +1544,13 @@ __global__ __launch_bounds__(WG) void k_pull(KArgs a, const uint32_t *fbm_cur,
   uint32_t n_found = 0;
   unsigned long long found_deg = 0, scanned = 0;
   uint32_t *fw = s_found[wv];
-  for (uint32_t c = blockIdx.x * NW + wv; c < n_chunks; c += gridDim.x * NW) {
+  for (uint32_t i = blockIdx.x * NW + wv; i < n_chunks << cut; i += gridDim.x * NW) {
+    const uint32_t c = i >> cut;
+    const bool own = lane >> (6 - cut) == (i & ((1u << cut) - 1));  // this wave's words
     const uint32_t wi = c * 64 + lane;
     const uint32_t vbase = wi * 32;
     const uint32_t vword = wi < n_words ? a.vis[wi] : ~0u;
-    uint32_t cm = ~vword;
+    uint32_t cm = own ? ~vword : 0u;
     if (vbase >= a.n_rows) cm = 0;
     else if (a.n_rows - vbase < 32) cm &= (1u << (a.n_rows - vbase)) - 1u;
     const uint32_t cnt = __popc(cm);
@@ -1601,7 +1603,7 @@ __global__ __launch_bounds__(WG) void k_pull(KArgs a, const uint32_t *fbm_cur,
     }
     wave_sync_lds();
     const uint32_t f = fw[lane];
-    if (wi < n_words) {
+    if (own && wi < n_words) {
       fbm_next[wi] = f;
       if (f) a.vis[wi] = vword | f;
     }
@@ -1647,7 +1649,9 @@ __global__ __launch_bounds__(WG) void k_pull(KArgs a, const uint32_t *fbm_cur,
 // R-MAT 26's second levels took 510 and 360 us, now 430 and 330.
 // Separating them keeps the short rounds of phase 1 from waiting for the
 // long chain (col_ptr, list line, probes) of a few undecided lanes.
-// Otherwise as k_pull: found vertices set bits in 64 LDS words the wave then
+// Otherwise as k_pull (a wave of a graph with few chunks takes a cut of one:
+// the candidates of its own words, ranked among the whole chunk's vertices):
+// found vertices set bits in 64 LDS words the wave then
 // writes as the next frontier bitmap and ORs into the visited bitmap; sizes
 // and degree sums leave with one atomic per work-group.
 template <typename PtrT, int WG, bool SUM>
@@ -1657,7 +1661,8 @@ __global__ __launch_bounds__(WG) void k_pull2(KArgs a, const uint32_t *fbm_cur,
                                               const uint32_t *fd, const uint16_t *fdd,
                                               const uint4 *fn, const uint32_t *iso,
                                               const uint32_t *crank, const uint32_t *hbm,
-                                              const uint32_t *hub, SpecGuard guard) {
+                                              const uint32_t *hub, uint32_t cut,
+                                              SpecGuard guard) {
   if (guard.skip()) return;
   constexpr int NW = WG / 64;
   constexpr int S1 = 2 * PULL_SLOTS;  // phase-1 candidates per lane per round
@@ -1679,11 +1684,13 @@ __global__ __launch_bounds__(WG) void k_pull2(KArgs a, const uint32_t *fbm_cur,
   unsigned long long found_deg = 0, scanned = 0;
   uint32_t *fw = s_found[wv];
   uint32_t *uw = s_undec[wv];
-  for (uint32_t c = blockIdx.x * NW + wv; c < n_chunks; c += gridDim.x * NW) {
+  for (uint32_t i = blockIdx.x * NW + wv; i < n_chunks << cut; i += gridDim.x * NW) {
+    const uint32_t c = i >> cut;
+    const bool own = lane >> (6 - cut) == (i & ((1u << cut) - 1));  // this wave's words
     const uint32_t wi = c * 64 + lane;
     const uint32_t vbase = wi * 32;
     const uint32_t vword = wi < n_words ? a.vis[wi] : ~0u;
-    uint32_t cm = ~vword;
+    uint32_t cm = own ? ~vword : 0u;
     uint32_t lw = wi < n_words ? ~iso[wi] : 0u;  // vertices with neighbours
     if (vbase >= a.n_rows) {
       cm = 0;
@@ -1824,7 +1831,7 @@ __global__ __launch_bounds__(WG) void k_pull2(KArgs a, const uint32_t *fbm_cur,
     }
     wave_sync_lds();
     const uint32_t f = fw[lane];
-    if (wi < n_words) {
+    if (own && wi < n_words) {
       fbm_next[wi] = f;
       if (f) a.vis[wi] = vword | f;
     }
@@ -2902,23 +2909,30 @@ static void launch_pull(unsigned grid, size_t lds, hipStream_t st, const KArgs &
                         uint32_t shift, const uint32_t *fd, const uint16_t *fdd,
                         const uint4 *fn, const uint32_t *iso,
                         const uint32_t *crank, const uint32_t *hbm, const uint32_t *hub,
-                        SpecGuard guard) {
+                        uint32_t cut, SpecGuard guard) {
   if (fd) {
     if (g_sum)
       hipLaunchKernelGGL((k_pull2<PtrT, WG, true>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
-                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard);
+                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, cut, guard);
     else
       hipLaunchKernelGGL((k_pull2<PtrT, WG, false>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
-                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard);
+                         s.fbm_next, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, cut, guard);
   } else {
     if (g_sum)
       hipLaunchKernelGGL((k_pull<PtrT, WG, true>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
-                         s.fbm_next, g_sum, sum_words, shift, guard);
+                         s.fbm_next, g_sum, sum_words, shift, cut, guard);
     else
       hipLaunchKernelGGL((k_pull<PtrT, WG, false>), dim3(grid), dim3(WG), lds, st, a, s.fbm_cur,
-                         s.fbm_next, g_sum, sum_words, shift, guard);
+                         s.fbm_next, g_sum, sum_words, shift, cut, guard);
   }
 }
+
+// The cut of a bottom-up step's chunks: with whole chunks, R-MAT 19 has 256
+// waves for 256 CUs and one long list holds 1/256 of the step.  Four waves per
+// CU, learned, level loop per search: R-MAT 16 124 -> 98 us, 19 138 -> 115, 20
+// 167 -> 135, 22 208 -> 191; eight or more per CU gain less there (every
+// work-group adds its totals to the same counters, 12 ns an addition).
+constexpr uint32_t PULL_MAX_CUT = 5, PULL_WAVES_PER_CU = 4;
 
 template <typename PtrT>
 static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
@@ -2955,7 +2969,12 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   uint32_t per_cu = 32 / nw;
   const uint32_t by_lds = ctx->lds_per_cu / (uint32_t)(static_lds + lds);
   per_cu = by_lds < per_cu ? (by_lds ? by_lds : 1) : per_cu;
-  const unsigned grid = cap_grid(((uint64_t)n_chunks + nw - 1) / nw,
+  // Waves take whole chunks of 2048 vertices where those fill the card, and
+  // halves down to 1/32 (two bitmap words) of one on smaller graphs.
+  uint32_t cut = 0;
+  while (cut < PULL_MAX_CUT && ((uint64_t)n_chunks << cut) < (uint64_t)ctx->cu_count * PULL_WAVES_PER_CU)
+    cut++;
+  const unsigned grid = cap_grid((((uint64_t)n_chunks << cut) + nw - 1) / nw,
                                  (unsigned)ctx->cu_count * per_cu);
   // the {first neighbour, degree} array belongs to the hub-first copy
   const uint32_t *fd = ctx->pull_fd.p && s.row_idx == ctx->row_idx_pull.as<uint32_t>()
@@ -2980,10 +2999,10 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   }
   KernelTimer kt(s, st);
   switch (wg) {
-    case 64: launch_pull<PtrT, 64>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
-    case 128: launch_pull<PtrT, 128>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
-    case 256: launch_pull<PtrT, 256>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
-    case 512: launch_pull<PtrT, 512>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, guard); break;
+    case 64: launch_pull<PtrT, 64>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, cut, guard); break;
+    case 128: launch_pull<PtrT, 128>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, cut, guard); break;
+    case 256: launch_pull<PtrT, 256>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, cut, guard); break;
+    case 512: launch_pull<PtrT, 512>(grid, lds, st, a, s, g_sum, sum_words, shift, fd, fdd, fn, iso, crank, hbm, hub, cut, guard); break;
     default: fail(BFSX_ERR_ARG, "pull_wg must be 64, 128, 256 or 512");
   }
 }

@@ -346,7 +346,13 @@ struct Walker {
     // bucketed GLB from n_cols/256 frontier edges on (below that its fixed
     // cost, about a pass over the visited bitmap, exceeds exact-once's
     // atomics) or wherever a marking step would run
-    a.bucket_ok = br != 0xFFFFFFFFu && (double)UE * 1024.0 >= (double)ctx->nnz * br &&
+    // and on graphs of more than 2^22 vertices: a slice of 2^16 is one
+    // work-group of the apply kernel, and up to 64 of them leave the card idle
+    // (fixed GLB bucketed / not, R-MAT 16 275 / 178 us, 19 358 / 248, 21 665 /
+    // 591, 22 1143 / 1140, 23 2008 / 2175, 24 4018 / 4565; learned R-MAT 20
+    // 177 / 152, 22 209 / 191, 23 258 / 301)
+    a.bucket_ok = br != 0xFFFFFFFFu && (br == 0 || ctx->n_cols > (1u << 22)) &&
+                  (double)UE * 1024.0 >= (double)ctx->nnz * br &&
                   (use_mark || EF * 256 >= ctx->n_cols) && mr.lo_E != ~0ull;
     a.mark = use_mark ? ctx->mark.as<uint8_t>() : nullptr;
     // Where many edges lead to each new vertex and the marks do not stay in

@@ -366,3 +366,37 @@ def test_batch_edges(engine, n, n_bits):
             lev, st = engine.run_multi(sources, bits, n_bits)
             engine.set_params(**before)
             assert (lev == want).all() and st["edges_count"] == ec, kw
+
+
+# small graphs: waves of the bottom-up step take down to two bitmap words of a
+# chunk, with and without the hub-first copy; GLB marks up to 2^22 vertices and
+# buckets beyond or when asked to
+@pytest.mark.parametrize("n", [40, 65, 2050, 33000, 300001])
+@pytest.mark.parametrize("order", ["", "pull_hub_first"])
+def test_small_graph_steps(engine, n, order):
+    say("small graphs", n, order)
+    rng = np.random.default_rng(n)
+    src = (rng.random(4 * n) ** 2 * n).astype(np.int64)
+    dst = rng.integers(0, n - n // 8, 4 * n)
+    cp, ri = csc_from_edges(n, *symmetrize(src, dst))
+    engine.upload_csc(cp, ri, symmetric=True)
+    if order:
+        engine.order_adjacency(order)
+    engine.load_scheduler()
+    before = engine.params
+    try:
+        for root in rng.choice(src, 3):
+            want, ec, _ = cpu.bfs_queue(cp, ri, int(root))
+            for wg in (64, 512):
+                engine.set_params(pull_wg=wg)
+                lev, st, par = engine.run(int(root), "pull", parents=True)
+                assert (lev == want).all() and st["edges_count"] == ec
+                assert cpu.check_parents(cp, ri, int(root), want, par) == 0
+                assert (engine.run(int(root), "learned")[0] == want).all()
+            for ratio in (0, 512):
+                engine.set_params(bucket_ratio_q10=ratio)
+                assert (engine.run(int(root), "glb")[0] == want).all()
+            engine.set_params(**before)
+    finally:
+        engine.set_params(**before)
+        engine.set_scheduler_weights(None)
