@@ -489,19 +489,19 @@ struct DevStep {
 };
 
 static_assert(offsetof(LevelCtl, q_count) == 0 && offsetof(LevelCtl, level) == 8 &&
-                  offsetof(LevelCtl, q_edges) == 16 && alignof(LevelCtl) >= 8,
-              "k_td_dev reads the control block's first 32 bytes as two uint4");
+                  offsetof(LevelCtl, q_edges) == 128 && alignof(LevelCtl) >= 8,
+              "k_td_dev reads the counts and the edge sums as a uint4 each");
 
 template <typename PtrT, int WG>
 __global__ __launch_bounds__(WG) void k_td_dev(KArgs a, LevelCtl *ctl, DevStep d) {
   __shared__ LlbShared<PtrT, WG> sh;
-  // The control block's fields (its first 32 bytes, counts, level and
-  // edges, as two 16-byte loads, and the choice) and this group's first LLB
+  // The control block's fields (counts and level, and edges, as two 16-byte
+  // loads, and the choice) and this group's first LLB
   // tile of the queue in one round trip: the queue holds n_cols + 1
   // entries, so the read is in bounds whatever F is; entries past F are not
   // used.
   const uint4 h0 = reinterpret_cast<const uint4 *>(ctl)[0];
-  const uint4 h1 = reinterpret_cast<const uint4 *>(ctl)[1];
+  const uint4 h1 = reinterpret_cast<const uint4 *>(ctl)[8];
   const uint32_t c_choice = ctl->choice;
   const uint32_t idx0 = blockIdx.x * WG + threadIdx.x;
   const uint32_t v0 = idx0 < a.n_cols ? a.q_in[idx0] : 0u;
