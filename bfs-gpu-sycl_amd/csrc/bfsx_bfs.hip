@@ -104,20 +104,26 @@ __device__ __forceinline__ void wave_append(bool isnew, uint32_t n, uint32_t *q_
   if (isnew) q_out[base + lanes_below(m)] = n;
 }
 
-// Adds a per-thread value over the work-group to *dst with one atomic.
-// Every thread of the group must call it.
+// Sum of a per-thread value over the work-group, in thread 0.  Every thread
+// of the group must call it.
 template <int WG>
-__device__ __forceinline__ void block_atomic_add(unsigned long long v, unsigned long long *dst) {
+__device__ __forceinline__ unsigned long long block_sum(unsigned long long v) {
   __shared__ unsigned long long s_part[WG / 64];
   v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
+  unsigned long long t = 0;
+  if (threadIdx.x == 0)
     for (int w = 0; w < WG / 64; w++) t += s_part[w];
-    if (t) atomicAdd(dst, t);
-  }
+  return t;
+}
+
+// Adds it to *dst with one atomic.
+template <int WG>
+__device__ __forceinline__ void block_atomic_add(unsigned long long v, unsigned long long *dst) {
+  const unsigned long long t = block_sum<WG>(v);
+  if (threadIdx.x == 0 && t) atomicAdd(dst, t);
 }
 
 // Out-degree of vertex v (v below the padded bitmap length) from the 16-bit
@@ -478,56 +484,12 @@ __global__ __launch_bounds__(WG) void k_llb(KArgs a, uint32_t n_tiles, uint32_t 
   if (a.q_out_edges && !a.mark) block_atomic_add<WG>(dacc, a.q_out_edges);
 }
 
-// Device-driven top-down step for captured level loops: the frontier size,
-// level, discovery mode and LLB/SLB choice come from the control block, and
-// a fixed grid walks the tiles.  Kernels after the search ended see F = 0.
+// A device-driven top-down step (k_td_dev).
 struct DevStep {
   uint32_t cur;                  // queue buffer holding the frontier
   int fixed;                     // BFSX_LLB or BFSX_SLB, or -1: read ctl->choice
   MarkRule mark;                 // which frontiers mark + compact
-  int spec;                      // speculative: skip the frontiers `mark` marks
 };
-
-static_assert(offsetof(LevelCtl, q_count) == 0 && offsetof(LevelCtl, level) == 8 &&
-                  offsetof(LevelCtl, q_edges) == 128 && alignof(LevelCtl) >= 8,
-              "k_td_dev reads the counts and the edge sums as a uint4 each");
-
-template <typename PtrT, int WG>
-__global__ __launch_bounds__(WG) void k_td_dev(KArgs a, LevelCtl *ctl, DevStep d) {
-  __shared__ LlbShared<PtrT, WG> sh;
-  // The control block's fields (counts and level, and edges, as two 16-byte
-  // loads, and the choice) and this group's first LLB
-  // tile of the queue in one round trip: the queue holds n_cols + 1
-  // entries, so the read is in bounds whatever F is; entries past F are not
-  // used.
-  const uint4 h0 = reinterpret_cast<const uint4 *>(ctl)[0];
-  const uint4 h1 = reinterpret_cast<const uint4 *>(ctl)[8];
-  const uint32_t c_choice = ctl->choice;
-  const uint32_t idx0 = blockIdx.x * WG + threadIdx.x;
-  const uint32_t v0 = idx0 < a.n_cols ? a.q_in[idx0] : 0u;
-  const uint32_t F = d.cur ? h0.y : h0.x;
-  const unsigned long long c_edges =
-      d.cur ? ((unsigned long long)h1.w << 32 | h1.z) : ((unsigned long long)h1.y << 32 | h1.x);
-  const int choice = d.fixed >= 0 ? d.fixed : (int)c_choice;
-  const bool marks = d.mark.marks(c_edges, F);
-  // one branch on all of them, so that no read waits for another's test
-  const bool run = (F != 0) & ((choice == BFSX_LLB) | (choice == BFSX_SLB)) &
-                   !(marks & (d.spec != 0));
-  if (!run) return;
-  a.F = F;
-  a.next_level = (int32_t)h0.z + 1;
-  if (!marks) a.mark = nullptr;
-  const uint32_t n_tiles = (F + WG - 1) / WG;
-  const uint32_t n_parts = llb_parts(c_edges, n_tiles, WG);
-  const bool llb = choice == BFSX_LLB;
-  unsigned long long dacc = 0;
-  for (uint64_t i = blockIdx.x; i < (uint64_t)n_tiles * n_parts; i += gridDim.x) {
-    const uint32_t tile = (uint32_t)(i % n_tiles);
-    llb_tile<PtrT, WG>(a, sh, tile, n_tiles, !llb, dacc, (uint32_t)(i / n_tiles), n_parts,
-                       llb && tile == blockIdx.x, v0);
-  }
-  if (a.q_out_edges && !a.mark) block_atomic_add<WG>(dacc, a.q_out_edges);
-}
 
 // ---------------------------------------------------------------------------
 // GLB: tile scan -> tile-offset scan -> global offsets + chunk table -> expand
@@ -1326,15 +1288,11 @@ struct SpecGuard {
   const LevelCtl *ctl;  // null: not speculative
   uint32_t consumed;    // the queue counter of the level's frontier
   uint32_t kinds;       // bit k: runs if the decision is kind k
-  MarkRule heavy;       // and if this rule does not mark the frontier
   __device__ __forceinline__ bool skip() const {
     if (!ctl) return false;
-    const uint32_t F = ctl->q_count[consumed];
-    return !((kinds >> (ctl->choice & 31u)) & 1u) || F == 0 ||
-           heavy.marks(ctl->q_edges[consumed], F);
+    return !((kinds >> (ctl->choice & 31u)) & 1u) || ctl->q_count[consumed] == 0;
   }
 };
-constexpr MarkRule NEVER_MARKS{~0ull, ~0ull};  // (frontier edges stay below 2^48)
 
 // hbm bit h = frontier bit of hub[h] (H a multiple of 64, and so is the
 // grid-stride: every wave runs whole rounds).
@@ -2116,11 +2074,9 @@ __device__ __forceinline__ bool level_end_body(LevelCtl *ctl, uint32_t consumed,
                    kc2 = ctl->kind_count[2], kc3 = ctl->kind_count[3];
     const uint32_t f0 = ctl->dec_F, d_pull = ctl->dec_pull, d_valid = ctl->dec_valid;
     const unsigned long long e0 = ctl->dec_EF;
-    const unsigned long long ec = ctl->q_edges[consumed];
     const uint32_t seq0 = ctl->seq;
     // a speculative launch whose guess failed changes nothing
-    const bool skip = guard.ctl && (!((guard.kinds >> (choice & 31u)) & 1u) || fc == 0 ||
-                                    guard.heavy.marks(ec, fc));
+    const bool skip = guard.ctl && (!((guard.kinds >> (choice & 31u)) & 1u) || fc == 0);
     s_skip = skip;
     s_live = 0;
     if (skip) {
@@ -2235,6 +2191,94 @@ __global__ __launch_bounds__(64) void k_level_end(LevelCtl *ctl, uint32_t consum
   if (mirror && threadIdx.x == 0) put_level_end(ctl, words, mirror);
 }
 
+// Device-driven top-down step: the frontier size, level, discovery mode and
+// LLB/SLB choice come from the control block, and a fixed grid walks the
+// tiles.  In captured level loops (SPEC false) k_compact_dev and k_level_end
+// follow it; kernels after the search ended see F = 0.
+//
+// SPEC: launched ahead of the decision for its level; it skips the frontiers
+// that d.mark marks, and ends the level itself.  Every group that had a tile
+// counts itself in the upper bits of its addition to the edge sum; the one
+// that the sum shows to be the last makes the level's end as k_level_end
+// does, without that kernel's start and drain and its gap behind this one:
+// learned searches of a 1024^2 grid 3330 -> 3150 us (296 levels), of a
+// 4096^2 one 7255 -> 6985 (351); of R-MATs, with a few such levels, the same.
+// The last group's sums are whole: a group's additions to the queue count
+// returned before it added to the edge sum.  A group without a tile only
+// reads the control block, whichever of its states it sees: before the end
+// its index is not below the tile count, after it the count is 0 (and a
+// mixture has fewer tiles, the edge sum being 0).
+struct TdEnd {
+  const float *Wg;  // scheduler weights
+  uint64_t n_cols, nnz, n_iso;
+  uint32_t allow;   // kinds the scheduler may pick
+  int reuse;
+  LevelMirror *mirror;
+};
+constexpr int TD_SUM_BITS = 48;  // (edge sums stay below 2^48, groups below 2^16)
+
+static_assert(offsetof(LevelCtl, q_count) == 0 && offsetof(LevelCtl, level) == 8 &&
+                  offsetof(LevelCtl, q_edges) == 128 && alignof(LevelCtl) >= 8,
+              "k_td_dev reads the counts and the edge sums as a uint4 each");
+
+template <typename PtrT, int WG, bool SPEC>
+__global__ __launch_bounds__(WG) void k_td_dev(KArgs a, LevelCtl *ctl, DevStep d, TdEnd e) {
+  __shared__ LlbShared<PtrT, WG> sh;
+  // The control block's fields (counts and level, and edges, as two 16-byte
+  // loads, and the choice) and this group's first LLB
+  // tile of the queue in one round trip: the queue holds n_cols + 1
+  // entries, so the read is in bounds whatever F is; entries past F are not
+  // used.
+  const uint4 h0 = reinterpret_cast<const uint4 *>(ctl)[0];
+  const uint4 h1 = reinterpret_cast<const uint4 *>(ctl)[8];
+  const uint32_t c_choice = ctl->choice;
+  const uint32_t idx0 = blockIdx.x * WG + threadIdx.x;
+  const uint32_t v0 = idx0 < a.n_cols ? a.q_in[idx0] : 0u;
+  const uint32_t F = d.cur ? h0.y : h0.x;
+  const unsigned long long c_edges =
+      d.cur ? ((unsigned long long)h1.w << 32 | h1.z) : ((unsigned long long)h1.y << 32 | h1.x);
+  const int choice = d.fixed >= 0 ? d.fixed : (int)c_choice;
+  const bool marks = d.mark.marks(c_edges, F);
+  // one branch on all of them, so that no read waits for another's test
+  const bool run = (F != 0) & ((choice == BFSX_LLB) | (choice == BFSX_SLB)) & !(marks & SPEC);
+  if (!run) return;
+  a.F = F;
+  a.next_level = (int32_t)h0.z + 1;
+  if (!marks) a.mark = nullptr;
+  const uint32_t n_tiles = (F + WG - 1) / WG;
+  const uint32_t n_parts = llb_parts(c_edges, n_tiles, WG);
+  const uint64_t n_work = (uint64_t)n_tiles * n_parts;
+  if (SPEC && blockIdx.x >= n_work) return;
+  const bool llb = choice == BFSX_LLB;
+  unsigned long long dacc = 0;
+  for (uint64_t i = blockIdx.x; i < n_work; i += gridDim.x) {
+    const uint32_t tile = (uint32_t)(i % n_tiles);
+    llb_tile<PtrT, WG>(a, sh, tile, n_tiles, !llb, dacc, (uint32_t)(i / n_tiles), n_parts,
+                       llb && tile == blockIdx.x, v0);
+  }
+  if constexpr (!SPEC) {
+    if (a.q_out_edges && !a.mark) block_atomic_add<WG>(dacc, a.q_out_edges);
+  } else {
+    __shared__ int s_last;
+    const unsigned long long sum = block_sum<WG>(dacc);  // (in thread 0)
+    if (threadIdx.x == 0) {
+      constexpr unsigned long long ONE = 1ull << TD_SUM_BITS;
+      const uint32_t groups = n_work < gridDim.x ? (uint32_t)n_work : gridDim.x;
+      const unsigned long long now = atomicAdd(a.q_out_edges, sum + ONE) + sum + ONE;
+      s_last = (uint32_t)(now >> TD_SUM_BITS) == groups;
+      if (s_last) *a.q_out_edges = now & (ONE - 1);
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // the other groups' additions, not this XCD's copy of the block
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    LevelEndWords words;
+    level_end_body(ctl, d.cur, d.cur ^ 1u, 0, choice, e.Wg, e.n_cols, e.nnz, e.n_iso, e.allow,
+                   e.reuse, SpecGuard{nullptr, 0, 0}, &words);
+    if (threadIdx.x == 0) put_level_end(ctl, words, e.mirror);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // device loop: consecutive thin top-down levels in one cooperative launch
 // ---------------------------------------------------------------------------
@@ -2324,7 +2368,7 @@ __global__ __launch_bounds__(WG) void k_coop_levels(KArgs base, LevelCtl *ctl, C
     block_atomic_add<WG>(dacc, a.q_out_edges);
     grid_barrier_last(ctl, gridDim.x, [&] {
       level_end_body(ctl, cur, cur ^ 1, 0, choice, c.Wg, c.n_cols, c.nnz, c.n_iso, c.allow, 1,
-                     SpecGuard{nullptr, 0, 0, NEVER_MARKS});
+                     SpecGuard{nullptr, 0, 0});
     });
     cur ^= 1;
   }
@@ -2523,7 +2567,7 @@ __global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl,
       s_ctl.q_edges[cur ^ 1] = s_edges;
     }
     level_end_body(&s_ctl, cur, cur ^ 1, 0, (int)choice, c.Wg, c.n_cols, c.nnz, c.n_iso, c.allow,
-                   1, SpecGuard{nullptr, 0, 0, NEVER_MARKS}, nullptr, s_W4);
+                   1, SpecGuard{nullptr, 0, 0}, nullptr, s_W4);
     __syncthreads();
     prev_F = F;
     cur ^= 1;
@@ -2953,7 +2997,7 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   // (a speculative step does not know its frontier's size: no summary)
   const bool use_sum = !speculative && max_words >= 64 &&
                        ((uint64_t)s.F << shift) * 4 <= (uint64_t)s.n_cols;
-  const SpecGuard guard{speculative ? s.ctl : nullptr, s.q_in_idx, 1u << BFSX_PULL, NEVER_MARKS};
+  const SpecGuard guard{speculative ? s.ctl : nullptr, s.q_in_idx, 1u << BFSX_PULL};
   const uint32_t *g_sum = nullptr;
   if (use_sum) {
     ensure(ctx->fsum, sizeof(uint32_t) * PULL_SUM_WORDS_MAX, ctx);
@@ -3097,27 +3141,24 @@ void level_begin(bfsx_ctx *ctx) {
   BFSX_HIP(hipGetLastError());
 }
 
+// Isolated vertices, which the scheduler counts as visited.
+static uint64_t known_isolated(const bfsx_ctx *ctx) {
+  return (ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols ? ctx->n_isolated : 0;
+}
+
 void level_end(bfsx_ctx *ctx, uint32_t consumed, uint32_t produced, bool stamp, int kind,
-               uint32_t decide_allow, bool reuse, uint32_t spec_kinds,
-               const MarkRule *spec_heavy) {
-  const uint64_t n_iso = (ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols
-                             ? ctx->n_isolated
-                             : 0;
+               uint32_t decide_allow, bool reuse, uint32_t spec_kinds) {
   hipLaunchKernelGGL(k_level_end, dim3(1), dim3(64), 0, ctx->stream, ctx->ctl.as<LevelCtl>(),
                      consumed, produced, stamp ? 1 : 0, kind,
                      decide_allow ? ctx->sched_w.as<float>() : (const float *)nullptr,
-                     (uint64_t)ctx->n_cols, (uint64_t)ctx->nnz, n_iso, decide_allow,
+                     (uint64_t)ctx->n_cols, (uint64_t)ctx->nnz, known_isolated(ctx), decide_allow,
                      reuse ? 1 : 0, ctx->d_mirror,
-                     SpecGuard{spec_kinds ? ctx->ctl.as<LevelCtl>() : nullptr, consumed,
-                               spec_kinds, spec_heavy ? *spec_heavy : NEVER_MARKS});
+                     SpecGuard{spec_kinds ? ctx->ctl.as<LevelCtl>() : nullptr, consumed, spec_kinds});
   BFSX_HIP(hipGetLastError());
 }
 
-// One device-driven top-down level (LLB or SLB, or the choice in the control
-// block when fixed < 0) for a captured loop: step, compaction, bookkeeping.
-template <typename PtrT>
-static void dev_level_t(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, MarkRule mark,
-                        bool speculative) {
+template <typename PtrT, bool SPEC>
+static void launch_td(bfsx_ctx *ctx, uint32_t cur, const DevStep &d, const TdEnd &e, bool track) {
   KArgs a{};
   a.col_ptr = ctx->col_ptr.p;
   a.row_idx = ctx->row_idx.as<uint32_t>();
@@ -3133,24 +3174,30 @@ static void dev_level_t(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, Mark
   a.parents = nullptr;
   a.hub_degree = ctx->params.hub_degree;
   a.mark = ctx->mark.as<uint8_t>();
-  const DevStep d{cur, fixed, mark, speculative ? 1 : 0};
   const uint32_t wg = ctx->params.llb_wg;
-  const unsigned grid = cap_grid(((uint64_t)ctx->n_cols + wg - 1) / wg, (unsigned)ctx->cu_count * 8);
+  const unsigned max_groups = std::min((unsigned)ctx->cu_count * 8, 0xFFFFu);
+  const unsigned grid = cap_grid(((uint64_t)ctx->n_cols + wg - 1) / wg, max_groups);
   hipStream_t s = ctx->stream;
   switch (wg) {
-    case 64: hipLaunchKernelGGL((k_td_dev<PtrT, 64>), dim3(grid), dim3(64), 0, s, a, ctl, d); break;
-    case 128: hipLaunchKernelGGL((k_td_dev<PtrT, 128>), dim3(grid), dim3(128), 0, s, a, ctl, d); break;
-    case 256: hipLaunchKernelGGL((k_td_dev<PtrT, 256>), dim3(grid), dim3(256), 0, s, a, ctl, d); break;
-    case 512: hipLaunchKernelGGL((k_td_dev<PtrT, 512>), dim3(grid), dim3(512), 0, s, a, ctl, d); break;
-    case 1024: hipLaunchKernelGGL((k_td_dev<PtrT, 1024>), dim3(grid), dim3(1024), 0, s, a, ctl, d); break;
+    case 64: hipLaunchKernelGGL((k_td_dev<PtrT, 64, SPEC>), dim3(grid), dim3(64), 0, s, a, ctl, d, e); break;
+    case 128: hipLaunchKernelGGL((k_td_dev<PtrT, 128, SPEC>), dim3(grid), dim3(128), 0, s, a, ctl, d, e); break;
+    case 256: hipLaunchKernelGGL((k_td_dev<PtrT, 256, SPEC>), dim3(grid), dim3(256), 0, s, a, ctl, d, e); break;
+    case 512: hipLaunchKernelGGL((k_td_dev<PtrT, 512, SPEC>), dim3(grid), dim3(512), 0, s, a, ctl, d, e); break;
+    case 1024: hipLaunchKernelGGL((k_td_dev<PtrT, 1024, SPEC>), dim3(grid), dim3(1024), 0, s, a, ctl, d, e); break;
     default: fail(BFSX_ERR_ARG, "llb_wg must be 64, 128, 256, 512 or 1024");
   }
-  if (speculative) {  // (it never marks)
-    BFSX_HIP(hipGetLastError());
-    return;
-  }
+  BFSX_HIP(hipGetLastError());
+}
+
+// One device-driven top-down level (LLB or SLB, or the choice in the control
+// block when fixed < 0) for a captured loop: step, compaction.
+template <typename PtrT>
+static void dev_level_t(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, MarkRule mark) {
+  const DevStep d{cur, fixed, mark};
+  launch_td<PtrT, false>(ctx, cur, d, TdEnd{}, track);
+  LevelCtl *ctl = ctx->ctl.as<LevelCtl>();
   const CompactShape c = compact_shape(ctx, ctx->n_cols);
-  hipLaunchKernelGGL(k_compact_dev<PtrT>, dim3(c.grid), dim3(COMPACT_WG), 0, s,
+  hipLaunchKernelGGL(k_compact_dev<PtrT>, dim3(c.grid), dim3(COMPACT_WG), 0, ctx->stream,
                      static_cast<const PtrT *>(ctx->col_ptr.p), ctx->deg16.as<uint16_t>(),
                      ctx->n_rows,
                      ctx->mark.as<uint8_t>(), c.n_chunks, c.per_group, ctx->vis.as<uint32_t>(),
@@ -3159,10 +3206,17 @@ static void dev_level_t(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, Mark
   BFSX_HIP(hipGetLastError());
 }
 
-void dev_level(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, MarkRule mark,
-               bool speculative) {
-  if (ctx->ptr_bytes == 8) dev_level_t<uint64_t>(ctx, cur, fixed, track, mark, speculative);
-  else dev_level_t<uint32_t>(ctx, cur, fixed, track, mark, speculative);
+void dev_level(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, MarkRule mark) {
+  if (ctx->ptr_bytes == 8) dev_level_t<uint64_t>(ctx, cur, fixed, track, mark);
+  else dev_level_t<uint32_t>(ctx, cur, fixed, track, mark);
+}
+
+void spec_td_level(bfsx_ctx *ctx, uint32_t cur, MarkRule mark, uint32_t decide_allow, bool reuse) {
+  const DevStep d{cur, -1, mark};
+  const TdEnd e{ctx->sched_w.as<float>(), ctx->n_cols, ctx->nnz, known_isolated(ctx),
+                decide_allow, reuse ? 1 : 0, ctx->d_mirror};
+  if (ctx->ptr_bytes == 8) launch_td<uint64_t, true>(ctx, cur, d, e, true);
+  else launch_td<uint32_t, true>(ctx, cur, d, e, true);
 }
 
 template <typename PtrT, int WG>
@@ -3217,7 +3271,7 @@ bool coop_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool le
   c.Wg = learned ? ctx->sched_w.as<float>() : nullptr;
   c.n_cols = ctx->n_cols;
   c.nnz = ctx->nnz;
-  c.n_iso = (ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols ? ctx->n_isolated : 0;
+  c.n_iso = known_isolated(ctx);
   c.allow = allow;
   c.mirror = ctx->d_mirror;
   return ctx->ptr_bytes == 8 ? coop_levels_t<uint64_t>(ctx, a, c) : coop_levels_t<uint32_t>(ctx, a, c);
@@ -3243,7 +3297,7 @@ void solo_levels(bfsx_ctx *ctx, uint32_t cur, int fixed, uint32_t allow, bool le
   c.Wg = learned ? ctx->sched_w.as<float>() : nullptr;
   c.n_cols = ctx->n_cols;
   c.nnz = ctx->nnz;
-  c.n_iso = (ctx->gflags & BFSX_GRAPH_SYMMETRIC) && ctx->n_rows == ctx->n_cols ? ctx->n_isolated : 0;
+  c.n_iso = known_isolated(ctx);
   c.allow = allow;
   c.mirror = ctx->d_mirror;
   LevelCtl *ctl = ctx->ctl.as<LevelCtl>();

@@ -446,9 +446,7 @@ struct Walker {
   // level runs the host-sized step).  That kernel records no parents: not
   // with a parent array.
   void launch_speculative_td(const MarkRule &mr) {
-    dev_level(ctx, cur ^ 1, -1, true, mr, true);
-    level_end(ctx, cur ^ 1, cur, false, -1, decide_allow, decide_reuse,
-              (1u << BFSX_LLB) | (1u << BFSX_SLB), &mr);
+    spec_td_level(ctx, cur ^ 1, mr, decide_allow, decide_reuse);
   }
 
   // Host bookkeeping after the control block of the level has been read.

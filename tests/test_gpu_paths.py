@@ -400,3 +400,43 @@ def test_small_graph_steps(engine, n, order):
     finally:
         engine.set_params(**before)
         engine.set_scheduler_weights(None)
+
+
+# the last of a speculative step's groups ends the level: frontiers of one
+# group, of whole and ragged tiles, of more tiles than the grid has groups
+@pytest.mark.parametrize("width", [700, 4096, 4097, 20011, 140003])
+@pytest.mark.parametrize("kind", [0, 2])  # LLB, SLB
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+def test_level_end_by_last_group(engine, width, kind, ptr):
+    say("last group", width, kind, ptr.__name__)
+    rng = np.random.default_rng(width)
+    depth, n = 6, 1 + 6 * width
+    lay = 1 + width * np.arange(depth)
+    src, dst = [np.zeros(width, np.int64)], [lay[0] + np.arange(width)]
+    for i in range(depth - 1):
+        for _ in range(4):
+            src.append(lay[i] + rng.integers(0, width, width))
+            dst.append(lay[i + 1] + np.arange(width))
+    cp, ri = csc_from_edges(n, *symmetrize(np.concatenate(src), np.concatenate(dst)))
+    want, ec, _ = cpu.bfs_queue(cp, ri, 0)
+    engine.upload_csc(cp.astype(ptr), ri, symmetric=True)
+    w = np.zeros(1476, np.float32)
+    w[-4:] = 1
+    w[-4 + kind] = 0  # constant outputs, the smallest one's kind is taken
+    before = engine.params
+    try:
+        engine.set_scheduler_weights(w)
+        for wg in (64, 256, 1024):
+            for hub in (0, 6):
+                engine.set_params(llb_wg=wg, hub_degree=hub, mark_ratio_q10=0xFFFFFFFF)
+                for spec in (1, 0, 1):
+                    engine.set_params(speculate=spec)
+                    lev, st = engine.run(0, "learned")
+                    assert np.array_equal(lev, want), (wg, hub, spec)
+                    assert st["edges_count"] == ec and st["reached"] == n
+                    assert st["n_levels"] == depth + 1
+                    # (the root's level runs LLB)
+                    assert st["steps"][("llb", "glb", "slb")[kind]] == depth + (kind == 0)
+    finally:
+        engine.set_scheduler_weights(None)
+        engine.set_params(**before)
