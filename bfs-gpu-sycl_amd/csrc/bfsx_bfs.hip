@@ -1294,22 +1294,28 @@ struct SpecGuard {
   }
 };
 
-// hbm bit h = frontier bit of hub[h] (H a multiple of 64, and so is the
-// grid-stride: every wave runs whole rounds).
-__global__ void k_hub_bits(const uint32_t *fbm, const uint32_t *hub, uint32_t H, uint32_t *hbm,
-                           SpecGuard guard) {
-  const uint32_t stride = gridDim.x * blockDim.x;
+// The hubs' frontier bits: hbm bit h = bit hub[h] of the frontier bitmap fbm
+// (H a multiple of 64).
+struct HubBits {
+  const uint32_t *fbm, *hub;
+  uint32_t *hbm;
+  uint32_t H;
+};
+
+// By the n_groups work-groups whose index among them is `group` (the stride
+// is a multiple of 64: every wave runs whole rounds).
+__device__ __forceinline__ void gather_hub_bits(const HubBits &b, uint32_t group,
+                                                uint32_t n_groups) {
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t h0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t v0 = h0 < H ? hub[h0] : 0u;  // in flight with the guard's reads
-  if (guard.skip()) return;
-  for (uint32_t h = h0; h < H; h += stride) {
-    const uint32_t v = h == h0 ? v0 : hub[h];
-    const unsigned long long m = __ballot((fbm[v >> 5] >> (v & 31)) & 1u);
-    if (lane == 0) hbm[h >> 5] = (uint32_t)m;
-    if (lane == 32) hbm[h >> 5] = (uint32_t)(m >> 32);
+  for (uint32_t h = group * blockDim.x + threadIdx.x; h < b.H; h += n_groups * blockDim.x) {
+    const uint32_t v = b.hub[h];
+    const unsigned long long m = __ballot((b.fbm[v >> 5] >> (v & 31)) & 1u);
+    if (lane == 0) b.hbm[h >> 5] = (uint32_t)m;
+    if (lane == 32) b.hbm[h >> 5] = (uint32_t)(m >> 32);
   }
 }
+
+__global__ void k_hub_bits(HubBits b) { gather_hub_bits(b, blockIdx.x, gridDim.x); }
 
 // Summary of a frontier bitmap: bit b = any frontier vertex in
 // [b << shift, (b + 1) << shift); shift >= 5, so a bit covers whole words.
@@ -2179,11 +2185,24 @@ __device__ __forceinline__ void write_level_end(LevelCtl *ctl, uint32_t produced
                 mirror);
 }
 
-__global__ __launch_bounds__(64) void k_level_end(LevelCtl *ctl, uint32_t consumed,
+// The first work-group ends the level.  After a step that wrote the next
+// frontier's bitmap the others, of WG 256, gather the hubs' bits from it for
+// a bottom-up step that may follow, beside the level's end instead of in a
+// launch after it (5-6 us at R-MAT 26, 3 at R-MAT 19, on every bottom-up
+// level; learned searches of R-MAT 16 / 19 / 22 / 24: 96.5 / 112.8 / 184.7 /
+// 312.6 -> 93.3 / 107.3 / 175.4 / 306.4 us).  They do so whatever the end decides: a speculative launch whose
+// guess failed leaves bits that no step reads.
+template <int WG>
+__global__ __launch_bounds__(WG) void k_level_end(LevelCtl *ctl, uint32_t consumed,
                                                   uint32_t produced, int stamp, int kind,
                                                   const float *Wg, uint64_t n_cols, uint64_t nnz,
                                                   uint64_t n_iso, uint32_t allow, int reuse,
-                                                  LevelMirror *mirror, SpecGuard guard) {
+                                                  LevelMirror *mirror, SpecGuard guard,
+                                                  HubBits hubs) {
+  if (WG > 64 && blockIdx.x > 0) {
+    gather_hub_bits(hubs, blockIdx.x - 1, gridDim.x - 1);
+    return;
+  }
   LevelEndWords words;
   if (!level_end_body(ctl, consumed, produced, stamp, kind, Wg, n_cols, nnz, n_iso, allow, reuse,
                       guard, &words))
@@ -2978,6 +2997,13 @@ static void launch_pull(unsigned grid, size_t lds, hipStream_t st, const KArgs &
 // work-group adds its totals to the same counters, 12 ns an addition).
 constexpr uint32_t PULL_MAX_CUT = 5, PULL_WAVES_PER_CU = 4;
 
+static HubBits hub_bits_of(bfsx_ctx *ctx, const uint32_t *fbm) {
+  return HubBits{fbm, ctx->pull_hub.as<uint32_t>(), ctx->pull_hbm.as<uint32_t>(), ctx->pull_hubs};
+}
+static unsigned hub_groups(const bfsx_ctx *ctx) {
+  return cap_grid(ctx->pull_hubs / 256 + 1, (unsigned)ctx->cu_count * 4);
+}
+
 template <typename PtrT>
 static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   const KArgs a = kargs(s, 0);
@@ -3033,13 +3059,14 @@ static void step_pull_t(bfsx_ctx *ctx, const StepArgs &s, bool speculative) {
   const uint32_t *iso = fd ? ctx->iso_bm.as<uint32_t>() : nullptr;
   const uint32_t *crank = fd ? ctx->pull_crank.as<uint32_t>() : nullptr;
   // hub indexing belongs to fd: the hubs' frontier bits, gathered first
+  // unless the previous level's end did
   const uint32_t *hbm = nullptr, *hub = nullptr;
   if (fd && ctx->pull_hubs) {
-    hub = ctx->pull_hub.as<uint32_t>();
-    hbm = ctx->pull_hbm.as<uint32_t>();
-    hipLaunchKernelGGL(k_hub_bits, dim3(cap_grid(ctx->pull_hubs / 256 + 1, (unsigned)ctx->cu_count * 4)),
-                       dim3(256), 0, st, s.fbm_cur, hub, ctx->pull_hubs, ctx->pull_hbm.as<uint32_t>(),
-                       guard);
+    const HubBits hb = hub_bits_of(ctx, s.fbm_cur);
+    hub = hb.hub;
+    hbm = hb.hbm;
+    if (!s.hubs_ready)
+      hipLaunchKernelGGL(k_hub_bits, dim3(hub_groups(ctx)), dim3(256), 0, st, hb);
   }
   KernelTimer kt(s, st);
   switch (wg) {
@@ -3147,13 +3174,21 @@ static uint64_t known_isolated(const bfsx_ctx *ctx) {
 }
 
 void level_end(bfsx_ctx *ctx, uint32_t consumed, uint32_t produced, bool stamp, int kind,
-               uint32_t decide_allow, bool reuse, uint32_t spec_kinds) {
-  hipLaunchKernelGGL(k_level_end, dim3(1), dim3(64), 0, ctx->stream, ctx->ctl.as<LevelCtl>(),
-                     consumed, produced, stamp ? 1 : 0, kind,
-                     decide_allow ? ctx->sched_w.as<float>() : (const float *)nullptr,
-                     (uint64_t)ctx->n_cols, (uint64_t)ctx->nnz, known_isolated(ctx), decide_allow,
-                     reuse ? 1 : 0, ctx->d_mirror,
-                     SpecGuard{spec_kinds ? ctx->ctl.as<LevelCtl>() : nullptr, consumed, spec_kinds});
+               uint32_t decide_allow, bool reuse, uint32_t spec_kinds, const uint32_t *next_fbm) {
+  const bool hubs = next_fbm && ctx->pull_fd.p && ctx->row_idx_pull.p && ctx->pull_hubs;
+  LevelCtl *ctl = ctx->ctl.as<LevelCtl>();
+  const float *w = decide_allow ? ctx->sched_w.as<float>() : nullptr;
+  const SpecGuard guard{spec_kinds ? ctl : nullptr, consumed, spec_kinds};
+  const HubBits hb = hubs ? hub_bits_of(ctx, next_fbm) : HubBits{};
+  if (hubs)
+    hipLaunchKernelGGL(k_level_end<256>, dim3(1 + hub_groups(ctx)), dim3(256), 0, ctx->stream, ctl,
+                       consumed, produced, stamp ? 1 : 0, kind, w, (uint64_t)ctx->n_cols,
+                       (uint64_t)ctx->nnz, known_isolated(ctx), decide_allow, reuse ? 1 : 0,
+                       ctx->d_mirror, guard, hb);
+  else
+    hipLaunchKernelGGL(k_level_end<64>, dim3(1), dim3(64), 0, ctx->stream, ctl, consumed, produced,
+                       stamp ? 1 : 0, kind, w, (uint64_t)ctx->n_cols, (uint64_t)ctx->nnz,
+                       known_isolated(ctx), decide_allow, reuse ? 1 : 0, ctx->d_mirror, guard, hb);
   BFSX_HIP(hipGetLastError());
 }
 

@@ -305,6 +305,7 @@ struct Walker {
   unsigned long long VE = 0;  // edges of the visited vertices
   int fbm_cur = 0;         // buffer holding the current frontier's bitmap
   bool fbm_valid = false;  // whether that bitmap is up to date
+  bool hubs_ready = false; // and the hubs' bits gathered from it
   bool queue_valid = true; // false after a bottom-up step (frontier only as bitmap)
   bool pull_possible = false;
   bool track = false;      // accumulate frontier degree sums
@@ -386,7 +387,9 @@ struct Walker {
         if (!pull_possible) fail(BFSX_ERR_UNSUPPORTED, "bottom-up step on a non-symmetric graph");
         if (ctx->row_idx_pull.p) a.row_idx = ctx->row_idx_pull.as<uint32_t>();
         // (the queue is valid whenever the bitmap is not: only a bottom-up
-        // step leaves the queue stale, and it writes the bitmap)
+        // step leaves the queue stale, and it writes the bitmap; the level
+        // end after a step that writes it makes the hubs ready)
+        a.hubs_ready = fbm_valid && hubs_ready;
         if (!fbm_valid) queue_to_fbm(ctx, a.q_in, F, ctx->fbm[fbm_cur].as<uint32_t>());
         a.fbm_cur = ctx->fbm[fbm_cur].as<uint32_t>();
         a.fbm_next = ctx->fbm[fbm_cur ^ 1].as<uint32_t>();
@@ -402,7 +405,8 @@ struct Walker {
       compact(ctx, a, a.mark, td_fbm_next);
       new_fbm = td_fbm_next != nullptr;
     }
-    level_end(ctx, cur, cur ^ 1, stamp, choice, decide_allow, decide_reuse);
+    level_end(ctx, cur, cur ^ 1, stamp, choice, decide_allow, decide_reuse, 0,
+              new_fbm ? ctx->fbm[fbm_cur ^ 1].as<uint32_t>() : nullptr);
     last = choice;
     return new_fbm;
   }
@@ -434,8 +438,10 @@ struct Walker {
     a.count_examined = count;
     a.fbm_cur = ctx->fbm[fbm_cur ^ 1].as<uint32_t>();
     a.fbm_next = ctx->fbm[fbm_cur].as<uint32_t>();
+    a.hubs_ready = true;
     step_pull(ctx, a, true);
-    level_end(ctx, cur ^ 1, cur, false, BFSX_PULL, decide_allow, decide_reuse, 1u << BFSX_PULL);
+    level_end(ctx, cur ^ 1, cur, false, BFSX_PULL, decide_allow, decide_reuse, 1u << BFSX_PULL,
+              a.fbm_next);
   }
 
   // The same after a top-down level, whose successor is often a thin
@@ -453,7 +459,7 @@ struct Walker {
   void advance(bool new_fbm) {
     ctx->mark_dirty = false;
     if (new_fbm) fbm_cur ^= 1;
-    fbm_valid = new_fbm;
+    fbm_valid = hubs_ready = new_fbm;
     queue_valid = last != BFSX_PULL;
     F = ctx->view.F;
     EF = ctx->view.EF;
@@ -888,6 +894,7 @@ static uint32_t record(bfsx_ctx *ctx, const uint32_t *roots, uint32_t n_roots, u
         for (uint32_t rep = 0; rep < repeats; rep++) {
           snapshot(ctx, false);
           w = saved;
+          w.hubs_ready = false;  // (another trial's level end gathered its own)
           // from an idle stream, as in a search, so that the time includes
           // the gaps of issuing the step's launches one after the other
           BFSX_HIP(hipStreamSynchronize(ctx->stream));
@@ -911,6 +918,7 @@ static uint32_t record(bfsx_ctx *ctx, const uint32_t *roots, uint32_t n_roots, u
       // run the chosen kind for real; the next row's inputs come from its state
       snapshot(ctx, false);
       w = saved;
+      w.hubs_ready = false;
       BFSX_HIP(hipMemcpyAsync(&ctx->ctl.as<LevelCtl>()->choice, &take, sizeof(uint32_t),
                               hipMemcpyHostToDevice, ctx->stream));
       const bool new_fbm = w.launch(take);  // its level end decides the next level

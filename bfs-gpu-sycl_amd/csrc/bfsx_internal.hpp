@@ -340,6 +340,7 @@ struct StepArgs {
   uint32_t *parents;       // nullable
   uint32_t *fbm_cur;       // frontier bitmap of this level (pull)
   uint32_t *fbm_next;      // next frontier bitmap (pull writes it)
+  bool hubs_ready;         // the hubs' bits of fbm_cur are gathered (see level_end)
   LevelCtl *ctl;
   int32_t next_level;
   bool track_degrees;      // accumulate degree sum of discovered vertices
@@ -372,9 +373,12 @@ void compact(bfsx_ctx *ctx, const StepArgs &s, uint8_t *mark, uint32_t *fbm_next
 // spec_kinds != 0: launched ahead of the previous level's decision; runs
 // only if that decision is one of these kinds (bit k for kind k) and the
 // frontier is not empty.
+// next_fbm: the next frontier's bitmap, if the level's step wrote it: the
+// same launch then makes the hubs ready for a bottom-up step on it
+// (StepArgs::hubs_ready).
 void level_end(bfsx_ctx *ctx, uint32_t consumed_idx, uint32_t produced_idx,
                bool stamp, int kind, uint32_t decide_allow = 0, bool reuse = false,
-               uint32_t spec_kinds = 0);
+               uint32_t spec_kinds = 0, const uint32_t *next_fbm = nullptr);
 // mark: which top-down levels mark and compact (needs track: the edge
 // counts are kept in the control block).
 void dev_level(bfsx_ctx *ctx, uint32_t cur, int fixed, bool track, MarkRule mark);

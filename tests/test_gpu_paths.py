@@ -440,3 +440,42 @@ def test_level_end_by_last_group(engine, width, kind, ptr):
     finally:
         engine.set_scheduler_weights(None)
         engine.set_params(**before)
+
+
+# hubs gathered at the level end: fixed and changing kinds of step, bottom-up
+# after bottom-up, after marking and bucketed steps and after thin ones, and
+# trials of every kind from one state (whose walk then covers each level)
+@pytest.mark.parametrize("scale", [9, 13, 16])
+@pytest.mark.parametrize("bucket", [0, 0xFFFFFFFF])
+def test_hubs_at_level_ends(engine, scale, bucket):
+    say("hubs", scale, bucket)
+    engine.generate_rmat(scale, 12, 0.57, 0.19, 0.19, 31 + scale, 41 + scale, 4)
+    cp, ri = engine.download_csc()
+    roots = engine.pick_roots(2, 9)
+    before = engine.params
+    try:
+        engine.set_params(bucket_ratio_q10=bucket)
+        engine.order_adjacency("pull_hub_first")
+        want = [cpu.bfs_queue(cp, ri, int(r)) for r in roots]
+        kinds = np.random.default_rng(scale)
+        for r, (lv, ec, _) in zip(roots, want):
+            for trial in range(6):
+                w = np.zeros(1476, np.float32)
+                w[:] = kinds.normal(0, 0.4, 1476)
+                engine.set_scheduler_weights(w)
+                for mark in (0, 4, 0xFFFFFFFF):
+                    engine.set_params(mark_ratio_q10=mark)
+                    lev, st = engine.run(int(r), "learned")
+                    assert np.array_equal(lev, lv) and st["edges_count"] == ec, (trial, mark)
+            for s in ("pull", "beamer"):
+                lev, st = engine.run(int(r), s)
+                assert np.array_equal(lev, lv) and st["edges_count"] == ec, s
+        engine.set_params(mark_ratio_q10=4)
+        X, _, _ = engine.sched_record(roots, repeats=2, epsilon=1.0, seed=3)
+        sizes = [int((lv == d).sum()) for lv, _, _ in want for d in range(int(lv.max()) + 1)]
+        got = np.rint(2.0 ** (X[:, 0].astype(np.float64) * 32) * (1 + len(cp) - 1) - 1).astype(int)
+        assert len(got) == len(sizes)
+        assert np.allclose(got, sizes, rtol=1e-3, atol=1)
+    finally:
+        engine.set_scheduler_weights(None)
+        engine.set_params(**before)
