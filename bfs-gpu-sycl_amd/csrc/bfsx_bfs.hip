@@ -2053,9 +2053,9 @@ __device__ __forceinline__ bool level_end_body(LevelCtl *ctl, uint32_t consumed,
                                                uint64_t n_iso, uint32_t allow, int reuse,
                                                const SpecGuard &guard,
                                                LevelEndWords *words = nullptr,
-                                               const float4 *staged = nullptr) {
+                                               const SchedLds *staged = nullptr) {
   __shared__ int s_live, s_skip;
-  __shared__ float4 s_W4[NPARAM / 4];
+  __shared__ SchedLds s_W;
   // the network's weights, loaded while thread 0 reads the control block
   // (both are round trips to memory; one waits for the other otherwise)
   constexpr int WPT = (NPARAM / 4 + 63) / 64;
@@ -2136,12 +2136,12 @@ __device__ __forceinline__ bool level_end_body(LevelCtl *ctl, uint32_t consumed,
 #pragma unroll
           for (int i = 0; i < WPT; i++) {
             const int j = (int)threadIdx.x + 64 * i;
-            if (j < NPARAM / 4) s_W4[j] = wr[i];
+            if (j < NPARAM / 4) stage_weights(s_W, j, wr[i]);
           }
         }
         __syncthreads();
       }
-      const uint32_t picked = decide_compute(ctl, staged ? staged : s_W4, produced, n_cols, nnz,
+      const uint32_t picked = decide_compute(ctl, staged ? *staged : s_W, produced, n_cols, nnz,
                                              n_iso, allow, 0);
       if (words && threadIdx.x == 0) words->choice = picked;
     }
@@ -2432,7 +2432,7 @@ struct SoloArgs {
 template <typename PtrT>
 __global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl, SoloArgs c) {
   __shared__ LevelCtl s_ctl;
-  __shared__ float4 s_W4[NPARAM / 4];
+  __shared__ SchedLds s_W;
   __shared__ PtrT s_nstart[SOLO_WG], s_start[SOLO_WG];       // next frontier's lists, this tile's
   __shared__ uint32_t s_ndeg[SOLO_WG], s_nv[SOLO_WG], s_v[SOLO_WG];
   __shared__ uint32_t s_scan[SOLO_WG], s_wave[SOLO_WG / 64 + 1];
@@ -2447,7 +2447,7 @@ __global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl,
     reinterpret_cast<uint32_t *>(&s_ctl)[t] = reinterpret_cast<const uint32_t *>(ctl)[t];
   if (c.Wg)
     for (uint32_t i = t; i < NPARAM / 4; i += SOLO_WG)
-      s_W4[i] = reinterpret_cast<const float4 *>(c.Wg)[i];
+      stage_weights(s_W, i, reinterpret_cast<const float4 *>(c.Wg)[i]);
   // (the queue holds n_cols + 1 entries: in bounds whatever the frontier)
   uint32_t v = t < a.n_cols ? c.queue[cur][t] : 0u;
   __syncthreads();
@@ -2586,7 +2586,7 @@ __global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl,
       s_ctl.q_edges[cur ^ 1] = s_edges;
     }
     level_end_body(&s_ctl, cur, cur ^ 1, 0, (int)choice, c.Wg, c.n_cols, c.nnz, c.n_iso, c.allow,
-                   1, SpecGuard{nullptr, 0, 0}, nullptr, s_W4);
+                   1, SpecGuard{nullptr, 0, 0}, nullptr, &s_W);
     __syncthreads();
     prev_F = F;
     cur ^= 1;
