@@ -395,17 +395,29 @@ struct LlbShared {
 // 160 K at R-MAT 16 229 -> 12 us; 7.6 K, 5.5 M at R-MAT 19 343 -> 39 us;
 // 78, 763 K at R-MAT 24 1507 -> 44 us; whole fixed-LLB searches of R-MAT 16 /
 // 19 / 22 / 24: 282 / 511 / 1855 / 8159 -> 112 / 180 / 1095 / 4661 us.
-constexpr uint32_t LLB_ROUNDS = 4, LLB_MAX_PARTS = 64;
+// A level of few tiles leaves CUs idle whatever its edges, and a group's
+// gathers take a cycle an address, so such tiles are shared by up to
+// LLB_FILL groups in all, with at least a wave's round of edges each; more
+// groups lose what they gain to their additions to the counts.  Learned
+// searches without / with this, us: R-MAT 10 80 / 74.5, 12 93 / 84, 14 83.8 /
+// 81.4, 19 104.5 / 101, 4096^2 grid 6885 / 6790 (at 16 groups 7000, at 256
+// 6980 where 128 had 6940); fixed LLB R-MAT 12 88.8 / 78.5.
+constexpr uint32_t LLB_ROUNDS = 4, LLB_MAX_PARTS = 64, LLB_FILL = 128;
 __host__ __device__ inline uint32_t llb_parts(unsigned long long EF, uint32_t n_tiles,
                                               uint32_t wg) {
   const unsigned long long per = (unsigned long long)wg * EPT * LLB_ROUNDS * n_tiles;
-  const unsigned long long p = per ? (EF + per - 1) / per : 1;
+  if (!per) return 1;
+  unsigned long long p = (EF + per - 1) / per;
+  const unsigned long long wave = 64ull * EPT * n_tiles;
+  const unsigned long long waves = (EF + wave - 1) / wave, few = LLB_FILL / n_tiles;
+  const unsigned long long fill = waves < few ? waves : few;
+  p = p < fill ? fill : p;
   return p < 1 ? 1u : p > LLB_MAX_PARTS ? LLB_MAX_PARTS : (uint32_t)p;
 }
 
 // One LLB tile: WG frontier entries (contiguous, or strided by n_tiles for
 // SLB), block scan of their degrees, cooperative expansion of their edges
-// (of slice `part` of n_parts; a slice holds at least one round of edges, so
+// (of slice `part` of n_parts; a slice holds at least a wave's round of edges, so
 // the later parts of a small tile have none).
 template <typename PtrT, int WG, bool HOT = false>
 __device__ __forceinline__ void llb_tile(const KArgs &a, LlbShared<PtrT, WG> &sh, uint32_t tile,
@@ -450,9 +462,9 @@ __device__ __forceinline__ void llb_tile(const KArgs &a, LlbShared<PtrT, WG> &sh
   // the next one and are skipped by taking the last)
   PtrT lo = 0, hi = total;
   if (n_parts > 1) {
-    constexpr PtrT ROUND = (PtrT)WG * EPT;
+    constexpr PtrT MIN = (PtrT)64 * EPT;
     PtrT per = total / n_parts + 1;  // (sums that fit PtrT whatever total is)
-    per = per < ROUND ? ROUND : (per + EPT - 1) / EPT * EPT;
+    per = per < MIN ? MIN : (per + EPT - 1) / EPT * EPT;
     lo = part < total / per + 1 ? (PtrT)part * per : total;
     hi = total - lo > per ? lo + per : total;
   }
