@@ -2616,15 +2616,19 @@ __global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl,
 // One pass over the levels and the 16-bit degrees (6 bytes per vertex), four
 // vertices per lane as wide loads.  What bounds it is not those bytes but
 // adding to a few hot counters: a power-law graph has about seven levels, so
-// a wave's 64 vertices share two or three.  A wave therefore adds up its
-// equal levels in registers first (a ballot per distinct level, up to
-// HIST_ROUNDS of them, a grid's many levels per wave go to LDS lane by
-// lane), work-groups add in LDS, and there is one large work-group per CU:
+// a wave's 256 vertices share four or five.  A wave therefore adds up its
+// equal levels in registers first (ballots and one wave sum per distinct
+// level, up to HIST_ROUNDS of them, a grid's many levels per wave go to LDS
+// lane by lane), work-groups add in LDS, and there is one large work-group per CU:
 // global atomics on one line take 12 ns each, and 1024 groups spent more on
 // them than on the pass.
-constexpr uint32_t HIST_LDS_LEVELS = 1024;
+// One ballot loop per 256 vertices instead of four per 64 each, and counters
+// for 4096 levels in LDS instead of 1024 (us a call): R-MAT 26 483 -> 248,
+// 4096^2 grid of 350 levels 250 -> 131, of more than 1024 levels 3630 -> 263
+// (vertex by vertex in memory: 2100).
+constexpr uint32_t HIST_LDS_LEVELS = 4096;
 constexpr uint32_t HIST_WG = 1024;
-constexpr int HIST_ROUNDS = 4;
+constexpr int HIST_ROUNDS = 6;
 
 template <typename PtrT>
 __global__ __launch_bounds__(HIST_WG) void k_level_hist(const PtrT *col_ptr,
@@ -2632,12 +2636,19 @@ __global__ __launch_bounds__(HIST_WG) void k_level_hist(const PtrT *col_ptr,
                                                         const int32_t *levels, uint32_t n_rows,
                                                         uint32_t n_cols, uint32_t max_levels,
                                                         unsigned long long *out) {
-  __shared__ unsigned long long s_cnt[HIST_LDS_LEVELS];
+  __shared__ uint32_t s_cnt[HIST_LDS_LEVELS];
   __shared__ unsigned long long s_edg[HIST_LDS_LEVELS];
   __shared__ int s_max;
   const bool lds = max_levels <= HIST_LDS_LEVELS;
-  unsigned long long *cnt = lds ? s_cnt : out + 1;
-  unsigned long long *edg = lds ? s_edg : out + 1 + max_levels;
+  auto add = [&](int32_t l, uint32_t n, unsigned long long d) {
+    if (lds) {
+      atomicAdd(&s_cnt[l], n);
+      if (d) atomicAdd(&s_edg[l], d);
+    } else {
+      atomicAdd(&out[1 + l], (unsigned long long)n);
+      if (d) atomicAdd(&out[1 + max_levels + l], d);
+    }
+  };
   if (lds)
     for (uint32_t i = threadIdx.x; i < max_levels; i += HIST_WG) s_cnt[i] = s_edg[i] = 0;
   if (threadIdx.x == 0) s_max = -1;
@@ -2648,52 +2659,57 @@ __global__ __launch_bounds__(HIST_WG) void k_level_hist(const PtrT *col_ptr,
   const uint64_t stride = (uint64_t)gridDim.x * HIST_WG;
   const uint64_t first = blockIdx.x * (uint64_t)HIST_WG + (threadIdx.x & ~63u);
   for (uint64_t base = first; base < n4; base += stride) {
-    const uint64_t v0 = (base + (threadIdx.x & 63)) * 4;
+    // A lane's four vertices: consecutive, or 64 apart where the adds go to
+    // memory (an instruction's 64 vertices then share few lines of counters).
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t v0 = lds ? (base + lane) * 4 : base * 4 + lane;
+    const uint32_t step = lds ? 1 : 64;
     int32_t l4[4] = {-1, -1, -1, -1};
     uint32_t d4[4] = {0, 0, 0, 0};
-    if (v0 + 4 <= n_cols) {
+    if (lds && v0 + 4 <= n_cols) {
       const int4 l = *reinterpret_cast<const int4 *>(levels + v0);
       const ushort4 d = *reinterpret_cast<const ushort4 *>(deg16 + v0);
       l4[0] = l.x, l4[1] = l.y, l4[2] = l.z, l4[3] = l.w;
       d4[0] = d.x, d4[1] = d.y, d4[2] = d.z, d4[3] = d.w;
     } else {
       for (int k = 0; k < 4; k++)
-        if (v0 + k < n_cols) {
-          l4[k] = levels[v0 + k];
-          d4[k] = deg16[v0 + k];
+        if (v0 + k * step < n_cols) {
+          l4[k] = levels[v0 + k * step];
+          d4[k] = deg16[v0 + k * step];
         }
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < 4; k++) {  // (a level of -1: nothing left to add)
       const int32_t l = l4[k];
       mx = l > mx ? l : mx;
-      const bool in = l >= 0 && (uint32_t)l < max_levels;
-      const uint32_t d = in && v0 + k < n_rows ? d4[k] : 0u;
-      bool todo = in;
-      if (d == DEG16_ESCAPE) {  // (few) the whole degree
-        const uint32_t v = (uint32_t)(v0 + k);
-        atomicAdd(&cnt[l], 1ull);
-        atomicAdd(&edg[l], (unsigned long long)(col_ptr[v + 1] - col_ptr[v]));
-        todo = false;
-      }
-      unsigned long long m = __ballot(todo);
-      for (int r = 0; m && r < HIST_ROUNDS; r++) {
-        const int leader = __ffsll(m) - 1;
-        const int32_t L = __shfl(l, leader, 64);
-        const unsigned long long same = __ballot(todo && l == L);
-        const uint32_t sum = wave_sum(todo && l == L ? d : 0u);  // below 64 * 2^16
-        if ((int)__lane_id() == leader) {
-          atomicAdd(&cnt[L], (unsigned long long)__popcll(same));
-          if (sum) atomicAdd(&edg[L], (unsigned long long)sum);
-        }
-        if (l == L) todo = false;
-        m &= ~same;
-      }
-      if (todo) {
-        atomicAdd(&cnt[l], 1ull);
-        if (d) atomicAdd(&edg[l], (unsigned long long)d);
+      if (l < 0 || (uint32_t)l >= max_levels) l4[k] = -1;
+      if (l4[k] < 0 || v0 + k * step >= n_rows) d4[k] = 0;
+      if (d4[k] == DEG16_ESCAPE) {  // (few) the whole degree
+        const uint64_t v = v0 + k * step;
+        add(l, 1, (unsigned long long)(col_ptr[v + 1] - col_ptr[v]));
+        l4[k] = -1;
       }
     }
+    for (int r = 0; r < HIST_ROUNDS; r++) {
+      const int32_t p01 = l4[0] > l4[1] ? l4[0] : l4[1], p23 = l4[2] > l4[3] ? l4[2] : l4[3];
+      const int32_t pick = p01 > p23 ? p01 : p23;
+      const unsigned long long m = __ballot(pick >= 0);
+      if (!m) break;
+      const int32_t L = __builtin_amdgcn_readlane(pick, __ffsll(m) - 1);
+      uint32_t n = 0, sum = 0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bool same = l4[k] == L;
+        n += (uint32_t)__popcll(__ballot(same));
+        sum += same ? d4[k] : 0u;
+        l4[k] = same ? -1 : l4[k];
+      }
+      sum = wave_sum(sum);  // below 256 * 2^16
+      if (__lane_id() == 0) add(L, n, sum);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (l4[k] >= 0) add(l4[k], 1, d4[k]);
   }
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
@@ -2705,7 +2721,7 @@ __global__ __launch_bounds__(HIST_WG) void k_level_hist(const PtrT *col_ptr,
   if (threadIdx.x == 0 && s_max >= 0) atomicMax(&out[0], (unsigned long long)s_max + 1);
   if (lds)
     for (uint32_t i = threadIdx.x; i < max_levels; i += HIST_WG) {
-      if (s_cnt[i]) atomicAdd(&out[1 + i], s_cnt[i]);
+      if (s_cnt[i]) atomicAdd(&out[1 + i], (unsigned long long)s_cnt[i]);
       if (s_edg[i]) atomicAdd(&out[1 + max_levels + i], s_edg[i]);
     }
 }

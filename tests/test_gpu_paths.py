@@ -479,3 +479,27 @@ def test_hubs_at_level_ends(engine, scale, bucket):
     finally:
         engine.set_scheduler_weights(None)
         engine.set_params(**before)
+
+
+# the histogram's two places to add: LDS up to 4096 levels, memory beyond
+@pytest.mark.parametrize("depth", [4095, 4096, 4097])
+@pytest.mark.parametrize("size", [1024, 4096, 4097, 9000])
+def test_level_histogram_depths(engine, depth, size):
+    say("histogram depths", depth, size)
+    rng = np.random.default_rng(depth)
+    # a path of `depth` vertices, some with leaves, the ids shuffled
+    k = 3000
+    at = rng.integers(0, depth - 1, k)
+    at[:200] = 77
+    name = rng.permutation(depth + k)
+    src = name[np.concatenate([np.arange(depth - 1), at])]
+    dst = name[np.concatenate([np.arange(1, depth), depth + np.arange(k)])]
+    cp, ri = csc_from_edges(depth + k, *symmetrize(src, dst))
+    engine.upload_csc(cp, ri, symmetric=True)
+    lev, st = engine.run(int(name[0]), "llb")
+    want, ec, _ = cpu.bfs_queue(cp, ri, int(name[0]))
+    assert (lev == want).all() and st["n_levels"] == depth
+    counts, edges = engine.level_histogram(size)
+    deg = np.diff(cp.astype(np.int64))
+    assert (counts == np.bincount(want)).all()
+    assert (edges == np.bincount(want, weights=deg)).all()
