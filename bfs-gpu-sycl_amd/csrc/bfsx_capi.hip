@@ -231,7 +231,8 @@ static void view_from_ctl(bfsx_ctx *ctx, uint32_t produced) {
   ctx->view.prev_F = 0;  // (not kept in the block)
 }
 
-// After a launch that ends with k_level_end: that kernel writes the values
+// After a launch that ends a level (k_level_end, a speculative top-down
+// step, a device loop): it writes the values
 // the host needs into the host-mapped mirror, every word tagged with its
 // sequence number, so the host polls the words (no copy, no stream
 // synchronisation) until all of them carry `seq` -- a word of the previous

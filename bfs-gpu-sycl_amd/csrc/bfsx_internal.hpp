@@ -57,7 +57,7 @@ struct LevelCtl {
   uint32_t pad_[30];  // bar_gen on another 128-byte line: polls do not hit the arrivals' line
   uint32_t bar_gen;
   uint32_t reserved;
-  // Level ends so far on this context: only the level-end kernel changes it
+  // Level ends so far on this context: only a level's end changes it
   // (+1 each), so the tag it puts on the host-mapped words never repeats;
   // every other writer of the block keeps it (CTL_RESET_BYTES).
   uint32_t seq;
@@ -67,7 +67,7 @@ static_assert(offsetof(LevelCtl, seq) + sizeof(uint32_t) == sizeof(LevelCtl),
 constexpr size_t CTL_RESET_BYTES = offsetof(LevelCtl, seq);
 
 // What the host reads at a level end without synchronising the stream:
-// 8-byte words in host-mapped memory, written by the level-end kernel.
+// 8-byte words in host-mapped memory, written by the level's end.
 // Device writes to host memory can reach it out of order even across a
 // system-scope fence, so every word carries the level end's sequence number
 // and the host takes the words only once all of them carry the number it
@@ -218,7 +218,7 @@ struct bfsx_ctx {
   bfsx::DevBuf scratch;  // generic scratch (reductions, root picking)
   bfsx::LevelCtl *h_ctl = nullptr;        // pinned: full copies of the control block
   bfsx::LevelMirror *h_mirror = nullptr;  // pinned, host-mapped: tagged level-end words (2 sets)
-  bfsx::LevelMirror *d_mirror = nullptr;  // device address of h_mirror (k_level_end writes it)
+  bfsx::LevelMirror *d_mirror = nullptr;  // device address of h_mirror (a level's end writes it)
   bfsx::LevelView view;                   // the values of the last level end the host read
   // level ends so far (LevelCtl::seq), while the host knows it: a search
   // that ran to its end knows the next one's first sequence number without

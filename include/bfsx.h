@@ -166,8 +166,10 @@ typedef struct bfsx_params {
                                every target, no random stores or atomics)
                                when the unvisited vertices' edges are at
                                least nnz * bucket_ratio_q10 / 1024, i.e. when
-                               most frontier edges lead to new vertices
-                               (0 = always, 0xFFFFFFFF = never; not with
+                               most frontier edges lead to new vertices, on
+                               graphs of more than 2^22 vertices
+                               (0 = always, on graphs of any size,
+                               0xFFFFFFFF = never; not with
                                mark_ratio_q10 = 0xFFFFFFFF or parents;
                                graphs of up to 2^27 vertices) */
   /* batched searches (bfsx_run_multi) */
