@@ -2554,11 +2554,15 @@ __global__ __launch_bounds__(SOLO_WG) void k_solo_levels(KArgs a, LevelCtl *ctl,
 #pragma unroll
           for (int k = 0; k < EPT; k++) {
             cand[k] = cand[k] && !(old[k] & bit[k]);
-            ndeg[k] = n[k] < a.n_rows ? (uint32_t)(end[k] - nstart[k]) : 0u;
+            const unsigned long long d =
+                n[k] < a.n_rows ? (unsigned long long)(end[k] - nstart[k]) : 0ull;
+            // (a list may hold 2^32 entries and more: the sum counts them all,
+            // and the loop leaves before a level whose lengths are cut here)
+            ndeg[k] = d > c.max_edges ? c.max_edges : (uint32_t)d;
             if (cand[k]) {
               a.levels[n[k]] = next_level;
               if (a.parents) a.parents[n[k]] = from[k];
-              dacc += ndeg[k];
+              dacc += d;
               cnt++;
             }
           }

@@ -503,3 +503,27 @@ def test_level_histogram_depths(engine, depth, size):
     deg = np.diff(cp.astype(np.int64))
     assert (counts == np.bincount(want)).all()
     assert (edges == np.bincount(want, weights=deg)).all()
+
+
+# a list of more than 2^32 entries (17 GB of zeroes, so the edges are repeats
+# of one) behind a level that one work-group's loop runs
+def test_list_beyond_32_bits(engine):
+    import bfsx
+    length = 2 ** 32 + 5
+    cp = np.array([0, 1, 1 + length, 2 + length, 3 + length, 3 + length, 3 + length], np.uint64)
+    ri = np.zeros(length + 3, np.uint32)
+    # 0 -> 1 -> {0 (often), 2, 3}, 2 -> 4, 3 -> 5
+    ri[[0, 1001, length, 1 + length, 2 + length]] = [1, 2, 3, 4, 5]
+    want = [0, 1, 2, 2, 3, 3]
+    with bfsx.Engine(0) as eng:
+        eng.upload_csc(cp, ri)
+        del ri
+        w = np.zeros(1476, np.float32)
+        w[-3:] = 1  # constant outputs: LLB, the smallest, at every level
+        eng.set_scheduler_weights(w)
+        for s in ("llb", "slb", "learned"):
+            say("long list", s)
+            lev, st, par = eng.run(0, s, parents=True)
+            assert lev.tolist() == want, s
+            assert st["edges_count"] == length + 3 and st["reached"] == 6, s
+            assert par[1:].tolist() == [0, 1, 1, 2, 3], s
