@@ -1111,15 +1111,21 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
                                 : static_cast<const uint32_t *>(col_ptr)[i];
     };
     if (at(0) != 0) fail(BFSX_ERR_ARG, "col_ptr[0] != 0");
-    auto refuse = [&](bool falls, bool outside) {
+    // row_idx has as many entries as col_ptr says: it is not touched before
+    // col_ptr is known to be sound and to end at nnz
+    auto refuse_offsets = [&](bool falls) {
       if (falls) fail(BFSX_ERR_ARG, "col_ptr is not monotone");
       if (at(n_rows) > nnz || at(n_cols) != nnz)
         fail(BFSX_ERR_ARG, "col_ptr end does not match nnz");
+    };
+    auto refuse_targets = [&](bool outside) {
       if (outside) fail(BFSX_ERR_ARG, "row_idx entry >= n_cols");
     };
     // The arrays go into buffers of their own and are checked on the card (a
     // pass over 64 MB took the host 3.5 ms, as long as their transfer): a
     // graph that is refused leaves the resident one as it was.
+    const size_t cp_bytes = (size_t)col_ptr_bytes * n1;
+    const size_t ri_bytes = sizeof(uint32_t) * (nnz ? nnz : 1);
     DevBuf cp, ri;
     struct Releaser {
       DevBuf *b[2];
@@ -1127,33 +1133,39 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
         for (DevBuf *x : b) release(*x);
       }
     } releaser{{&cp, &ri}};
-    bool beside = true;
-    try {
-      ensure(cp, (size_t)col_ptr_bytes * n1, ctx);
-      ensure(ri, sizeof(uint32_t) * (nnz ? nnz : 1), ctx);
-    } catch (const Error &e) {
-      if (e.status != BFSX_ERR_NOMEM) throw;
-      beside = false;
+    auto room_for = [&](DevBuf &b, size_t bytes) {
+      try {
+        ensure(b, bytes, ctx);
+        return true;
+      } catch (const Error &e) {
+        if (e.status != BFSX_ERR_NOMEM) throw;
+        (void)hipGetLastError();
+        return false;
+      }
+    };
+    bool beside = room_for(cp, cp_bytes);
+    if (beside) {
+      copy_in(ctx, cp.p, col_ptr, cp_bytes);
+      refuse_offsets(offsets_fall(ctx, cp.p, col_ptr_bytes, n_cols));
+      beside = room_for(ri, ri_bytes);
     }
-    if (!beside) {  // no room for both graphs: checked on the host first
-      (void)hipGetLastError();
-      release(cp);
-      release(ri);
+    if (beside) {
+      copy_in(ctx, ri.p, row_idx, sizeof(uint32_t) * nnz);
+      refuse_targets(targets_outside(ctx, ri.as<uint32_t>(), nnz, n_cols));
+    } else {  // no room for both graphs: checked on the host first
       bool falls = false, outside = false;
       for (uint64_t i = 1; i < n1; i++) falls |= at(i) < at(i - 1);
+      refuse_offsets(falls);
       for (uint64_t i = 0; i < nnz; i++) outside |= row_idx[i] >= n_cols;
-      refuse(falls, outside);
+      refuse_targets(outside);
       ctx->has_graph = false;
+      release(cp);
       release(ctx->col_ptr);
       release(ctx->row_idx);
-      ensure(cp, (size_t)col_ptr_bytes * n1, ctx);
-      ensure(ri, sizeof(uint32_t) * (nnz ? nnz : 1), ctx);
-    }
-    copy_in(ctx, cp.p, col_ptr, (size_t)col_ptr_bytes * n1);
-    copy_in(ctx, ri.p, row_idx, sizeof(uint32_t) * nnz);
-    if (beside) {
-      const uint32_t bad = check_csc(ctx, cp.p, col_ptr_bytes, n_cols, ri.as<uint32_t>(), nnz);
-      refuse(bad & 1u, bad & 2u);
+      ensure(cp, cp_bytes, ctx);
+      ensure(ri, ri_bytes, ctx);
+      copy_in(ctx, cp.p, col_ptr, cp_bytes);
+      copy_in(ctx, ri.p, row_idx, sizeof(uint32_t) * nnz);
     }
     ctx->has_graph = false;
     std::swap(ctx->col_ptr, cp);

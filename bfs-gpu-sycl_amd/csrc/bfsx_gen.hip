@@ -380,44 +380,67 @@ void graph_summary(bfsx_ctx *ctx) {
 }
 
 // ---- check of an uploaded graph ------------------------------------------------
-// flags[0] = 1 where col_ptr falls, flags[1] = 1 for a row_idx entry >= n_cols
-// (all writers store the same value); 16 bytes per lane and step.
+// *flag = 1 where an entry is wrong (one store per wave that saw one).  The
+// flag is a host-mapped word that no level end writes: the host clears it and
+// reads it after the kernel, so a check is one launch and one wait (a flag on
+// the card takes a fill and a copy more).
+__device__ __forceinline__ void raise_flag(bool bad, uint32_t *flag) {
+  if (__ballot(bad) && (threadIdx.x & 63) == 0) *flag = 1;
+}
+
 template <typename PtrT>
-__global__ __launch_bounds__(256) void k_check_csc(const PtrT *col_ptr, uint32_t n_cols,
-                                                   const uint32_t *row_idx, uint64_t nnz,
-                                                   uint32_t *flags) {
+__global__ __launch_bounds__(256) void k_check_offsets(const PtrT *col_ptr, uint32_t n_cols,
+                                                       uint32_t *flag) {
+  const uint64_t stride = (uint64_t)gridDim.x * 256;
+  bool falls = false;
+  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n_cols; i += stride)
+    falls |= col_ptr[i + 1] < col_ptr[i];
+  raise_flag(falls, flag);
+}
+
+// (16 bytes per lane and step)
+__global__ __launch_bounds__(256) void k_check_targets(const uint32_t *row_idx, uint64_t nnz,
+                                                       uint32_t n_cols, uint32_t *flag) {
   const uint64_t stride = (uint64_t)gridDim.x * 256;
   const uint64_t t0 = blockIdx.x * 256ull + threadIdx.x;
-  bool falls = false, outside = false;
-  for (uint64_t i = t0; i < n_cols; i += stride) falls |= col_ptr[i + 1] < col_ptr[i];
+  bool outside = false;
   const uint64_t n4 = nnz / 4;
   for (uint64_t i = t0; i < n4; i += stride) {
     const uint4 x = reinterpret_cast<const uint4 *>(row_idx)[i];
     outside |= x.x >= n_cols || x.y >= n_cols || x.z >= n_cols || x.w >= n_cols;
   }
   for (uint64_t i = n4 * 4 + t0; i < nnz; i += stride) outside |= row_idx[i] >= n_cols;
-  if (falls) flags[0] = 1;
-  if (outside) flags[1] = 1;
+  raise_flag(outside, flag);
 }
 
-uint32_t check_csc(bfsx_ctx *ctx, const void *col_ptr, int col_ptr_bytes, uint32_t n_cols,
-                   const uint32_t *row_idx, uint64_t nnz) {
-  hipStream_t s = ctx->stream;
-  ensure(ctx->scratch, 64, ctx);
-  uint32_t *flags = ctx->scratch.as<uint32_t>();
-  BFSX_HIP(hipMemsetAsync(flags, 0, 2 * sizeof(uint32_t), s));
-  const unsigned grid = grid_for(std::max<uint64_t>(n_cols, nnz / 4));
-  if (col_ptr_bytes == 8)
-    hipLaunchKernelGGL(k_check_csc<uint64_t>, dim3(grid), dim3(256), 0, s,
-                       static_cast<const uint64_t *>(col_ptr), n_cols, row_idx, nnz, flags);
-  else
-    hipLaunchKernelGGL(k_check_csc<uint32_t>, dim3(grid), dim3(256), 0, s,
-                       static_cast<const uint32_t *>(col_ptr), n_cols, row_idx, nnz, flags);
+// What launch(flag) leaves in the flag.
+template <class F> static bool checked(bfsx_ctx *ctx, F launch) {
+  volatile unsigned long long *flag = &ctx->h_mirror->w[MIRROR_FLAG];
+  *flag = 0;
+  launch(reinterpret_cast<uint32_t *>(&ctx->d_mirror->w[MIRROR_FLAG]));
   BFSX_HIP(hipGetLastError());
-  uint32_t h[2] = {0, 0};
-  BFSX_HIP(hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, s));
-  BFSX_HIP(hipStreamSynchronize(s));
-  return (h[0] ? 1u : 0u) | (h[1] ? 2u : 0u);
+  BFSX_HIP(hipStreamSynchronize(ctx->stream));
+  return *flag != 0;
+}
+
+bool offsets_fall(bfsx_ctx *ctx, const void *col_ptr, int col_ptr_bytes, uint32_t n_cols) {
+  return checked(ctx, [&](uint32_t *flag) {
+    const dim3 grid(grid_for(n_cols));
+    if (col_ptr_bytes == 8)
+      hipLaunchKernelGGL(k_check_offsets<uint64_t>, grid, dim3(256), 0, ctx->stream,
+                         static_cast<const uint64_t *>(col_ptr), n_cols, flag);
+    else
+      hipLaunchKernelGGL(k_check_offsets<uint32_t>, grid, dim3(256), 0, ctx->stream,
+                         static_cast<const uint32_t *>(col_ptr), n_cols, flag);
+  });
+}
+
+bool targets_outside(bfsx_ctx *ctx, const uint32_t *row_idx, uint64_t nnz, uint32_t n_cols) {
+  if (nnz == 0) return false;
+  return checked(ctx, [&](uint32_t *flag) {
+    hipLaunchKernelGGL(k_check_targets, dim3(grid_for(nnz / 4)), dim3(256), 0, ctx->stream, row_idx,
+                       nnz, n_cols, flag);
+  });
 }
 
 // ---- adjacency order --------------------------------------------------------

@@ -84,8 +84,9 @@ constexpr size_t CTL_RESET_BYTES = offsetof(LevelCtl, seq);
 // of the host's read of the previous one (a speculative step) writes the
 // other set, so it cannot overwrite words the host has not read yet.
 struct LevelMirror {
-  unsigned long long w[8];  // (w[7] unused: a set is one 64-byte line)
+  unsigned long long w[8];  // a set is one 64-byte line
 };
+constexpr int MIRROR_FLAG = 7;  // no level end's word: of set 0, the flag of graph checks
 constexpr int MIRROR_SLOTS = 2;
 constexpr unsigned long long MIRROR_48 = (1ull << 48) - 1;
 constexpr uint32_t MIRROR_LEVEL_MASK = (1u << 23) - 1;
@@ -282,9 +283,9 @@ uint64_t gen_grid_pairs(bfsx_ctx *ctx, uint32_t side, uint32_t t_drop,
                         uint32_t n_long, uint64_t seed, uint32_t *d_u,
                         uint32_t *d_v);
 void graph_summary(bfsx_ctx *ctx);  // max degree, isolated bitmap/count
-// Bit 0: col_ptr falls somewhere; bit 1: a row_idx entry is >= n_cols.
-uint32_t check_csc(bfsx_ctx *ctx, const void *col_ptr, int col_ptr_bytes, uint32_t n_cols,
-                   const uint32_t *row_idx, uint64_t nnz);
+// Whether col_ptr falls somewhere; whether a row_idx entry is >= n_cols.
+bool offsets_fall(bfsx_ctx *ctx, const void *col_ptr, int col_ptr_bytes, uint32_t n_cols);
+bool targets_outside(bfsx_ctx *ctx, const uint32_t *row_idx, uint64_t nnz, uint32_t n_cols);
 // re-sorts every adjacency list by neighbour id or hub first (needs graph_summary)
 // Sorts every adjacency list (id order, or hub first) into `out`, which is
 // ctx->row_idx (in place) or a copy of the same size.  With hub_first,

@@ -1,0 +1,209 @@
+// The engine's host side (libbfsx.so) on the CPU, over a stand-in for the HIP
+// runtime: device memory is host memory behind a limit, copies and fills run
+// at once, kernel launches do nothing but are counted.  The executable's
+// definitions come before the runtime library's.  For what happens before and
+// between kernels: what a refused call has touched, and which memory is held
+// when an allocation fails.
+#include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "bfsx.h"
+
+// ---- the stand-in --------------------------------------------------------------
+static std::mutex mu;
+static std::map<void *, size_t> blocks;  // device memory
+static size_t live = 0, limit = 1u << 30, launches = 0;
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) {
+  std::lock_guard<std::mutex> g(mu);
+  if (n > limit || live > limit - n) return hipErrorOutOfMemory;
+  *p = calloc(n, 1);
+  if (!*p) return hipErrorOutOfMemory;
+  blocks[*p] = n;
+  live += n;
+  return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+  std::lock_guard<std::mutex> g(mu);
+  auto it = blocks.find(p);
+  if (it == blocks.end()) return p ? hipErrorInvalidValue : hipSuccess;
+  live -= it->second;
+  blocks.erase(it);
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  *p = calloc(n, 1);
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void *p) {
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) {
+  *d = h;
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+  memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
+  memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) {
+  return hipErrorInvalidValue;  // no pointer of the callers is the runtime's
+}
+hipError_t hipGetDeviceCount(int *n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {  // (the header's versioned name)
+  memset(p, 0, sizeof(*p));
+  p->multiProcessorCount = 256;
+  p->sharedMemPerBlock = 65536;
+  p->warpSize = 64;
+  strcpy(p->gcnArchName, "gfx950");
+  return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) {
+  *v = 0;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevice(int *d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+  *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+int hipGetStreamDeviceId(hipStream_t) { return 0; }
+hipError_t hipEventCreate(hipEvent_t *e) {
+  *e = nullptr;
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *m, hipStream_t *s) {
+  *g = *b = dim3(1);
+  *m = 0;
+  *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) {
+  launches++;
+  return hipSuccess;
+}
+void **__hipRegisterFatBinary(const void *) { return reinterpret_cast<void **>(&launches); }
+void __hipRegisterFunction(void **, const void *, char *, const char *, int, void *, void *, void *,
+                           void *, int *) {}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+void __hipUnregisterFatBinary(void **) {}
+}
+
+// ---- the checks ----------------------------------------------------------------
+static bfsx_ctx *ctx;
+
+#define CHECK(x)                                                                  \
+  do {                                                                            \
+    if (!(x)) {                                                                   \
+      fprintf(stderr, "line %d: %s (last error: %s)\n", __LINE__, #x, bfsx_last_error(ctx)); \
+      exit(1);                                                                    \
+    }                                                                             \
+  } while (0)
+
+static bool says(const char *text) { return strstr(bfsx_last_error(ctx), text) != nullptr; }
+
+// n bytes that end where the process may not read on
+static void *fenced(size_t n) {
+  const size_t page = 4096, room = (n + page - 1) / page * page;
+  char *p = static_cast<char *>(
+      mmap(nullptr, room + page, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0));
+  mprotect(p + room, page, PROT_NONE);
+  return p + room - n;
+}
+
+// a cycle of n vertices: one entry per list
+template <class P> struct Cycle {
+  std::vector<P> cp;
+  std::vector<uint32_t> ri;
+  explicit Cycle(uint32_t n) : cp(n + 1), ri(n) {
+    for (uint32_t i = 0; i <= n; i++) cp[i] = i;
+    for (uint32_t i = 0; i < n; i++) ri[i] = (i + 1) % n;
+  }
+  int upload() {
+    const uint32_t n = (uint32_t)ri.size();
+    return bfsx_upload_csc(ctx, n, n, cp.data(), sizeof(P), ri.data(), n, 0);
+  }
+  // whether this is the resident graph
+  bool resident() {
+    std::vector<P> c(cp.size());
+    std::vector<uint32_t> r(ri.size());
+    bfsx_graph_info g;
+    return bfsx_graph_info_get(ctx, &g) == BFSX_OK && g.nnz == ri.size() &&
+           g.col_ptr_bytes == (int)sizeof(P) &&
+           bfsx_download_csc(ctx, c.data(), r.data()) == BFSX_OK && c == cp && r == ri;
+  }
+};
+
+// A caller's nnz above col_ptr's end: refused before row_idx is read, with
+// room for the arrays and without.
+template <class P> static void wrong_nnz() {
+  Cycle<P> old(100);
+  for (uint32_t n : {1u, 5u, 1000u, 300000u}) {
+    P *cp = static_cast<P *>(fenced(sizeof(P) * (n + 1)));
+    uint32_t *ri = static_cast<uint32_t *>(fenced(4 * (size_t)n));
+    const Cycle<P> g(n);
+    memcpy(cp, g.cp.data(), sizeof(P) * (n + 1));
+    memcpy(ri, g.ri.data(), 4 * (size_t)n);
+    for (uint64_t nnz : {(uint64_t)n + 1, (uint64_t)n + 70000, (uint64_t)n + (3u << 20), (uint64_t)1 << 45})
+      for (size_t room : {(size_t)1 << 30, (size_t)0}) {
+        limit = 1u << 30;
+        CHECK(old.upload() == BFSX_OK);
+        limit = room ? room : live;
+        CHECK(bfsx_upload_csc(ctx, n, n, cp, sizeof(P), ri, nnz, 0) == BFSX_ERR_ARG);
+        CHECK(says("col_ptr end does not match nnz"));
+        CHECK(old.resident());
+      }
+    limit = 1u << 30;
+    CHECK(bfsx_upload_csc(ctx, n, n, cp, sizeof(P), ri, n, 0) == BFSX_OK);
+  }
+}
+
+int main(int argc, char **argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
+  if (what == "wrong_nnz") {
+    wrong_nnz<uint32_t>();
+    wrong_nnz<uint64_t>();
+  } else {
+    return 2;
+  }
+  bfsx_destroy(ctx);
+  ctx = nullptr;
+  if (live != 0) {
+    fprintf(stderr, "%zu bytes of device memory left\n", live);
+    return 1;
+  }
+  printf("%s ok\n", what.c_str());
+  return 0;
+}
