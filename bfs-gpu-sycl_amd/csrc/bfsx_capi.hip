@@ -53,7 +53,8 @@ void ensure(DevBuf &b, size_t bytes, bfsx_ctx *ctx) {
   size_t best = pool.spare.size();
   for (size_t i = 0; i < pool.spare.size(); i++) {
     const size_t have = pool.spare[i].bytes;
-    if (have >= bytes && have <= bytes * 2 &&
+    // (a buffer twice the size would hold memory that the next one needs)
+    if (have >= bytes && have <= bytes + bytes / 8 &&
         (best == pool.spare.size() || have < pool.spare[best].bytes))
       best = i;
   }
@@ -1170,6 +1171,8 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
     ctx->has_graph = false;
     std::swap(ctx->col_ptr, cp);
     std::swap(ctx->row_idx, ri);
+    release(cp);  // the replaced graph's arrays: the new search state may need their room
+    release(ri);
     ctx->n_cols = n_cols;
     ctx->n_rows = n_rows;
     ctx->nnz = nnz;

@@ -142,17 +142,17 @@ static void *fenced(size_t n) {
   return p + room - n;
 }
 
-// a cycle of n vertices: one entry per list
+// n vertices with k entries each: the k vertices that follow
 template <class P> struct Cycle {
   std::vector<P> cp;
   std::vector<uint32_t> ri;
-  explicit Cycle(uint32_t n) : cp(n + 1), ri(n) {
-    for (uint32_t i = 0; i <= n; i++) cp[i] = i;
-    for (uint32_t i = 0; i < n; i++) ri[i] = (i + 1) % n;
+  explicit Cycle(uint32_t n, uint32_t k = 1) : cp(n + 1), ri((size_t)n * k) {
+    for (uint32_t i = 0; i <= n; i++) cp[i] = (P)i * k;
+    for (size_t i = 0; i < ri.size(); i++) ri[i] = (uint32_t)((i / k + i % k + 1) % n);
   }
   int upload() {
-    const uint32_t n = (uint32_t)ri.size();
-    return bfsx_upload_csc(ctx, n, n, cp.data(), sizeof(P), ri.data(), n, 0);
+    const uint32_t n = (uint32_t)cp.size() - 1;
+    return bfsx_upload_csc(ctx, n, n, cp.data(), sizeof(P), ri.data(), ri.size(), 0);
   }
   // whether this is the resident graph
   bool resident() {
@@ -164,6 +164,12 @@ template <class P> struct Cycle {
            bfsx_download_csc(ctx, c.data(), r.data()) == BFSX_OK && c == cp && r == ri;
   }
 };
+
+static void reset() {
+  limit = (size_t)1 << 30;
+  bfsx_destroy(ctx);
+  if (bfsx_create(0, &ctx) != BFSX_OK) exit(2);
+}
 
 // A caller's nnz above col_ptr's end: refused before row_idx is read, with
 // room for the arrays and without.
@@ -189,12 +195,31 @@ template <class P> static void wrong_nnz() {
   }
 }
 
+// A graph that replaces another needs room for both graphs' arrays at most
+// until it is accepted, not beside its own search state.
+template <class P> static void replace() {
+  Cycle<P> old(1000, 8000), next(4000000);  // many entries; many vertices
+  CHECK(next.upload() == BFSX_OK);
+  const size_t alone = live;
+  reset();
+  CHECK(old.upload() == BFSX_OK);
+  const size_t margin = alone / 8, arrays = sizeof(P) * next.cp.size() + 4 * next.ri.size();
+  CHECK(live + arrays < alone + margin);  // both graphs fit while it is checked
+  limit = alone + margin;
+  CHECK(next.upload() == BFSX_OK);
+  CHECK(next.resident());
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
   if (what == "wrong_nnz") {
     wrong_nnz<uint32_t>();
     wrong_nnz<uint64_t>();
+  } else if (what == "replace") {
+    replace<uint32_t>();
+    reset();
+    replace<uint64_t>();
   } else {
     return 2;
   }

@@ -29,3 +29,7 @@ def check(driver, what):
 
 def test_wrong_nnz_is_refused_before_row_idx_is_read(driver):
     check(driver, "wrong_nnz")
+
+
+def test_replaced_arrays_leave_before_the_search_state_comes(driver):
+    check(driver, "replace")
