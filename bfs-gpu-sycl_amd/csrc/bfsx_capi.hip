@@ -147,7 +147,10 @@ static void drop_pull_fd(bfsx_ctx *ctx) {
   ctx->hot_n = 0;
 }
 
+// Makes the graph in col_ptr / row_idx the resident one.  Until its search
+// state stands there is none: calls after a failure in here are refused.
 static void after_graph_change(bfsx_ctx *ctx) {
+  ctx->has_graph = false;
   // edge counts travel in 48-bit fields of the level-end words
   if (ctx->nnz > MIRROR_48) fail(BFSX_ERR_ARG, "graphs above 2^48 stored edges are not supported");
   release(ctx->row_idx_pull);  // a copy of the old lists
@@ -156,6 +159,7 @@ static void after_graph_change(bfsx_ctx *ctx) {
   free_search_state(ctx);
   graph_summary(ctx);
   alloc_search_state(ctx);
+  ctx->has_graph = true;
 }
 
 static bfsx_params default_params() {
@@ -1178,7 +1182,6 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
     ctx->nnz = nnz;
     ctx->ptr_bytes = col_ptr_bytes;
     ctx->gflags = flags & BFSX_GRAPH_SYMMETRIC;
-    ctx->has_graph = true;
     after_graph_change(ctx);
   });
 }

@@ -309,7 +309,6 @@ void build_symmetric_csc(bfsx_ctx *ctx, uint32_t n, uint32_t *d_u, uint32_t *d_v
   ctx->nnz = nnz;
   ctx->ptr_bytes = ptr_bytes;
   ctx->gflags = BFSX_GRAPH_SYMMETRIC;
-  ctx->has_graph = true;
 }
 
 // ---- graph summary: max degree, isolated-vertex bitmap and count ---------

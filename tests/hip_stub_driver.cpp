@@ -210,6 +210,43 @@ template <class P> static void replace() {
   CHECK(next.resident());
 }
 
+// Memory that ends at any of the allocations of a new graph's search state:
+// afterwards there is no graph, and no call launches anything on one.
+static void state_oom() {
+  Cycle<uint32_t> old(100), next(500000);
+  CHECK(next.upload() == BFSX_OK);
+  const size_t alone = live;
+  int failed = 0;
+  for (size_t room = 1 << 20; room < alone + (alone >> 2); room += 100000) {
+    reset();
+    CHECK(old.upload() == BFSX_OK);
+    limit = room > live ? room : live;
+    const int rc = next.upload();
+    if (rc == BFSX_OK) {
+      CHECK(next.resident());
+      continue;
+    }
+    CHECK(rc == BFSX_ERR_NOMEM);
+    bfsx_graph_info g;
+    if (bfsx_graph_info_get(ctx, &g) == BFSX_OK) {  // (failed before the old one was given up)
+      CHECK(old.resident());
+      continue;
+    }
+    failed++;
+    const size_t before = launches;
+    std::vector<int32_t> lev(next.ri.size());
+    bfsx_run_stats st;
+    for (int strategy : {BFSX_LLB, BFSX_GLB, BFSX_LEARNED, BFSX_BEAMER})
+      CHECK(bfsx_run(ctx, 0, strategy, 0, lev.data(), nullptr, &st) == BFSX_ERR_STATE);
+    CHECK(bfsx_order_adjacency(ctx, BFSX_ORDER_PULL_HUB_FIRST) == BFSX_ERR_STATE);
+    CHECK(launches == before);
+    limit = (size_t)1 << 30;
+    CHECK(next.upload() == BFSX_OK);
+    CHECK(next.resident());
+  }
+  CHECK(failed > 5);
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
@@ -220,6 +257,8 @@ int main(int argc, char **argv) {
     replace<uint32_t>();
     reset();
     replace<uint64_t>();
+  } else if (what == "state_oom") {
+    state_oom();
   } else {
     return 2;
   }

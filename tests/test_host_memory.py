@@ -33,3 +33,7 @@ def test_wrong_nnz_is_refused_before_row_idx_is_read(driver):
 
 def test_replaced_arrays_leave_before_the_search_state_comes(driver):
     check(driver, "replace")
+
+
+def test_no_graph_after_a_failure_to_allocate_its_search_state(driver):
+    check(driver, "state_oom")
