@@ -1274,6 +1274,18 @@ int bfsx_order_adjacency(bfsx_ctx *ctx, int order) {
       fail(BFSX_ERR_ARG,
            "order must be BFSX_ORDER_ID, BFSX_ORDER_HUB_FIRST or BFSX_ORDER_PULL_HUB_FIRST");
     if (order == BFSX_ORDER_PULL_HUB_FIRST) {
+      // (bottom-up steps and batches use whatever of the copy is there: one
+      // that a failure leaves unfinished goes, whole)
+      struct Copy {
+        bfsx_ctx *ctx;
+        bool whole;
+        ~Copy() {
+          if (whole) return;
+          release(ctx->row_idx_pull);
+          drop_pull_fd(ctx);
+          ctx->gflags &= ~BFSX_GRAPH_PULL_COPY;
+        }
+      } copy{ctx, false};
       ensure(ctx->row_idx_pull, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), ctx);
       DevBuf by_degree, hrank;  // the vertices, largest degree first; hub indexes
       struct Releaser {
@@ -1291,6 +1303,7 @@ int bfsx_order_adjacency(bfsx_ctx *ctx, int order) {
       }
       build_hot_copy(ctx, by_degree.as<uint32_t>());
       ctx->gflags |= BFSX_GRAPH_PULL_COPY;
+      copy.whole = true;
       return;
     }
     release(ctx->row_idx_pull);

@@ -247,6 +247,40 @@ static void state_oom() {
   CHECK(failed > 5);
 }
 
+// Memory held by the context's arrays, without its spare buffers (which it
+// gives back when an allocation fails).
+static size_t held() {
+  limit = live;
+  double ms;
+  CHECK(bfsx_stream_copy(ctx, 1 << 26, 1, &ms) == BFSX_ERR_NOMEM);
+  return live;
+}
+
+// An ordering that fails on its way leaves nothing of the bottom-up copy.
+static void order_oom() {
+  Cycle<uint32_t> g(200000, 3);
+  CHECK(g.upload() == BFSX_OK);
+  const size_t plain = held();
+  int failed = 0;
+  for (size_t room = 0; room < 12u << 20; room += 250000) {
+    reset();
+    CHECK(g.upload() == BFSX_OK);
+    CHECK(held() == plain);
+    limit = live + room;
+    // (also with memory to spare: the kernels do nothing here, so that the
+    // copy's counts do not agree)
+    CHECK(bfsx_order_adjacency(ctx, BFSX_ORDER_PULL_HUB_FIRST) != BFSX_OK);
+    failed += says("hipMalloc");
+    bfsx_graph_info i;
+    CHECK(bfsx_graph_info_get(ctx, &i) == BFSX_OK);
+    CHECK(!(i.flags & BFSX_GRAPH_PULL_COPY) && i.pull_hubs == 0 && i.hot_vertices == 0);
+    limit = (size_t)1 << 30;
+    CHECK(g.resident());
+    CHECK(held() <= plain + (1 << 16));  // (the checks' scratch)
+  }
+  CHECK(failed > 5);
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
@@ -259,6 +293,8 @@ int main(int argc, char **argv) {
     replace<uint64_t>();
   } else if (what == "state_oom") {
     state_oom();
+  } else if (what == "order_oom") {
+    order_oom();
   } else {
     return 2;
   }

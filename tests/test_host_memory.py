@@ -37,3 +37,7 @@ def test_replaced_arrays_leave_before_the_search_state_comes(driver):
 
 def test_no_graph_after_a_failure_to_allocate_its_search_state(driver):
     check(driver, "state_oom")
+
+
+def test_nothing_of_a_bottom_up_copy_stays_after_a_failure(driver):
+    check(driver, "order_oom")
