@@ -478,7 +478,9 @@ __device__ __forceinline__ void llb_tile(const KArgs &a, LlbShared<PtrT, WG> &sh
       const uint32_t slot = s_hub[h];
       const PtrT b = s_start[slot];
       const PtrT len = col_ptr[s_v[slot] + 1] - b;
-      for (PtrT e = l + 64 * part; e < len; e += 64 * n_parts)
+      // (64 bits: a stride past the end of a list of nearly 2^32 entries must
+      // not come back to its start)
+      for (uint64_t e = l + 64 * part; e < len; e += 64 * n_parts)
         discover<PtrT, HOT>(a, col_ptr, a.row_idx[b + e], s_v[slot], dacc);
     }
   }

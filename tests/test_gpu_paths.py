@@ -527,3 +527,22 @@ def test_list_beyond_32_bits(engine):
             assert lev.tolist() == want, s
             assert st["edges_count"] == length + 3 and st["reached"] == 6, s
             assert par[1:].tolist() == [0, 1, 1, 2, 3], s
+
+
+# 4-byte offsets and a hub's list (17 GB) that ends less than a stride of the
+# groups sharing it below 2^32
+def test_hub_list_near_32_bits(engine):
+    import bfsx
+    length = 2 ** 32 - 3000
+    cp = np.array([0, 1, 1 + length, 2 + length, 3 + length, 3 + length, 3 + length], np.uint32)
+    ri = np.zeros(length + 3, np.uint32)
+    ri[[0, 1001, length, 1 + length, 2 + length]] = [1, 2, 3, 4, 5]
+    with bfsx.Engine(0) as eng:
+        eng.upload_csc(cp, ri)
+        del ri
+        for s, mark in (("llb", 4), ("slb", 0xFFFFFFFF)):
+            say("long hub", s, mark)
+            eng.set_params(hub_degree=1024, mark_ratio_q10=mark)
+            lev, st = eng.run(0, s)
+            assert lev.tolist() == [0, 1, 2, 2, 3, 3], s
+            assert st["edges_count"] == length + 3, s
