@@ -2801,8 +2801,8 @@ template <typename PtrT, bool STRIDED, bool HOT>
 static void launch_llb_t(bfsx_ctx *ctx, const KArgs &a, unsigned long long EF) {
   const uint32_t wg = ctx->params.llb_wg;
   const uint32_t tiles = (uint32_t)(((uint64_t)a.F + wg - 1) / wg);
-  const uint32_t parts = llb_parts(EF, tiles, wg);
-  const dim3 grid(tiles * parts);  // (below 2^26 tiles of 64; parts follow the edges)
+  const uint32_t parts = launch_parts(llb_parts(EF, tiles, wg), tiles, wg);
+  const dim3 grid(tiles * parts);
   hipStream_t s = ctx->stream;
   switch (wg) {
     case 64: hipLaunchKernelGGL((k_llb<PtrT, 64, STRIDED, HOT>), grid, dim3(64), 0, s, a, tiles, parts); break;

@@ -92,6 +92,14 @@ constexpr unsigned long long MIRROR_48 = (1ull << 48) - 1;
 constexpr uint32_t MIRROR_LEVEL_MASK = (1u << 23) - 1;
 constexpr uint32_t MIRROR_KIND_MASK = (1u << 24) - 1;
 
+// The parts per tile that one launch of wg threads per part can hold: a
+// launch holds fewer than 2^32 threads (frontiers of 10^9 vertices with dozens
+// of edges each would pass that).
+inline uint32_t launch_parts(uint32_t parts, uint32_t tiles, uint32_t wg) {
+  const uint64_t fit = 0xFFFFFFFFull / ((uint64_t)tiles * wg);
+  return parts <= fit ? parts : fit ? (uint32_t)fit : 1u;
+}
+
 // Whether a top-down level marks and compacts or discovers exact-once.  A
 // level marks from hi_E frontier edges on, and from lo_E on when its
 // frontier averages at least MARK_MIN_AVG_DEGREE edges per vertex.  Many

@@ -15,7 +15,7 @@
 #include <string>
 #include <vector>
 
-#include "bfsx.h"
+#include "bfsx_internal.hpp"
 
 // ---- the stand-in --------------------------------------------------------------
 static std::mutex mu;
@@ -181,7 +181,8 @@ template <class P> static void wrong_nnz() {
     const Cycle<P> g(n);
     memcpy(cp, g.cp.data(), sizeof(P) * (n + 1));
     memcpy(ri, g.ri.data(), 4 * (size_t)n);
-    for (uint64_t nnz : {(uint64_t)n + 1, (uint64_t)n + 70000, (uint64_t)n + (3u << 20), (uint64_t)1 << 45})
+    for (uint64_t nnz : {(uint64_t)n + 1, (uint64_t)n + 70000, (uint64_t)n + (3u << 20),
+                         (uint64_t)1 << 45})
       for (size_t room : {(size_t)1 << 30, (size_t)0}) {
         limit = 1u << 30;
         CHECK(old.upload() == BFSX_OK);
@@ -281,6 +282,21 @@ static void order_oom() {
   CHECK(failed > 5);
 }
 
+// Tiles shared by groups: every part the rule wants while they fit a launch.
+static void launch_size() {
+  for (uint32_t wg = 64; wg <= 1024; wg *= 2)
+    for (uint64_t F : {1ull, 255ull, 1ull << 20, 1000000007ull, 1100000000ull, 2147483647ull,
+                       2147483649ull, 4294967295ull - 1024})
+      for (uint32_t parts : {1u, 2u, 3u, 4u, 5u, 63u, 64u}) {
+        const uint32_t tiles = (uint32_t)((F + wg - 1) / wg);
+        const uint32_t got = bfsx::launch_parts(parts, tiles, wg);
+        const uint64_t tile_threads = (uint64_t)tiles * wg;
+        CHECK(got >= 1 && got <= parts);
+        CHECK(got * tile_threads < 1ull << 32);
+        CHECK(got == parts || (got + 1) * tile_threads >= 1ull << 32);
+      }
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
@@ -295,6 +311,8 @@ int main(int argc, char **argv) {
     state_oom();
   } else if (what == "order_oom") {
     order_oom();
+  } else if (what == "launch_size") {
+    launch_size();
   } else {
     return 2;
   }

@@ -15,7 +15,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 def driver(tmp_path_factory):
     out = tmp_path_factory.mktemp("stub") / "hip_stub_driver"
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__", "-rdynamic",
-                    "-I", os.path.join(ROOT, "include"), "-isystem", os.path.join(ROCM, "include"),
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(PKG, "csrc"),
+                    "-isystem", os.path.join(ROCM, "include"),
                     os.path.join(ROOT, "tests", "hip_stub_driver.cpp"), "-o", str(out), "-L", PKG,
                     "-lbfsx", f"-Wl,-rpath,{PKG}", f"-Wl,-rpath-link,{os.path.join(ROCM, 'lib')}"],
                    check=True)
@@ -41,3 +42,7 @@ def test_no_graph_after_a_failure_to_allocate_its_search_state(driver):
 
 def test_nothing_of_a_bottom_up_copy_stays_after_a_failure(driver):
     check(driver, "order_oom")
+
+
+def test_shared_tiles_fit_a_launch(driver):
+    check(driver, "launch_size")
