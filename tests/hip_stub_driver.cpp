@@ -297,6 +297,37 @@ static void launch_size() {
       }
 }
 
+// No room for a graph beside the resident one: it is checked on the host,
+// refused with the resident one kept, or takes its place.
+template <class P> static void no_room() {
+  Cycle<P> old(300000, 20);
+  const Cycle<P> good(250000, 22);
+  CHECK(old.upload() == BFSX_OK);
+  limit = live + (1u << 16);
+  auto refused = [&](Cycle<P> g, const char *text) {
+    CHECK(g.upload() == BFSX_ERR_ARG);
+    CHECK(says(text));
+    CHECK(old.resident());
+  };
+  for (uint32_t at : {1u, 125000u, 249999u}) {
+    Cycle<P> g(good);
+    g.cp[at] = (P)g.ri.size() + 5;
+    refused(g, "col_ptr is not monotone");
+    g = good;
+    g.ri[at] = 250000;
+    refused(g, "row_idx entry >= n_cols");
+  }
+  Cycle<P> g(good);
+  g.ri.back() = 0xFFFFFFFFu;
+  refused(g, "row_idx entry >= n_cols");
+  g = good;
+  g.ri.pop_back();
+  refused(g, "col_ptr end does not match nnz");
+  g = good;
+  CHECK(g.upload() == BFSX_OK);
+  CHECK(g.resident());
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
@@ -313,6 +344,10 @@ int main(int argc, char **argv) {
     order_oom();
   } else if (what == "launch_size") {
     launch_size();
+  } else if (what == "no_room") {
+    no_room<uint32_t>();
+    reset();
+    no_room<uint64_t>();
   } else {
     return 2;
   }

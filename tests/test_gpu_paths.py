@@ -546,3 +546,61 @@ def test_hub_list_near_32_bits(engine):
             lev, st = eng.run(0, s)
             assert lev.tolist() == [0, 1, 2, 2, 3, 3], s
             assert st["edges_count"] == length + 3, s
+
+
+# the ring wraps: more batches than it has slots, for levels of one byte (four
+# pieces a batch) and of two (two), into destinations at any 4-byte offset
+@pytest.mark.parametrize("depth", [200, 60000])
+@pytest.mark.parametrize("offset", [0, 37])
+def test_ring_wraps(engine, depth, offset):
+    import ctypes as C
+    import os
+    import re
+
+    import bfsx
+    head = open(os.path.join(bfsx.HERE, "csrc", "bfsx_internal.hpp")).read()
+    mib = int(re.search(r"RING_PIECE_BYTES = (\d+)u << 20", head).group(1))
+    slots = int(re.search(r"RING_SLOTS = (\d+);", head).group(1))
+    per_batch = 4 if depth < 255 else 2
+    n = (slots * per_batch + 3 * per_batch // 2) * (mib << 20) // 4 + 4091
+    say("ring wraps", depth, offset, n)
+    # a path spread over all ids, its first vertex next to a third of the others
+    step = n // (depth + 1)
+    path = np.arange(depth + 1) * step
+    leaf = np.arange(1, n, 3)
+    leaf = leaf[(leaf % step != 0) | (leaf > path[-1])]
+    deg = np.zeros(n, np.int64)
+    deg[path[:-1]] = 1
+    deg[0] += len(leaf)
+    cp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    ri = np.concatenate([leaf, path[1:]]).astype(np.uint32)
+    want = np.full(n, -1, np.int32)
+    want[leaf] = 1
+    want[path] = np.arange(depth + 1)
+    engine.upload_csc(cp, ri)
+    got_cp, got_ri = engine.download_csc()
+    assert np.array_equal(got_cp, cp) and np.array_equal(got_ri, ri)
+    room = np.full(n + offset + 100, 12345, np.int32)
+    for _ in range(2):
+        room[:] = 12345
+        st = bfsx.RunStats()
+        rc = bfsx.lib().bfsx_run(engine._h, 0, 0, 0, room[offset:].ctypes.data, None, C.byref(st))
+        assert rc == 0 and st.max_level == depth
+        assert np.array_equal(room[offset:offset + n], want)
+        assert (room[:offset] == 12345).all() and (room[offset + n:] == 12345).all()
+
+
+# the histogram that is added up in memory, on the same graphs as in LDS
+@pytest.mark.parametrize("name", ["one", "3", "4", "257", "4096", "4099", "20001", "path2500",
+                                  "star70001", "directed4099"])
+def test_level_histogram_edges_in_memory(engine, name):
+    say("histogram in memory", name)
+    cp, ri, n_rows, sym, root = some_graph(name)
+    engine.upload_csc(cp, ri, n_rows=n_rows, symmetric=sym)
+    want, _, _ = cpu.bfs_queue(cp, ri, root, n_rows=n_rows)
+    deg = np.where(np.arange(len(want)) < n_rows, np.diff(cp.astype(np.int64)), 0)
+    engine.run(root, "llb")
+    for size in (4097, 20000):
+        counts, edges = engine.level_histogram(size)
+        assert (counts == np.bincount(want[want >= 0])).all()
+        assert (edges == np.bincount(want[want >= 0], weights=deg[want >= 0])).all()

@@ -46,3 +46,7 @@ def test_nothing_of_a_bottom_up_copy_stays_after_a_failure(driver):
 
 def test_shared_tiles_fit_a_launch(driver):
     check(driver, "launch_size")
+
+
+def test_upload_without_room_for_both_graphs(driver):
+    check(driver, "no_room")
