@@ -472,21 +472,26 @@ __global__ void k_ranks(const uint64_t *sorted, uint32_t n, uint64_t mask, uint3
 }
 
 // key of edge e in column c: (c << B) | rank(row_idx[e]).  A work-group takes
-// EDGE_RUN consecutive edges whatever columns they belong to: two waves search
-// the first and the last column, the offsets between go to LDS, and every
+// `run` consecutive edges whatever columns they belong to: two waves search
+// the first and the last column (64 candidates at a time: what bounds a small
+// graph is that chain of reads), the offsets between go to LDS, and every
 // edge finds its column there.  (With a wave per column, the longest list set
 // the time: 339 us for 16 M edges and 1 M vertices, 129 now, most of it the
-// random reads of the ranks.)
-constexpr uint32_t EDGE_RUN = 4096, EDGE_RUN_COLS = 4096;
+// random reads of the ranks.)  Runs are EDGE_RUN edges, and shorter, down to
+// an edge per thread, on graphs that would leave CUs without one.  Sorting by
+// id / hub first, whole call, us: runs of 4096 and a search by halves R-MAT 8
+// 38 / 57, 12 54 / 75, 16 130 / 179; now 29 / 49, 41 / 61, 120 / 166; a wave
+// per column 32 / 54, 43 / 67, 235 / 270.
+constexpr uint32_t EDGE_RUN = 4096, EDGE_RUN_MIN = 256, EDGE_RUN_COLS = 4096;
 template <typename PtrT>
 __global__ __launch_bounds__(256) void k_edge_rank_keys(const PtrT *col_ptr, uint32_t n_cols,
                                                         const uint32_t *row_idx, uint64_t nnz,
-                                                        const uint32_t *rank, int B,
+                                                        uint32_t run, const uint32_t *rank, int B,
                                                         uint64_t *keys) {
   __shared__ uint32_t s_end[EDGE_RUN_COLS];  // end of each column, from the run's first edge
   __shared__ uint32_t s_col[2];
-  const uint64_t e0 = blockIdx.x * (uint64_t)EDGE_RUN;
-  const uint32_t m = (uint32_t)(nnz - e0 < EDGE_RUN ? nnz - e0 : EDGE_RUN);
+  const uint64_t e0 = blockIdx.x * (uint64_t)run;
+  const uint32_t m = (uint32_t)(nnz - e0 < run ? nnz - e0 : run);
   // column of edge e: the first one that ends after it
   auto column = [&](uint64_t e) {
     uint32_t lo = 0, hi = n_cols - 1;
@@ -499,8 +504,17 @@ __global__ __launch_bounds__(256) void k_edge_rank_keys(const PtrT *col_ptr, uin
   };
   const uint32_t w = threadIdx.x >> 6;
   if (w < 2) {
-    const uint32_t c = column(w == 0 ? e0 : e0 + m - 1);
-    if ((threadIdx.x & 63) == 0) s_col[w] = c;
+    const uint64_t e = w == 0 ? e0 : e0 + m - 1;
+    const uint32_t lane = threadIdx.x & 63;
+    uint64_t lo = 0, hi = n_cols - 1;
+    while (lo < hi) {  // (uniform over the wave)
+      const uint64_t step = (hi - lo + 63) / 64, c = lo + lane * step;
+      const unsigned long long after = __ballot(c >= hi || (uint64_t)col_ptr[c + 1] > e);
+      const uint32_t f = after ? (uint32_t)__ffsll(after) - 1 : 64u;  // the first that ends after e
+      if (f < 64 && lo + f * step < hi) hi = lo + f * step;
+      if (f > 0) lo += (f - 1) * step + 1;
+    }
+    if (lane == 0) s_col[w] = (uint32_t)lo;
   }
   __syncthreads();
   const uint32_t c0 = s_col[0], nc = s_col[1] - c0 + 1;
@@ -578,9 +592,12 @@ static void order_adjacency_t(bfsx_ctx *ctx, bool hub_first, uint32_t *out, DevB
   }
   if (nnz) {
     ensure(keys, sizeof(uint64_t) * nnz, ctx);
-    // (nnz > 0: there are columns; the grid is below 2^31 groups up to 2^43 edges)
-    hipLaunchKernelGGL(k_edge_rank_keys<PtrT>, dim3((unsigned)((nnz + EDGE_RUN - 1) / EDGE_RUN)),
-                       dim3(256), 0, s, cp, n, ctx->row_idx.as<uint32_t>(), nnz,
+    uint32_t run = EDGE_RUN;
+    while (run > EDGE_RUN_MIN && nnz < (uint64_t)run * ctx->cu_count) run /= 2;
+    // (nnz > 0: there are columns; a launch holds the 2^24 groups of up to
+    // 2^36 edges, whose keys alone would be a terabyte)
+    hipLaunchKernelGGL(k_edge_rank_keys<PtrT>, dim3((unsigned)((nnz + run - 1) / run)),
+                       dim3(256), 0, s, cp, n, ctx->row_idx.as<uint32_t>(), nnz, run,
                        hub_first ? rank.as<uint32_t>() : (const uint32_t *)nullptr, B,
                        keys.as<uint64_t>());
     BFSX_HIP(hipGetLastError());

@@ -604,3 +604,25 @@ def test_level_histogram_edges_in_memory(engine, name):
         counts, edges = engine.level_histogram(size)
         assert (counts == np.bincount(want[want >= 0])).all()
         assert (edges == np.bincount(want[want >= 0], weights=deg[want >= 0])).all()
+
+
+# adjacency orders by runs of 256 edges (small graphs) up to 4096, the search
+# for a run's columns over few and many of them
+@pytest.mark.parametrize("m", [1, 255, 257, 65537, 131071, 300007, 1048575, 1048577, 1500001])
+@pytest.mark.parametrize("n", [2, 64, 65, 66, 4097, 40011])
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+def test_order_adjacency_run_lengths(engine, m, n, ptr):
+    say("runs", m, n, ptr.__name__)
+    rng = np.random.default_rng(m + n)
+    col = np.sort((rng.random(m) ** 2 * n).astype(np.int64))
+    ri = rng.integers(0, n, m).astype(np.uint32)
+    deg = np.bincount(col, minlength=n)
+    cp = np.concatenate([[0], np.cumsum(deg)]).astype(ptr)
+    rank = np.empty(n, np.int64)
+    rank[np.lexsort((np.arange(n), -deg))] = np.arange(n)
+    for order in ("hub_first", "id"):
+        engine.upload_csc(cp, ri)
+        engine.order_adjacency(order)
+        got_cp, got = engine.download_csc()
+        key = rank[ri] if order == "hub_first" else ri
+        assert np.array_equal(got_cp, cp) and np.array_equal(got, ri[np.lexsort((key, col))])
