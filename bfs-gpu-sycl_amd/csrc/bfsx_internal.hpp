@@ -438,9 +438,13 @@ void gen_rmat_pairs_offset(bfsx_ctx *ctx, int scale, uint64_t m, uint32_t tA, ui
 
 // ---- host transfers (bfsx_transfer.hip) ------------------------------------
 // Copies between the card and the caller's memory, after all work queued on
-// the context's stream; they return when the copy is done.
-void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes);
+// the context's stream; they return when the copy is done.  after_search: the
+// stream holds a search's launches.
+void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes, bool after_search = false);
 void copy_in(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes);
+// two arrays; small ones with one wait
+void copy_in_both(bfsx_ctx *ctx, void *dst0, const void *src0, size_t bytes0, void *dst1,
+                  const void *src1, size_t bytes1);
 // n levels, none above max_level
 void copy_levels_out(bfsx_ctx *ctx, int32_t *dst, const int32_t *levels, uint32_t n,
                      uint32_t max_level);

@@ -24,6 +24,14 @@ namespace bfsx {
 namespace {
 
 constexpr size_t PIECE = RING_PIECE_BYTES;  // host bytes of a piece; a slot holds one
+// Copies of up to SMALL host bytes go through the ring whole, as one transfer
+// and a wait (to / from the card, us: 16 KB 12 / 12, 128 KB 11 / 14, 512 KB 24
+// / 30; the runtime's copy of pageable memory takes 18 / 26, 59 / 61 and 35 /
+// 32 until some 16 MB have warmed its buffers, 12 / 12 to 26 / 30 then).  They
+// wait for the stream; after a search for an event, which takes 7 us more
+// from 32 KB on but leaves the bookkeeping of the search's launches, some 20
+// us, to a later call (R-MAT-like graph of 10^4 edges, levels: 131 -> 110).
+constexpr size_t SMALL = PIECE / 4;
 constexpr int MAX_HELPERS = 3;              // threads that move pieces beside the caller's
 constexpr uint64_t HELP_PIECES = 3;         // copies of fewer pieces: the caller's thread alone
 
@@ -170,7 +178,18 @@ bool known_memory(const void *p) {
 // of an R-MAT 22 search's levels took 215 us instead of 150).
 template <class Issue, class Take>
 void stream_out(bfsx_ctx *ctx, const void *dst, uint64_t items, size_t width, size_t ring_width,
-                Issue issue, Take take) {
+                bool after_search, Issue issue, Take take) {
+  if (items * width <= SMALL) {
+    issue(0, items, 0);
+    if (after_search) {
+      BFSX_HIP(hipEventRecord(ctx->ring_ev[0], ctx->stream));
+      BFSX_HIP(hipEventSynchronize(ctx->ring_ev[0]));
+    } else {
+      BFSX_HIP(hipStreamSynchronize(ctx->stream));
+    }
+    take(0, items, ctx->ring);
+    return;
+  }
   const Pieces P(dst, items, width);
   const uint64_t B = std::max<uint64_t>(1, std::min<uint64_t>(P.n / 4, width / ring_width));
   const uint64_t batches = (P.n + B - 1) / B;
@@ -202,7 +221,7 @@ void stream_out(bfsx_ctx *ctx, const void *dst, uint64_t items, size_t width, si
 
 }  // namespace
 
-void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes) {
+void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes, bool after_search) {
   if (bytes == 0) return;
   if (known_memory(dst)) {
     BFSX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -210,7 +229,7 @@ void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes) {
     return;
   }
   stream_out(
-      ctx, dst, bytes, 1, 1,
+      ctx, dst, bytes, 1, 1, after_search,
       [&](uint64_t first, uint64_t n, size_t at) {
         BFSX_HIP(hipMemcpyAsync(ctx->ring + at, static_cast<const uint8_t *>(src) + first, n,
                                 hipMemcpyDeviceToHost, ctx->stream));
@@ -224,11 +243,11 @@ void copy_levels_out(bfsx_ctx *ctx, int32_t *dst, const int32_t *levels, uint32_
                      uint32_t max_level) {
   const int width = max_level < 255 ? 1 : max_level < 65535 ? 2 : 4;
   if (width == 4 || known_memory(dst)) {
-    copy_out(ctx, dst, levels, sizeof(int32_t) * (size_t)n);
+    copy_out(ctx, dst, levels, sizeof(int32_t) * (size_t)n, true);
     return;
   }
   stream_out(
-      ctx, dst, n, sizeof(int32_t), width,
+      ctx, dst, n, sizeof(int32_t), width, true,
       [&](uint64_t first, uint64_t k, size_t at) {
         const dim3 grid((unsigned)((k + 2047) / 2048)), block(256);
         if (width == 1)
@@ -244,10 +263,29 @@ void copy_levels_out(bfsx_ctx *ctx, int32_t *dst, const int32_t *levels, uint32_
       });
 }
 
+// A copy of known memory, or of up to SMALL bytes through slot `at` of the
+// ring, is queued here; the caller waits for it.
+static bool queue_in(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes, int at) {
+  const void *from = src;
+  if (!known_memory(src)) {
+    if (bytes > SMALL) return false;
+    from = std::memcpy(ctx->ring + at * PIECE, src, bytes);
+  }
+  BFSX_HIP(hipMemcpyAsync(dst, from, bytes, hipMemcpyHostToDevice, ctx->stream));
+  return true;
+}
+
+void copy_in_both(bfsx_ctx *ctx, void *dst0, const void *src0, size_t bytes0, void *dst1,
+                  const void *src1, size_t bytes1) {
+  if (bytes0 && !queue_in(ctx, dst0, src0, bytes0, 0)) copy_in(ctx, dst0, src0, bytes0);
+  const bool queued = !bytes1 || queue_in(ctx, dst1, src1, bytes1, 1);
+  BFSX_HIP(hipStreamSynchronize(ctx->stream));  // (before the ring is used again)
+  if (!queued) copy_in(ctx, dst1, src1, bytes1);
+}
+
 void copy_in(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
-  if (bytes <= PIECE / 4 || known_memory(src)) {  // (the runtime copies small ones at once)
-    BFSX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+  if (queue_in(ctx, dst, src, bytes, 0)) {
     BFSX_HIP(hipStreamSynchronize(ctx->stream));
     return;
   }

@@ -182,7 +182,7 @@ template <class P> static void wrong_nnz() {
     memcpy(cp, g.cp.data(), sizeof(P) * (n + 1));
     memcpy(ri, g.ri.data(), 4 * (size_t)n);
     for (uint64_t nnz : {(uint64_t)n + 1, (uint64_t)n + 70000, (uint64_t)n + (3u << 20),
-                         (uint64_t)1 << 45})
+                         (uint64_t)1 << 45, ((uint64_t)1 << 62) + n})
       for (size_t room : {(size_t)1 << 30, (size_t)0}) {
         limit = 1u << 30;
         CHECK(old.upload() == BFSX_OK);

@@ -626,3 +626,42 @@ def test_order_adjacency_run_lengths(engine, m, n, ptr):
         got_cp, got = engine.download_csc()
         key = rank[ri] if order == "hub_first" else ri
         assert np.array_equal(got_cp, cp) and np.array_equal(got, ri[np.lexsort((key, col))])
+
+
+# arrays of up to 256 KB are checked on the host, larger ones on the card
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+@pytest.mark.parametrize("nnz", [65535, 65536, 65537])
+def test_refused_graphs_where_the_check_moves(engine, ptr, nnz):
+    test_refused_graphs(engine, ptr, nnz)
+
+
+# copies of up to 512 KB go whole, larger ones in pieces: levels, parents and
+# graphs around that, small arrays of a graph together, destinations that
+# straddle two of the ring's pages
+@pytest.mark.parametrize("n", [3, 32766, 32767, 65535, 131071, 131072, 131073, 150001])
+@pytest.mark.parametrize("ptr", [np.uint32, np.uint64])
+def test_small_transfers(engine, n, ptr):
+    import ctypes as C
+
+    import bfsx
+    say("small transfers", n, ptr.__name__)
+    rng = np.random.default_rng(n)
+    src, dst = rng.integers(0, n, n), rng.integers(0, n, n)
+    cp, ri = csc_from_edges(n, *symmetrize(src, dst), dtype=ptr)
+    engine.upload_csc(cp, ri, symmetric=True)
+    got_cp, got_ri = engine.download_csc()
+    assert np.array_equal(got_cp, cp) and np.array_equal(got_ri, ri)
+    root = int(np.argmax(np.diff(cp.astype(np.int64))))
+    want, ec, _ = cpu.bfs_queue(cp, ri, root)
+    page = 2 << 20
+    room = np.zeros(4 * page, np.uint8)
+    edge = -room.ctypes.data % page + page  # (a page boundary inside)
+    for at in (edge, edge - 4, edge - 2 * n // 4 * 4):
+        lev = room[at:at + 4 * n].view(np.int32)
+        par = np.empty(n + 1, np.uint32)[1:]
+        st = bfsx.RunStats()
+        room[:] = 7
+        rc = bfsx.lib().bfsx_run(engine._h, root, 0, 0, lev.ctypes.data, par.ctypes.data, C.byref(st))
+        assert rc == 0 and st.edges_count == ec and np.array_equal(lev, want)
+        assert (room[:at] == 7).all() and (room[at + 4 * n:] == 7).all()
+        assert cpu.check_parents(cp, ri, root, want, par) == 0
