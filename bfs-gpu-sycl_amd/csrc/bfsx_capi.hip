@@ -1050,8 +1050,7 @@ int bfsx_create(int device, bfsx_ctx **out) {
                            hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(ctx->h_mirror, 0, sizeof(LevelMirror) * MIRROR_SLOTS);
     BFSX_HIP(hipHostGetDevicePointer((void **)&ctx->d_mirror, ctx->h_mirror, 0));
-    BFSX_HIP(hipHostMalloc((void **)&ctx->ring, RING_PIECE_BYTES * RING_SLOTS, hipHostMallocMapped));
-    BFSX_HIP(hipHostGetDevicePointer((void **)&ctx->ring_dev, ctx->ring, 0));
+    take_ring(ctx);
     for (hipEvent_t &e : ctx->ring_ev)
       BFSX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     ctx->params = default_params();
@@ -1082,7 +1081,7 @@ void bfsx_destroy(bfsx_ctx *ctx) {
   ctx->pool.drop();
   if (ctx->h_ctl) (void)hipHostFree(ctx->h_ctl);
   if (ctx->h_mirror) (void)hipHostFree(ctx->h_mirror);
-  if (ctx->ring) (void)hipHostFree(ctx->ring);
+  give_ring(ctx);
   for (hipEvent_t e : ctx->ring_ev)
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : {ctx->ev0, ctx->ev1, ctx->ev_step0, ctx->ev_step1, ctx->ev_k0, ctx->ev_k1})

@@ -437,6 +437,10 @@ void gen_rmat_pairs_offset(bfsx_ctx *ctx, int scale, uint64_t m, uint32_t tA, ui
                            uint32_t offset, uint32_t *d_u, uint32_t *d_v);
 
 // ---- host transfers (bfsx_transfer.hip) ------------------------------------
+// The context's ring of pinned buffers, from its creation to its end (the
+// stream idle).
+void take_ring(bfsx_ctx *ctx);
+void give_ring(bfsx_ctx *ctx);
 // Copies between the card and the caller's memory, after all work queued on
 // the context's stream; they return when the copy is done.  after_search: the
 // stream holds a search's launches.

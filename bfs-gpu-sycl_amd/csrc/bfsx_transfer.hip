@@ -15,7 +15,9 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <thread>
+#include <utility>
 
 #include "bfsx_internal.hpp"
 
@@ -146,6 +148,16 @@ class Crew {
   std::exception_ptr error_;
 };
 
+// A closed context's ring, one per device, kept for the next context (a second
+// one is freed): pinning 16 MB and the first touches of its pages cost a
+// program that makes a context per graph 1 to 3 ms for each.  Context, upload,
+// search and close, us: 5 K vertices and 30 K edges 1500-1740 -> 700-890, 700 K
+// and 4 M 4200-4500 -> 1900-3400 (the spread is the driver's: device memory
+// freed just before is slow to come back).
+constexpr int RING_DEVICES = 64;
+std::mutex spare_mu;
+uint8_t *spare_ring[RING_DEVICES];
+
 // Pieces of `items` items of `width` bytes each at host address p: whole
 // PIECE-sized pages of it (cut at multiples of 64 items).
 struct Pieces {
@@ -220,6 +232,29 @@ void stream_out(bfsx_ctx *ctx, const void *dst, uint64_t items, size_t width, si
 }
 
 }  // namespace
+
+void take_ring(bfsx_ctx *ctx) {
+  uint8_t *p = nullptr;
+  if (ctx->device < RING_DEVICES) {
+    std::lock_guard<std::mutex> g(spare_mu);
+    std::swap(p, spare_ring[ctx->device]);
+  }
+  // (a device reset in between has taken it away)
+  if (p && !known_memory(p)) p = nullptr;
+  if (!p) BFSX_HIP(hipHostMalloc((void **)&p, RING_PIECE_BYTES * RING_SLOTS, hipHostMallocMapped));
+  ctx->ring = p;
+  BFSX_HIP(hipHostGetDevicePointer((void **)&ctx->ring_dev, p, 0));
+}
+
+void give_ring(bfsx_ctx *ctx) {
+  uint8_t *p = ctx->ring;
+  ctx->ring = ctx->ring_dev = nullptr;
+  if (p && ctx->device < RING_DEVICES) {
+    std::lock_guard<std::mutex> g(spare_mu);
+    if (!spare_ring[ctx->device]) std::swap(p, spare_ring[ctx->device]);
+  }
+  if (p) (void)hipHostFree(p);
+}
 
 void copy_out(bfsx_ctx *ctx, void *dst, const void *src, size_t bytes, bool after_search) {
   if (bytes == 0) return;

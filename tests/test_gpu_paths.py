@@ -665,3 +665,42 @@ def test_small_transfers(engine, n, ptr):
         assert rc == 0 and st.edges_count == ec and np.array_equal(lev, want)
         assert (room[:at] == 7).all() and (room[at + 4 * n:] == 7).all()
         assert cpu.check_parents(cp, ri, root, want, par) == 0
+
+
+# contexts in turn and side by side, a thread each: a closed one's pinned ring
+# goes to the next, and no two share one
+def test_contexts_in_turn_and_side_by_side():
+    import threading
+
+    import bfsx
+    rng = np.random.default_rng(5)
+    graphs = []
+    for n in (5, 3001, 300007, 900001):
+        cp, ri = csc_from_edges(n, rng.integers(0, n, 3 * n), rng.integers(0, n, 3 * n))
+        root = int(np.argmax(np.diff(cp.astype(np.int64))))
+        graphs.append((cp, ri, root, cpu.bfs_queue(cp, ri, root)[0]))
+    wrong = []
+
+    def work(k):
+        try:
+            for i in range(6):
+                cp, ri, root, want = graphs[(i + k) % len(graphs)]
+                with bfsx.Engine(0) as eng:
+                    eng.upload_csc(cp, ri)
+                    got_cp, got_ri = eng.download_csc()
+                    lev, _, par = eng.run(root, "llb", parents=True)
+                    if not (np.array_equal(lev, want) and np.array_equal(got_ri, ri)
+                            and np.array_equal(got_cp, cp)
+                            and cpu.check_parents(cp, ri, root, want, par) == 0):
+                        wrong.append((k, i))
+        except Exception as e:  # (a thread's failure is the test's)
+            wrong.append((k, repr(e)))
+
+    for count in (1, 4):
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(count)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        say("contexts", count)
+        assert not wrong
