@@ -23,7 +23,8 @@ struct LevelCtl {
   // work-group of a step adds to both, 12 ns an addition on one line.
   // Together -> apart: 4096^2 grid 7600 -> 7260 us, R-MAT 24 338 -> 314,
   // R-MAT 19 117 -> 114; a 1024^2 grid, whose levels have few groups, pays
-  // for the second line read: 3276 -> 3332 us.
+  // for the second line read: 3276 -> 3332 us, a 300^2 grid in the captured
+  // loop 2740 -> 2850.
   uint32_t pad0_[28];
   unsigned long long q_edges[2];   // sum of out-degree of queue 0 / 1
   unsigned long long glb_total;    // edges of the current GLB frontier

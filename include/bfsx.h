@@ -359,8 +359,9 @@ int bfsx_autotune(bfsx_ctx *ctx, const uint32_t *roots, uint32_t n_roots, int st
                   double *gteps_after);
 
 /* ---- allocation-free search (no counterpart in the reference) -----------
- * For callers that cannot allocate device memory: code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc.  One BFS
+ * For callers that cannot allocate device memory: tight serving loops,
+ * harnesses that forbid hipMalloc (not on a stream under capture: the call
+ * waits for it).  One BFS
  * from `root` over a CSC graph the caller already holds in device memory
  * (col_ptr: n_cols+1 entries of col_ptr_bytes, row_idx: nnz entries; only
  * vertices < n_rows are expanded), writing int32 levels (-1 unreached) to the

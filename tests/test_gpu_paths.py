@@ -34,7 +34,7 @@ def some_graph(name):
 
 
 # a work-group of the histogram takes 4096 vertices, a lane four; tables of
-# more than 1024 levels are counted in global memory; degrees of 65535 and
+# more than 4096 levels are counted in global memory; degrees of 65535 and
 # more are not in the 16-bit array
 @pytest.mark.parametrize("name", ["one", "3", "4", "257", "4096", "4099", "20001", "path2500",
                                   "star70001", "directed4099"])
@@ -199,7 +199,7 @@ def test_noalloc_edges(engine, name, ptr, shift):
 
 
 # levels cross as 1, 2 or 4 bytes each (up to 254, 65534 or more levels) in
-# pieces of 1 MB through four pinned buffers, a piece's slices by up to four
+# pieces of 2 MB through eight pinned buffers, whole pieces by up to four
 # threads; graphs cross as bytes the same way
 @pytest.mark.parametrize("depth", [254, 255, 256, 65535, 65536])
 @pytest.mark.parametrize("n", [70001, 1 << 20, (1 << 20) + 1, 5 * (1 << 20) + 13])
