@@ -1138,12 +1138,7 @@ int bfsx_upload_csc(bfsx_ctx *ctx, uint32_t n_cols, uint32_t n_rows, const void 
     const size_t cp_bytes = (size_t)col_ptr_bytes * n1;
     const size_t ri_bytes = sizeof(uint32_t) * (nnz ? nnz : 1);
     DevBuf cp, ri;
-    struct Releaser {
-      DevBuf *b[2];
-      ~Releaser() {
-        for (DevBuf *x : b) release(*x);
-      }
-    } releaser{{&cp, &ri}};
+    Temporaries on_exit{&cp, &ri};
     auto room_for = [&](DevBuf &b, size_t bytes) {
       try {
         ensure(b, bytes, ctx);
@@ -1222,6 +1217,7 @@ int bfsx_generate_rmat(bfsx_ctx *ctx, int scale, int edge_factor, double a, doub
     release(ctx->col_ptr);
     release(ctx->row_idx);
     DevBuf du, dv;
+    Temporaries on_exit{&du, &dv};
     ensure(du, sizeof(uint32_t) * m, ctx);
     ensure(dv, sizeof(uint32_t) * m, ctx);
     gen_rmat_pairs(ctx, scale, m, thresh32(a), thresh32(a + b), thresh32(a + b + c), seed_graph,
@@ -1249,6 +1245,7 @@ int bfsx_generate_grid(bfsx_ctx *ctx, uint32_t side, double drop_prob, uint32_t 
     release(ctx->col_ptr);
     release(ctx->row_idx);
     DevBuf du, dv;
+    Temporaries on_exit{&du, &dv};
     ensure(du, sizeof(uint32_t) * m, ctx);
     ensure(dv, sizeof(uint32_t) * m, ctx);
     gen_grid_pairs(ctx, side, thresh32(drop_prob), n_long, seed, du.as<uint32_t>(), dv.as<uint32_t>());
@@ -1300,12 +1297,7 @@ int bfsx_order_adjacency(bfsx_ctx *ctx, int order) {
       } copy{ctx, false};
       ensure(ctx->row_idx_pull, sizeof(uint32_t) * std::max<uint64_t>(ctx->nnz, 1), ctx);
       DevBuf by_degree, hrank;  // the vertices, largest degree first; hub indexes
-      struct Releaser {
-        DevBuf *b[2];
-        ~Releaser() {
-          for (DevBuf *x : b) release(*x);
-        }
-      } releaser{{&by_degree, &hrank}};
+      Temporaries on_exit{&by_degree, &hrank};
       order_adjacency(ctx, true, ctx->row_idx_pull.as<uint32_t>(), &by_degree);
       if (ctx->max_degree < 0xFFFFFFFFull) {  // degrees fit the array's 32 bits
         ensure(ctx->pull_fd, sizeof(uint2) * std::max<uint64_t>(ctx->n_rows, 1), ctx);
@@ -1350,13 +1342,13 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
     if (mode == 2) {
       const uint32_t k = std::min(n_roots, ctx->n_rows);
       DevBuf dv;
+      Temporaries on_exit{&dv};
       ensure(dv, sizeof(uint32_t) * std::max(k, 1u), ctx);
       top_degree_vertices(ctx, k, dv.as<uint32_t>());
       if (k) {
         BFSX_HIP(hipMemcpyAsync(roots_out, dv.p, sizeof(uint32_t) * k, hipMemcpyDeviceToHost, s));
         BFSX_HIP(hipStreamSynchronize(s));
       }
-      release(dv);
       if (n_found) *n_found = k;
       return;
     }
@@ -1369,6 +1361,7 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
       const uint32_t probe_batch = 64;
       std::vector<uint32_t> cand(probe_batch);
       DevBuf dv, dok;
+      Temporaries on_exit{&dv, &dok};
       ensure(dv, sizeof(uint32_t) * probe_batch, ctx);
       ensure(dok, probe_batch, ctx);
       std::vector<uint8_t> ok(probe_batch);
@@ -1384,13 +1377,12 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
           if (search(ctx, cand[i], BFSX_LLB, 0, false).reached * 2 > ctx->n_cols) found = true;
         }
       }
-      release(dv);
-      release(dok);
       if (!found) fail(BFSX_ERR_UNSUPPORTED, "no component holds more than half the vertices");
       comp = ctx->levels.as<int32_t>();
     }
     const uint32_t batch = 1u << 16;
     DevBuf dv, dok;
+    Temporaries on_exit{&dv, &dok};
     ensure(dv, sizeof(uint32_t) * batch, ctx);
     ensure(dok, batch, ctx);
     std::vector<uint32_t> cand(batch);
@@ -1407,8 +1399,6 @@ int bfsx_pick_roots(bfsx_ctx *ctx, uint32_t n_roots, uint64_t seed, int mode, ui
         if (std::find(got.begin(), got.end(), cand[i]) == got.end()) got.push_back(cand[i]);
       }
     }
-    release(dv);
-    release(dok);
     std::copy(got.begin(), got.end(), roots_out);
     if (n_found) *n_found = (uint32_t)got.size();
   });
@@ -1478,6 +1468,7 @@ int bfsx_stream_copy(bfsx_ctx *ctx, uint64_t bytes, int repeats, double *ms) {
     if (bytes < 16 || repeats < 1) fail(BFSX_ERR_ARG, "bytes >= 16 and repeats >= 1 required");
     bytes &= ~15ull;
     DevBuf a, b;
+    Temporaries on_exit{&a, &b};
     ensure(a, bytes, ctx);
     ensure(b, bytes, ctx);
     BFSX_HIP(hipMemsetAsync(a.p, 1, bytes, ctx->stream));
@@ -1489,8 +1480,6 @@ int bfsx_stream_copy(bfsx_ctx *ctx, uint64_t bytes, int repeats, double *ms) {
     float t = 0;
     BFSX_HIP(hipEventElapsedTime(&t, ctx->ev0, ctx->ev1));
     if (ms) *ms = t / repeats;
-    release(a);
-    release(b);
   });
 }
 
@@ -1539,6 +1528,7 @@ int bfsx_generate_rmat_union(bfsx_ctx *ctx, uint32_t n_graphs, const int *scales
     release(ctx->col_ptr);
     release(ctx->row_idx);
     DevBuf du, dv;
+    Temporaries on_exit{&du, &dv};
     ensure(du, sizeof(uint32_t) * M, ctx);
     ensure(dv, sizeof(uint32_t) * M, ctx);
     for (uint32_t g = 0; g < n_graphs; g++)

@@ -201,6 +201,7 @@ void gen_rmat_pairs_offset(bfsx_ctx *ctx, int scale, uint64_t m, uint32_t tA, ui
   BFSX_HIP(hipGetLastError());
   // permutation: perm[x] = rank of (random high bits | x)
   DevBuf keys, sorted, perm, tmp;
+  Temporaries on_exit{&keys, &sorted, &perm, &tmp};
   ensure(keys, sizeof(uint64_t) * n, ctx);
   ensure(sorted, sizeof(uint64_t) * n, ctx);
   ensure(perm, sizeof(uint32_t) * n, ctx);
@@ -220,10 +221,6 @@ void gen_rmat_pairs_offset(bfsx_ctx *ctx, int scale, uint64_t m, uint32_t tA, ui
                      perm.as<uint32_t>(), offset, d_u, d_v);
   BFSX_HIP(hipGetLastError());
   BFSX_HIP(hipStreamSynchronize(s));
-  release(keys);
-  release(sorted);
-  release(perm);
-  release(tmp);
 }
 
 uint64_t gen_grid_pairs(bfsx_ctx *ctx, uint32_t side, uint32_t t_drop, uint32_t n_long,
@@ -249,6 +246,7 @@ void build_symmetric_csc(bfsx_ctx *ctx, uint32_t n, uint32_t *d_u, uint32_t *d_v
   const int end_bit = B + bits_for((uint64_t)n + 1);
   const uint64_t K = 2 * m;
   DevBuf keys, sorted, tmp, cnt;
+  Temporaries on_exit{&keys, &sorted, &tmp, &cnt};
   ensure(keys, sizeof(uint64_t) * (K ? K : 1), ctx);
   hipLaunchKernelGGL(k_sym_keys, dim3(grid_for(m)), dim3(256), 0, s, m, B, sentinel, d_u,
                      d_v, keys.as<uint64_t>());
@@ -357,6 +355,7 @@ void graph_summary(bfsx_ctx *ctx) {
                        ctx->col_ptr.as<uint32_t>(), ctx->n_rows, n_pad, ctx->deg16.as<uint16_t>());
   ensure(ctx->iso_bm, sizeof(uint32_t) * (nwords ? nwords : 2), ctx);
   DevBuf out;
+  Temporaries on_exit{&out};
   ensure(out, 2 * sizeof(unsigned int), ctx);
   BFSX_HIP(hipMemsetAsync(out.p, 0, 2 * sizeof(unsigned int), s));
   if (ctx->ptr_bytes == 8)
@@ -373,7 +372,6 @@ void graph_summary(bfsx_ctx *ctx) {
   unsigned int h[2] = {0, 0};
   BFSX_HIP(hipMemcpyAsync(h, out.p, sizeof(h), hipMemcpyDeviceToHost, s));
   BFSX_HIP(hipStreamSynchronize(s));
-  release(out);
   ctx->max_degree = h[0];
   ctx->n_isolated = h[1];
 }
@@ -561,12 +559,7 @@ static void order_adjacency_t(bfsx_ctx *ctx, bool hub_first, uint32_t *out, DevB
   const uint64_t mask = (1ull << B) - 1;
   const PtrT *cp = ctx->col_ptr.as<PtrT>();
   DevBuf keys, sorted, tmp, rank, order;
-  struct Releaser {  // temporaries go on every exit path
-    DevBuf *b[5];
-    ~Releaser() {
-      for (DevBuf *x : b) release(*x);
-    }
-  } releaser{{&keys, &sorted, &tmp, &rank, &order}};
+  Temporaries on_exit{&keys, &sorted, &tmp, &rank, &order};
   size_t tbytes = 0;
   if (hub_first) {
     ensure(keys, sizeof(uint64_t) * n, ctx);
@@ -798,10 +791,7 @@ void compact_first_neighbours(bfsx_ctx *ctx, const uint32_t *hrank) {
   BFSX_HIP(hipStreamSynchronize(s));
   if (linked != n - ctx->n_isolated) fail(BFSX_ERR_DEVICE, "isolated-vertex count mismatch");
   DevBuf out;
-  struct Releaser {
-    DevBuf &b;
-    ~Releaser() { release(b); }
-  } releaser{out};
+  Temporaries on_exit{&out};
   ensure(out, sizeof(uint32_t) * ((uint64_t)linked + 1), ctx);
   ensure(ctx->pull_fdd, sizeof(uint16_t) * ((uint64_t)linked + 1), ctx);
   ensure(ctx->pull_fn, sizeof(uint4) * ((uint64_t)linked + 1), ctx);
@@ -859,6 +849,7 @@ void build_hot_copy(bfsx_ctx *ctx, const uint32_t *by_degree) {
   BFSX_HIP(hipMemcpyAsync(ctx->hot_id.p, by_degree, sizeof(uint32_t) * H,
                           hipMemcpyDeviceToDevice, s));
   DevBuf hrank;
+  Temporaries on_exit{&hrank};
   ensure(hrank, sizeof(uint32_t) * ctx->n_cols, ctx);
   BFSX_HIP(hipMemsetAsync(hrank.p, 0xFF, sizeof(uint32_t) * ctx->n_cols, s));
   hipLaunchKernelGGL(k_hub_rank, dim3(grid_for(H)), dim3(256), 0, s, ctx->hot_id.as<uint32_t>(),
@@ -868,7 +859,6 @@ void build_hot_copy(bfsx_ctx *ctx, const uint32_t *by_degree) {
                      ctx->row_idx_hot.as<uint32_t>());
   BFSX_HIP(hipGetLastError());
   BFSX_HIP(hipStreamSynchronize(s));
-  release(hrank);
   ctx->hot_n = (uint32_t)H;
 }
 
@@ -955,12 +945,7 @@ static void relabel_t(bfsx_ctx *ctx, uint32_t *rank, uint32_t *order, PtrT *new_
   const uint64_t mask = (1ull << B) - 1;
   const PtrT *cp = ctx->col_ptr.as<PtrT>();
   DevBuf keys, sorted, tmp, deg;
-  struct Releaser {
-    DevBuf *b[4];
-    ~Releaser() {
-      for (DevBuf *x : b) release(*x);
-    }
-  } releaser{{&keys, &sorted, &tmp, &deg}};
+  Temporaries on_exit{&keys, &sorted, &tmp, &deg};
   // vertex order
   ensure(keys, sizeof(uint64_t) * n, ctx);
   ensure(sorted, sizeof(uint64_t) * n, ctx);
@@ -1042,12 +1027,7 @@ void top_degree_vertices(bfsx_ctx *ctx, uint32_t k, uint32_t *d_out) {
   if (k > n) k = n;
   if (k == 0) return;
   DevBuf keys, sorted, tmp;
-  struct Releaser {
-    DevBuf *b[3];
-    ~Releaser() {
-      for (DevBuf *x : b) release(*x);
-    }
-  } releaser{{&keys, &sorted, &tmp}};
+  Temporaries on_exit{&keys, &sorted, &tmp};
   ensure(keys, sizeof(uint64_t) * n, ctx);
   ensure(sorted, sizeof(uint64_t) * n, ctx);
   if (ctx->ptr_bytes == 8)

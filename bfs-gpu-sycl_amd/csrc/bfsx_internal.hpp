@@ -279,6 +279,14 @@ void check_hip(hipError_t e, const char *what);
 
 void ensure(DevBuf &b, size_t bytes, bfsx_ctx *ctx);
 void release(DevBuf &b);
+// Releases temporaries on every way out of their scope.
+template <size_t N> struct Temporaries {
+  DevBuf *b[N];
+  ~Temporaries() {
+    for (DevBuf *x : b) release(*x);
+  }
+};
+template <class... B> Temporaries(B *...) -> Temporaries<sizeof...(B)>;
 
 // ---- graph construction (bfsx_gen.hip) -----------------------------------
 // Builds a symmetric CSC in ctx from n undirected pairs (u[i], v[i]) resident

@@ -873,10 +873,7 @@ static MsResult ms_run_t(bfsx_ctx *ctx, const uint32_t *d_src, const uint16_t *d
   r.edges = edges;
   if (levels_out) {  // the per-search level rows, in the caller's vertex ids
     DevBuf out;
-    struct Releaser {
-      DevBuf &b;
-      ~Releaser() { release(b); }
-    } releaser{out};
+    Temporaries on_exit{&out};
     ensure(out, (size_t)n_bits * n, ctx);
     hipLaunchKernelGGL((k_ms_transpose<W>), dim3((unsigned)((n + MS_TV - 1) / MS_TV)), dim3(256), 0,
                        s, lv, n_bits, (uint32_t)n, G.rank, n % 4 == 0 ? 1 : 0, out.as<uint8_t>());

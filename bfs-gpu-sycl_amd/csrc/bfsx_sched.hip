@@ -245,6 +245,7 @@ void mlp_forward(bfsx_ctx *ctx, const float *X, uint32_t n, const float *W, floa
   try {
     upload_batch(ctx, b, X, nullptr, nullptr, n, W);
     DevBuf y;
+    Temporaries on_exit{&y};
     ensure(y, sizeof(float) * OUT * (size_t)n, ctx);
     hipLaunchKernelGGL(k_mlp_forward, dim3((n + 255) / 256), dim3(256), 0, ctx->stream,
                        b.X.as<float>(), n, b.W.as<float>(), y.as<float>());
@@ -252,7 +253,6 @@ void mlp_forward(bfsx_ctx *ctx, const float *X, uint32_t n, const float *W, floa
     BFSX_HIP(hipMemcpyAsync(Y, y.p, sizeof(float) * OUT * (size_t)n, hipMemcpyDeviceToHost,
                             ctx->stream));
     BFSX_HIP(hipStreamSynchronize(ctx->stream));
-    release(y);
   } catch (...) {
     release_batch(b);
     throw;

@@ -328,6 +328,40 @@ template <class P> static void no_room() {
   CHECK(g.resident());
 }
 
+// Memory that ends anywhere in a call that makes temporaries: they are given
+// back, and with the context everything is.
+static void leaks() {
+  const size_t empty = held();
+  int failed = 0;
+  for (size_t room = 0; room < 8u << 20; room += 150000) {
+    reset();
+    CHECK(held() == empty);
+    uint64_t nnz;
+    uint32_t off[3], roots[4];
+    double ms;
+    const int scales[2] = {9, 12}, factors[2] = {8, 8};
+    const uint64_t seeds[2] = {1, 2};
+    std::vector<float> X(8 * 4000), W(BFSX_SCHED_PARAMS), Y(4 * 4000);
+    for (int call = 0; call < 6; call++) {
+      limit = live + room;
+      int rc = BFSX_OK;
+      if (call == 0) rc = bfsx_generate_rmat(ctx, 13, 8, 0.57, 0.19, 0.19, 1, 2, 4, &nnz);
+      if (call == 1) rc = bfsx_generate_grid(ctx, 150, 0.05, 9, 1, 8, &nnz);
+      if (call == 2)
+        rc = bfsx_generate_rmat_union(ctx, 2, scales, factors, seeds, seeds, 4, off, &nnz);
+      if (call == 3) rc = bfsx_mlp_forward(ctx, X.data(), 4000, W.data(), Y.data());
+      if (call == 4) rc = bfsx_stream_copy(ctx, 1 << 20, 1, &ms);
+      if (call == 5) rc = bfsx_pick_roots(ctx, 4, 1, 2, roots, nullptr);
+      failed += rc == BFSX_ERR_NOMEM;
+      bfsx_graph_info g;
+      if (bfsx_graph_info_get(ctx, &g) != BFSX_OK)  // (what a graph holds is not a leak)
+        CHECK(held() <= empty + (2 << 20));  // (state that the next graph takes over)
+    }
+    limit = (size_t)1 << 30;
+  }
+  CHECK(failed > 20);
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (bfsx_create(0, &ctx) != BFSX_OK) return 2;
@@ -348,6 +382,8 @@ int main(int argc, char **argv) {
     no_room<uint32_t>();
     reset();
     no_room<uint64_t>();
+  } else if (what == "leaks") {
+    leaks();
   } else {
     return 2;
   }

@@ -50,3 +50,7 @@ def test_shared_tiles_fit_a_launch(driver):
 
 def test_upload_without_room_for_both_graphs(driver):
     check(driver, "no_room")
+
+
+def test_temporaries_are_given_back_where_memory_ends(driver):
+    check(driver, "leaks")
